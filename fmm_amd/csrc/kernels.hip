@@ -838,10 +838,10 @@ __global__ __launch_bounds__(64) void k_expand(int p, uint32_t rows, const uint3
 }
 
 // ---- evaluation at targets: L2P (regular) and M2P (irregular) ------------------------
-// One wave per target leaf; every entry's coefficients go to LDS with the derived
-// coefficients of the gradient (the ladders of CONVENTIONS §3.11 "L2P and M2P" moved
-// onto the coefficients), then the lanes of a target (one, or up to 8 for leaves of at
-// most 32 targets) walk the recursion of its columns and contract on the fly.  Regular: grad_k = sum_{n<p} G_k R_n, with
+// A box's coefficients go to LDS with the derived coefficients of the gradient (the
+// ladders of CONVENTIONS §3.11 "L2P and M2P" moved onto the coefficients), then the lanes
+// of a target (one, or up to 8 for leaves of at most 32 targets) walk the recursion of
+// their columns and contract on the fly.  Regular: grad_k = sum_{n<p} G_k R_n, with
 // Gz_n^m = L_{n+1}^m, Gx_n^m = (L_{n+1}^{m+1} - L_{n+1}^{m-1})/2,
 // Gy_n^m = i (L_{n+1}^{m+1} + L_{n+1}^{m-1})/2.  Irregular: grad_k = sum_{1<=n<=p+1}
 // G_k I_n, with Gz_n^m = -M_{n-1}^m, Gx_n^m = (M_{n-1}^{m+1} - M_{n-1}^{m-1})/2,
@@ -862,15 +862,18 @@ __device__ __forceinline__ void read_order(const double *c, int n, int q, int pm
   }
 }
 
-template <bool IRREG, bool GRAD>
-__global__ __launch_bounds__(IRREG ? 128 : 64) void k_evaluate(int p, uint32_t rows, const uint32_t *row_leaf,
-                                                           const uint32_t *row_off,
-                                                           const uint32_t *row_box, const uint32_t *box_cell,
-                                                           const uint32_t *leaf_cell, const uint32_t *tgt_start,
-                                                           const double *tx, const double *ty, const double *tz,
-                                                           const double *coeffs, double *phi, double *grad) {
-  // LDS sized to the degree (eval_lds_bytes): the coefficients, then the three gradient
-  // coefficient sets, so that more waves share a CU at low p
+// The sub-lanes per target of a leaf with nt targets: a wave serves 64 / L targets a pass.
+__device__ __forceinline__ int sub_lanes(uint32_t nt) {
+  return nt > 32 ? 1 : (64 / int(nt) < 8 ? 64 / int(nt) : 8);
+}
+
+template <bool GRAD>
+__global__ __launch_bounds__(64) void k_l2p(int p, uint32_t rows, const uint32_t *row_leaf, const uint32_t *row_off,
+                                            const uint32_t *row_box, const uint32_t *tgt_start, const double *tx,
+                                            const double *ty, const double *tz, const double *coeffs, double *phi,
+                                            double *grad) {
+  // LDS sized to the degree: the coefficients, then the three gradient coefficient sets,
+  // so that more waves share a CU at low p
   extern __shared__ __align__(16) double eval_smem[];
   const int nc = (p + 1) * (p + 1);
   const uint32_t row = xcd_index(rows);
@@ -878,118 +881,84 @@ __global__ __launch_bounds__(IRREG ? 128 : 64) void k_evaluate(int p, uint32_t r
   const uint32_t lf = row_leaf[row];
   const uint32_t t0 = tgt_start[lf], t1 = tgt_start[lf + 1];
   if (t0 == t1) return;
-  const int pg = IRREG ? p + 1 : p - 1;  // degree of the gradient coefficients
+  const int pg = p - 1;  // degree of the gradient coefficients
   const int ng = pg >= 0 ? (pg + 1) * (pg + 1) : 0;
   double *C = eval_smem, *G0 = C + nc, *G1 = G0 + ng, *G2 = G1 + ng;
-  // L2P: one wave per leaf; leaves of more than 32 targets one lane per target, in
-  // passes of 64, smaller ones L = min(8, 64 / n) sub-lanes per target, which share its
-  // columns.  M2P: two waves, one thread per target (a row's W-list boxes are taken in
-  // turn, so the per-box set-up and passes stay short on long rows).
-  constexpr int NT = IRREG ? 128 : 64;
+  // one wave per leaf: leaves of more than 32 targets one lane per target, in passes of
+  // 64, smaller ones L = min(8, 64 / n) sub-lanes per target, which share its columns
   const int lane = threadIdx.x;
   const uint32_t nt = t1 - t0;
-  const int L = (IRREG || nt > 32) ? 1 : (64 / int(nt) < 8 ? 64 / int(nt) : 8);
-  const int per = NT / L;  // targets per pass
+  const int L = sub_lanes(nt);
+  const int per = 64 / L;  // targets per pass
   const int u = lane % L, tl = lane / L;
   for (uint32_t e = row_off[row]; e < row_off[row + 1]; ++e) {
     const uint32_t box = row_box[e];
-    double c[3] = {0.0, 0.0, 0.0}, r = 1.0;
-    if (IRREG) relative_frame<double>(box_cell + 4 * size_t(box), leaf_cell + 4 * size_t(lf), c, r);
     __syncthreads();
-    for (int k = lane; k < nc; k += NT) C[k] = coeffs[size_t(box) * nc + k];
+    for (int k = lane; k < nc; k += 64) C[k] = coeffs[size_t(box) * nc + k];
     __syncthreads();
     if (GRAD)
-      for (int k = lane; k < ng; k += NT) {
+      for (int k = lane; k < ng; k += 64) {
         int n = 0;
         while ((n + 1) * (n + 1) <= k) ++n;
         const int m = k - n * n - n;
         if (m < 0) continue;  // slot -m is written with slot +m
-        const int src = IRREG ? n - 1 : n + 1;
         double ar, ai, br, bi, zr, zi;
-        read_order(C, src, m + 1, p, ar, ai);
-        read_order(C, src, m - 1, p, br, bi);
-        read_order(C, src, m, p, zr, zi);
-        const double xr = 0.5 * (ar - br), xi = 0.5 * (ai - bi);
-        const double yr = -0.5 * (ai + bi), yi = 0.5 * (ar + br);
-        if (IRREG) {
-          zr = -zr;
-          zi = -zi;
-        }
-        G0[idx(n, m)] = xr;
-        G1[idx(n, m)] = yr;
+        read_order(C, n + 1, m + 1, p, ar, ai);
+        read_order(C, n + 1, m - 1, p, br, bi);
+        read_order(C, n + 1, m, p, zr, zi);
+        G0[idx(n, m)] = 0.5 * (ar - br);
+        G1[idx(n, m)] = -0.5 * (ai + bi);
         G2[idx(n, m)] = zr;
         if (m > 0) {
-          G0[idx(n, -m)] = xi;
-          G1[idx(n, -m)] = yi;
+          G0[idx(n, -m)] = 0.5 * (ai - bi);
+          G1[idx(n, -m)] = 0.5 * (ar + br);
           G2[idx(n, -m)] = zi;
         }
       }
     __syncthreads();
-    const double inv_r = 1.0 / r;
     for (uint32_t b = 0; b < nt; b += uint32_t(per)) {
       const uint32_t ti = b + uint32_t(tl);
       const bool valid = tl < per && ti < nt;
       const uint32_t i = t0 + (valid ? ti : 0u);
       double sp = 0.0, sx = 0.0, sy = 0.0, sz = 0.0;
       if (valid) {
-        double x = tx[i], y = ty[i], z = tz[i];
-        if (IRREG) {
-          x = (x - c[0]) * inv_r;
-          y = (y - c[1]) * inv_r;
-          z = (z - c[2]) * inv_r;
-        }
+        const double x = tx[i], y = ty[i], z = tz[i];
         const double r2 = x * x + y * y + z * z;
-        const double inv_r2 = IRREG ? 1.0 / r2 : 0.0;
-        double dr = IRREG ? rsqrt_t<double>(r2) : 1.0, di = 0.0;
+        double dr = 1.0, di = 0.0;
         int md = 0;  // order of the diagonal entry (dr, di)
-        const int ptop = IRREG ? (GRAD ? p + 1 : p) : p;
         // columns m of this sub-lane: block jb holds m = jb L .. jb L + L - 1, dealt to
         // the sub-lanes forwards in even blocks and backwards in odd ones
-        for (int jb = 0; jb * L <= ptop; ++jb) {
+        for (int jb = 0; jb * L <= p; ++jb) {
           const int m = jb * L + ((jb & 1) ? L - 1 - u : u);
-          if (m > ptop) continue;
+          if (m > p) continue;
           while (md < m) {
             ++md;
-            const double f = IRREG ? (2.0 * md - 1.0) * inv_r2 : c_inv_2m[md];
+            const double f = c_inv_2m[md];
             const double nr = f * (x * dr - y * di), ni = f * (x * di + y * dr);
             dr = nr;
             di = ni;
           }
           double pr = 0.0, pi = 0.0, cr = dr, ci = di;
           const double w = m == 0 ? 1.0 : 2.0;
-          for (int n = m; n <= ptop; ++n) {
+          for (int n = m; n <= p; ++n) {
             if (n > m) {
               double nr, ni;
-              if (IRREG) {
-                if (n == m + 1) {
-                  const double f = (2.0 * m + 1.0) * z * inv_r2;
-                  nr = f * cr;
-                  ni = f * ci;
-                } else {
-                  const double a = (2.0 * n - 1.0) * z, bb = double((n - 1) * (n - 1) - m * m);
-                  nr = (a * cr - bb * pr) * inv_r2;
-                  ni = (a * ci - bb * pi) * inv_r2;
-                }
+              if (n == m + 1) {
+                nr = z * cr;
+                ni = z * ci;
               } else {
-                if (n == m + 1) {
-                  nr = z * cr;
-                  ni = z * ci;
-                } else {
-                  const double a = (2.0 * n - 1.0) * z, inv = c_inv_reg[idx(n, m)];
-                  nr = (a * cr - r2 * pr) * inv;
-                  ni = (a * ci - r2 * pi) * inv;
-                }
+                const double a = (2.0 * n - 1.0) * z, inv = c_inv_reg[idx(n, m)];
+                nr = (a * cr - r2 * pr) * inv;
+                ni = (a * ci - r2 * pi) * inv;
               }
               pr = cr;
               pi = ci;
               cr = nr;
               ci = ni;
             }
-            if (n <= p) {
-              const double lr = C[idx(n, m)], li = m > 0 ? C[idx(n, -m)] : 0.0;
-              sp += w * (lr * cr - li * ci);
-            }
-            if (GRAD && n <= pg && (!IRREG || n >= 1)) {
+            const double lr = C[idx(n, m)], li = m > 0 ? C[idx(n, -m)] : 0.0;
+            sp += w * (lr * cr - li * ci);
+            if (GRAD && n <= pg) {
               const int ia = idx(n, m), ib = idx(n, -m);
               const double xr = G0[ia], yr = G1[ia], zr = G2[ia];
               const double xi = m > 0 ? G0[ib] : 0.0, yi = m > 0 ? G1[ib] : 0.0, zi = m > 0 ? G2[ib] : 0.0;
@@ -1019,15 +988,218 @@ __global__ __launch_bounds__(IRREG ? 128 : 64) void k_evaluate(int p, uint32_t r
         sz = uz;
       }
       if (valid && u == 0) {
-        phi[i] += sp * inv_r;
+        phi[i] += sp;
         if (GRAD) {
-          const double s2 = inv_r * inv_r;
-          grad[3 * size_t(i) + 0] += sx * s2;
-          grad[3 * size_t(i) + 1] += sy * s2;
-          grad[3 * size_t(i) + 2] += sz * s2;
+          grad[3 * size_t(i) + 0] += sx;
+          grad[3 * size_t(i) + 1] += sy;
+          grad[3 * size_t(i) + 2] += sz;
         }
       }
     }
+  }
+}
+
+// M2P: one workgroup per target leaf, its waves taking the boxes of the row in turn (wave w
+// the boxes w, w + W, ...), each with its own region of LDS and no barrier until the
+// waves' sums meet, added in wave order.  A row can hold a hundred boxes and a launch few
+// rows, so with one wave a row the launch was one chain of boxes.  Per box an entry
+// (n, m >= 0) of LDS holds what the lane needs at that step of its column, weighted by 2
+// for m > 0: (Re, Im) of the coefficient of I_n^m and, with gradients, of its three
+// derivative coefficients, in the order the columns are walked.  150,000 Plummer points,
+// p = 8 (1,886 rows of 27 boxes, at most 98): 1.85 -> 0.46 ms; 43 rows of 123 boxes, p = 9,
+// potentials alone: 1.28 -> 0.07 ms.
+struct M2pEntry {
+  double c[2], x[2], y[2], z[2];
+};
+
+static size_t m2p_wave_lds(int p, int gradients) {
+  const size_t entries = gradients ? size_t(p + 2) * (p + 3) / 2 : size_t(p + 1) * (p + 2) / 2;
+  const size_t bytes = entries * (gradients ? sizeof(M2pEntry) : 2 * sizeof(double));
+  const size_t sums = 64 * (gradients ? 4 : 1) * sizeof(double);
+  return bytes > sums ? bytes : sums;
+}
+
+// eight waves, fewer where their regions would not fit 64 KB
+static int m2p_waves(int p, int gradients) {
+  const size_t w = 65536 / m2p_wave_lds(p, gradients);
+  return w < 8 ? int(w) : 8;
+}
+
+// Ordering of LDS between the lanes of one wave: its LDS operations complete in order, so
+// only the compiler must not move them.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <bool GRAD>
+__global__ __launch_bounds__(512) void k_m2p(int p, int wave_doubles, uint32_t rows, const uint32_t *row_leaf,
+                                             const uint32_t *row_off, const uint32_t *row_box,
+                                             const uint32_t *box_cell, const uint32_t *leaf_cell,
+                                             const uint32_t *tgt_start, const double *tx, const double *ty,
+                                             const double *tz, const double *coeffs, double *phi, double *grad) {
+  extern __shared__ __align__(16) double eval_smem[];
+  constexpr int ED = GRAD ? 8 : 2;  // doubles per entry
+  constexpr int ME = (kMaxDegree + 2) * (kMaxDegree + 3) / 2;
+  constexpr int EL = (ME + 63) / 64;  // entries per lane
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, W = blockDim.x >> 6;
+  const int nc = (p + 1) * (p + 1), ptop = GRAD ? p + 1 : p;
+  const int ne = (ptop + 1) * (ptop + 2) / 2;
+  const uint32_t row = xcd_index(rows);
+  if (row >= rows) return;
+  const uint32_t lf = row_leaf[row];
+  const uint32_t t0 = tgt_start[lf], t1 = tgt_start[lf + 1];
+  if (t0 == t1) return;
+  double *E = eval_smem + size_t(wave) * wave_doubles;
+  // (n, m) of the entries this lane fills: columns m = 0 .. ptop, each n = m .. ptop
+  int en[EL], em[EL];
+#pragma unroll
+  for (int k = 0; k < EL; ++k) {
+    int t = lane + 64 * k, m = 0;
+    while (m <= ptop && t >= ptop + 1 - m) {
+      t -= ptop + 1 - m;
+      ++m;
+    }
+    en[k] = m + t;
+    em[k] = m;
+  }
+  const uint32_t nt = t1 - t0;
+  const int L = sub_lanes(nt);
+  const int per = 64 / L;  // targets per pass
+  const int u = lane % L, tl = lane / L;
+  const uint32_t e0 = row_off[row], e1 = row_off[row + 1];
+  for (uint32_t b = 0; b < nt; b += uint32_t(per)) {
+    const uint32_t ti = b + uint32_t(tl);
+    const bool valid = tl < per && ti < nt;
+    const uint32_t i = t0 + (valid ? ti : 0u);
+    const double tgx = tx[i], tgy = ty[i], tgz = tz[i];
+    double sp = 0.0, sx = 0.0, sy = 0.0, sz = 0.0;
+    for (uint32_t e = e0 + uint32_t(wave); e < e1; e += uint32_t(W)) {
+      const uint32_t box = row_box[e];
+      double c[3], r;
+      relative_frame<double>(box_cell + 4 * size_t(box), leaf_cell + 4 * size_t(lf), c, r);
+      const double *M = coeffs + size_t(box) * nc;
+      wave_sync();  // the previous box's entries are read
+#pragma unroll
+      for (int k = 0; k < EL; ++k)
+        if (lane + 64 * k < ne) {
+          const int n = en[k], m = em[k];
+          const double w = m == 0 ? 1.0 : 2.0;
+          double *o = E + (lane + 64 * k) * ED;
+          double cr, ci;
+          read_order(M, n, m, p, cr, ci);
+          o[0] = w * cr;
+          o[1] = w * ci;
+          if (GRAD) {
+            double ar, ai, br, bi, zr, zi;
+            read_order(M, n - 1, m + 1, p, ar, ai);
+            read_order(M, n - 1, m - 1, p, br, bi);
+            read_order(M, n - 1, m, p, zr, zi);
+            o[2] = 0.5 * w * (ar - br);
+            o[3] = m > 0 ? 0.5 * w * (ai - bi) : 0.0;
+            o[4] = -0.5 * w * (ai + bi);
+            o[5] = m > 0 ? 0.5 * w * (ar + br) : 0.0;
+            o[6] = -w * zr;
+            o[7] = m > 0 ? -w * zi : 0.0;
+          }
+        }
+      wave_sync();
+      if (valid) {
+        const double inv_r = 1.0 / r;  // a power of two
+        const double x = (tgx - c[0]) * inv_r, y = (tgy - c[1]) * inv_r, z = (tgz - c[2]) * inv_r;
+        const double r2 = x * x + y * y + z * z;
+        const double inv_r2 = 1.0 / r2, zi2 = z * inv_r2;
+        double dr = rsqrt_t<double>(r2), di = 0.0;
+        int md = 0;  // order of the diagonal entry (dr, di)
+        double bp = 0.0, bx = 0.0, by = 0.0, bz = 0.0;
+        // columns m of this sub-lane: block jb holds m = jb L .. jb L + L - 1, dealt to
+        // the sub-lanes forwards in even blocks and backwards in odd ones
+        for (int jb = 0; jb * L <= ptop; ++jb) {
+          const int m = jb * L + ((jb & 1) ? L - 1 - u : u);
+          if (m > ptop) continue;
+          while (md < m) {
+            ++md;
+            const double f = (2.0 * md - 1.0) * inv_r2;
+            const double nr = f * (x * dr - y * di), ni = f * (x * di + y * dr);
+            dr = nr;
+            di = ni;
+          }
+          double pr = 0.0, pi = 0.0, cr = dr, ci = di;
+          const double *o = E + (m * (ptop + 1) - m * (m - 1) / 2) * ED;
+#pragma unroll 2
+          for (int n = m; n <= ptop; ++n, o += ED) {
+            double v[ED];
+#pragma unroll
+            for (int k = 0; k < ED; ++k) v[k] = o[k];
+            bp += v[0] * cr - v[1] * ci;
+            if (GRAD) {
+              bx += v[2] * cr - v[3] * ci;
+              by += v[4] * cr - v[5] * ci;
+              bz += v[6] * cr - v[7] * ci;
+            }
+            // X_{n+1}^m from X_n^m and X_{n-1}^m (zero at n = m)
+            const double a = (2.0 * n + 1.0) * zi2, bb = double(n * n - m * m) * inv_r2;
+            const double nr = a * cr - bb * pr, ni = a * ci - bb * pi;
+            pr = cr;
+            pi = ci;
+            cr = nr;
+            ci = ni;
+          }
+        }
+        sp += bp * inv_r;
+        if (GRAD) {
+          const double s2 = inv_r * inv_r;
+          sx += bx * s2;
+          sy += by * s2;
+          sz += bz * s2;
+        }
+      }
+    }
+    if (L > 1) {
+      // the target's sub-lanes add their sums in sub-lane order (every lane takes part)
+      const int base = lane - u;
+      double tp = 0.0, ux = 0.0, uy = 0.0, uz = 0.0;
+      for (int k = 0; k < L; ++k) {
+        const int src = base + k < 64 ? base + k : 63;
+        tp += __shfl(sp, src);
+        if (GRAD) {
+          ux += __shfl(sx, src);
+          uy += __shfl(sy, src);
+          uz += __shfl(sz, src);
+        }
+      }
+      sp = tp;
+      sx = ux;
+      sy = uy;
+      sz = uz;
+    }
+    // the waves' sums through their regions, added in wave order
+    __syncthreads();
+    E[lane] = sp;
+    if (GRAD) {
+      E[64 + lane] = sx;
+      E[128 + lane] = sy;
+      E[192 + lane] = sz;
+    }
+    __syncthreads();
+    if (wave == 0 && valid && u == 0) {
+      for (int k = 1; k < W; ++k) {
+        const double *o = eval_smem + size_t(k) * wave_doubles;
+        sp += o[lane];
+        if (GRAD) {
+          sx += o[64 + lane];
+          sy += o[128 + lane];
+          sz += o[192 + lane];
+        }
+      }
+      phi[i] += sp;
+      if (GRAD) {
+        grad[3 * size_t(i) + 0] += sx;
+        grad[3 * size_t(i) + 1] += sy;
+        grad[3 * size_t(i) + 2] += sz;
+      }
+    }
+    __syncthreads();  // the next pass fills the regions again
   }
 }
 
@@ -1193,25 +1365,26 @@ void evaluate(hipStream_t s, int p, int irregular, int gradients, uint32_t rows,
               const uint32_t *leaf_cell, const uint32_t *tgt_start, const double *tx, const double *ty,
               const double *tz, const double *coeffs, double *phi, double *grad) {
   if (rows == 0) return;
-  // LDS: (p+1)^2 coefficients and, with gradients, three sets of (pg+1)^2 (pg = p + 1 for
-  // M2P, p - 1 for L2P); at most 1,123 doubles at p = 15
-  const int pg = irregular ? p + 1 : p - 1;
-  const size_t lds = sizeof(double) * (size_t((p + 1) * (p + 1)) + (gradients && pg >= 0 ? 3 * size_t((pg + 1) * (pg + 1)) : 0));
-#define FMMH_EVAL(I, G)                                                                                          \
-  hipLaunchKernelGGL((k_evaluate<I, G>), dim3(xcd_grid(rows)), dim3(I ? 128 : 64), lds, s, p, rows, row_leaf, \
-                     row_off, row_box, box_cell, leaf_cell, tgt_start, tx, ty, tz, coeffs, phi, grad)
   if (irregular) {
+    const size_t wave_lds = m2p_wave_lds(p, gradients);
+    const int waves = m2p_waves(p, gradients), wd = int(wave_lds / sizeof(double));
     if (gradients)
-      FMMH_EVAL(true, true);
+      hipLaunchKernelGGL(k_m2p<true>, dim3(xcd_grid(rows)), dim3(64 * waves), waves * wave_lds, s, p, wd, rows,
+                         row_leaf, row_off, row_box, box_cell, leaf_cell, tgt_start, tx, ty, tz, coeffs, phi, grad);
     else
-      FMMH_EVAL(true, false);
-  } else {
-    if (gradients)
-      FMMH_EVAL(false, true);
-    else
-      FMMH_EVAL(false, false);
+      hipLaunchKernelGGL(k_m2p<false>, dim3(xcd_grid(rows)), dim3(64 * waves), waves * wave_lds, s, p, wd, rows,
+                         row_leaf, row_off, row_box, box_cell, leaf_cell, tgt_start, tx, ty, tz, coeffs, phi, grad);
+    return;
   }
-#undef FMMH_EVAL
+  // LDS: (p+1)^2 coefficients and, with gradients, three sets of p^2; at most 931 doubles
+  // at p = 15
+  const size_t lds = sizeof(double) * (size_t((p + 1) * (p + 1)) + (gradients ? 3 * size_t(p * p) : 0));
+  if (gradients)
+    hipLaunchKernelGGL(k_l2p<true>, dim3(xcd_grid(rows)), dim3(64), lds, s, p, rows, row_leaf, row_off, row_box,
+                       tgt_start, tx, ty, tz, coeffs, phi, grad);
+  else
+    hipLaunchKernelGGL(k_l2p<false>, dim3(xcd_grid(rows)), dim3(64), lds, s, p, rows, row_leaf, row_off, row_box,
+                       tgt_start, tx, ty, tz, coeffs, phi, grad);
 }
 
 }  // namespace dev

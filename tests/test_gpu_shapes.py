@@ -1,0 +1,50 @@
+"""The kernels at the shapes where their splits of the work can go wrong, against the oracle
+on the same tree: f64 within 1e-12 (the sums' order and 2^-53 per term, amplified by at most
+the M2L's cancellation), the mixed precision within 1e-6."""
+import sys
+
+import numpy as np
+import pytest
+
+import fmm_amd
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _log(msg):
+    print(msg, flush=True)
+    sys.stdout.flush()
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    if fmm_amd.device_count() < 1:
+        pytest.skip("no GPU")
+
+
+def _check(fmm, ref, q, gradients=True, tol=1e-12):
+    out = fmm.evaluate(q)
+    phi, grad = ref.evaluate(q)
+    errs = [O.error_norms(out.potential, phi)[0]]
+    if gradients:
+        errs.append(O.error_norms(out.gradient, grad, True)[0])
+    _log(f"  errors {errs}")
+    assert max(errs) < tol, errs
+    again = fmm.evaluate(q)
+    assert np.array_equal(out.potential, again.potential)
+
+
+@pytest.mark.parametrize("p,leaf,gradients", [(0, 3, True), (1, 5, False), (4, 70, True), (9, 150, False),
+                                              (14, 64, True), (15, 33, True), (15, 9, False)])
+def test_m2p_rows_over_waves(p, leaf, gradients):
+    """Long W rows (a dense cluster beside large leaves), leaves of one target to several
+    passes of targets, the degrees where a workgroup holds fewer than eight waves."""
+    _log(f"case M2P rows p={p} leaf={leaf} gradients={gradients}")
+    rng = O.Rng(77)
+    pts = np.vstack([rng.plummer(1500, (0.5, 0.5, 0.5), 0.01), rng.cube(600)])
+    q = rng.normals(len(pts))
+    fmm = fmm_amd.FmmBuilder(p).max_points_per_leaf(leaf).gradients(gradients).build(pts)
+    rows = [len(fmm.plan.list("w", level)[1]) for level in range(fmm.plan.nlevels)]
+    assert sum(rows) > 0
+    _check(fmm, O.Fmm(pts, p=p, leaf_points=leaf, gradients=gradients), q, gradients)
