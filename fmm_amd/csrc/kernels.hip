@@ -67,12 +67,12 @@ __device__ __forceinline__ float rsqrt_t<float>(float x) {
 
 template <>
 __device__ __forceinline__ double rsqrt_t<double>(double x) {
-  // v_rsq_f64 estimate refined by two Newton steps y += y (1 - x y^2) / 2
+  // v_rsq_f64 (relative error up to 5.2e-8, measured over [1, 4)) and one third-order step
+  // y += y e (1/2 + 3/8 e), e = 1 - x y^2: 2.7e-16, as two Newton steps give (2.65e-16) in
+  // three operations more
   double y = __builtin_amdgcn_rsq(x);
-  double e = fma(-x * y, y, 1.0);
-  y = fma(0.5 * y, e, y);
-  e = fma(-x * y, y, 1.0);
-  y = fma(0.5 * y, e, y);
+  const double e = fma(-x * y, y, 1.0);
+  y = fma(y * e, fma(0.375, e, 0.5), y);
   return y;
 }
 
@@ -219,17 +219,17 @@ __global__ void k_vjp_combine(size_t n, const double *q, const double *g, const 
 // r^2, the inverse square root and the sums of a tile (at most 64 sources) are f32; the
 // tile sums are added in f64.  Coincident points give d = 0 exactly in both forms.
 
-// Lane mapping (one wave per target leaf, targets processed in chunks of 128): a chunk of
-// n <= 64 targets uses np = n lanes per source phase and floor(64 / n) phases, phase f
-// taking the sources j = f, f + phases, ... of every tile (tiles of phases x floor(64 /
-// phases) sources); a chunk of 65..128 targets puts two targets in each lane.  A tile is
-// padded with zero charges far away to a multiple of the phase count, so every lane runs
-// the same number of steps; the phases' partial sums are added in phase order through
-// LDS, so results are the same on every run.  The next tile's coordinates and charges
-// are loaded into registers while the current tile is computed.
+// Lane mapping (one wave per target leaf, targets processed in chunks of 128): the staged
+// form puts one or two targets in each lane (the fuller use of the lanes), np lanes per
+// source phase and floor(64 / np) phases, phase f taking the sources j = f, f + phases, ...
+// of every tile (tiles of phases x floor(64 / phases) sources).  A tile is padded with
+// zero charges far away to a multiple of the phase count, so every lane runs the same
+// number of steps; the phases' partial sums are added in phase order through LDS, so
+// results are the same on every run.  The next tile's coordinates and charges are loaded
+// into registers while the current tile is computed.
 //
 // Only a target's own leaf can hold a source at r^2 == 0 (equal coordinates give equal
-// leaves): that tile selects 0 for r^2 == 0; other tiles clamp r^2 below at the smallest
+// leaves): that tile selects 0 for r^2 == 0; other tiles start r^2 from the smallest
 // normal number, which changes nothing for distinct points (r^2 >= 1e-22 in leaf units
 // at the deepest level) and keeps a separation rounded to zero finite.
 // Chunks of at least `umin` targets in the mixed path (33 by the static rule): each lane
@@ -408,6 +408,270 @@ __device__ __forceinline__ void p2p_uniform(uint32_t lf, uint32_t tb, uint32_t n
   }
 }
 
+// Shared memory of one wave of the staged form.
+template <typename T>
+struct P2pStage {
+  // a source: (x, y, z, q) and, for the split form, (x_lo, y_lo, z_lo, 0), so a lane reads
+  // it with one or two 16-byte loads
+  using V4 = typename std::conditional<sizeof(T) == 4, float4, double4>::type;
+  V4 ys[64];
+  float4 yl[sizeof(T) == 4 ? 64 : 1];
+  double fr[64][4];     // frame (c, r) of each entry of a chunk of the near row
+  uint32_t fstart[64];  // first source of each entry
+  uint32_t fcum[65];    // exclusive prefix sums of the entries' source counts
+};
+
+// Lanes of a staged chunk of n targets with A targets per lane: np = ceil(n / A) lanes per
+// phase, floor(64 / np) phases.
+__device__ __forceinline__ int staged_lanes(uint32_t n, int A) { return (int(n) + A - 1) / A; }
+
+template <typename T, bool GRAD, int A>
+__device__ __forceinline__ void p2p_staged(P2pStage<T> &sh, uint32_t lf, uint32_t tb, uint32_t n, uint32_t e0,
+                                           uint32_t e1, const uint32_t *__restrict__ near_ent,
+                                           const uint32_t *__restrict__ leaf_cell,
+                                           const uint32_t *__restrict__ src_start, const double *__restrict__ sx,
+                                           const double *__restrict__ sy, const double *__restrict__ sz,
+                                           const double *__restrict__ sq, const double *__restrict__ tx,
+                                           const double *__restrict__ ty, const double *__restrict__ tz,
+                                           double *__restrict__ phi, double *__restrict__ grad) {
+  constexpr bool SPLIT = sizeof(T) == 4;
+  constexpr int TILE = 64;
+  constexpr T TINY = sizeof(T) == 4 ? T(1.17549435e-38f) : T(2.2250738585072014e-308);
+  constexpr double FAR = 1024.0;  // padding position, in target-leaf units
+  using V4 = typename P2pStage<T>::V4;
+  const int lane = threadIdx.x;
+  const uint32_t *ct = leaf_cell + 4 * size_t(lf);
+  const int np = staged_lanes(n, A), phases = 64 / np;
+  const int tsz = phases * (64 / phases);  // sources per tile: a multiple of the phases
+  const bool lane_ok = lane < np * phases;
+  const int slot = lane % np, phase = lane_ok ? lane / np : 0;
+  T ux[A], uy[A], uz[A], lx[A], ly[A], lz[A], ap[A], ax[A], ay[A], az[A];
+  bool ok[A];
+#pragma unroll
+  for (int a = 0; a < A; ++a) {
+    const uint32_t i = tb + uint32_t(slot + a * np);
+    ok[a] = lane_ok && uint32_t(slot + a * np) < n;
+    const double x = ok[a] ? tx[i] : 0.0, y = ok[a] ? ty[i] : 0.0, z = ok[a] ? tz[i] : 0.0;
+    ux[a] = T(x);
+    uy[a] = T(y);
+    uz[a] = T(z);
+    lx[a] = T(x - double(ux[a]));
+    ly[a] = T(y - double(uy[a]));
+    lz[a] = T(z - double(uz[a]));
+    ap[a] = ax[a] = ay[a] = az[a] = T(0);
+  }
+  // f32 sums are per tile (at most 64 terms) and go into f64 after each tile, so long
+  // near rows do not lose digits to one growing f32 sum
+  double cp[A], cx[A], cy[A], cz[A];
+#pragma unroll
+  for (int a = 0; a < A; ++a) cp[a] = cx[a] = cy[a] = cz[a] = 0.0;
+  auto flush = [&]() {
+    if (SPLIT) {
+#pragma unroll
+      for (int a = 0; a < A; ++a) {
+        cp[a] += double(ap[a]);
+        cx[a] += double(ax[a]);
+        cy[a] += double(ay[a]);
+        cz[a] += double(az[a]);
+        ap[a] = ax[a] = ay[a] = az[a] = T(0);
+      }
+    }
+  };
+  // one source j of the tile against the lane's targets
+  auto step = [&](int j, auto check) {
+    const V4 v = sh.ys[j];
+    const T yx = v.x, yy = v.y, yz = v.z, q = v.w;
+    T yxl = T(0), yyl = T(0), yzl = T(0);
+    if (SPLIT) {
+      const float4 w = sh.yl[j];
+      yxl = w.x;
+      yyl = w.y;
+      yzl = w.z;
+    }
+#pragma unroll
+    for (int a = 0; a < A; ++a) {
+      T dx = ux[a] - yx, dy = uy[a] - yy, dz = uz[a] - yz;
+      if (SPLIT) {
+        dx += lx[a] - yxl;
+        dy += ly[a] - yyl;
+        dz += lz[a] - yzl;
+      }
+      T inv;
+      if constexpr (decltype(check)::value) {
+        const T r2 = dx * dx + dy * dy + dz * dz;
+        inv = r2 == T(0) ? T(0) : rsqrt_t<T>(r2);
+      } else {
+        inv = rsqrt_t<T>(fma(dz, dz, fma(dy, dy, fma(dx, dx, TINY))));
+      }
+      const T qi = q * inv;
+      ap[a] += qi;
+      if (GRAD) {
+        const T qi3 = qi * (inv * inv);
+        ax[a] -= qi3 * dx;
+        ay[a] -= qi3 * dy;
+        az[a] -= qi3 * dz;
+      }
+    }
+  };
+  // stage one tile: lane < cnt holds the source (x, y, z, q) in the target frame;
+  // lanes cnt .. steps * phases - 1 hold zero charges far away
+  auto stage = [&](int cnt, int steps, bool valid, double yx, double yy, double yz, double q) {
+    __syncthreads();
+    if (lane < steps * phases) {
+      if (!(valid && lane < cnt)) {
+        yx = yy = yz = FAR;
+        q = 0.0;
+      }
+      V4 v;
+      v.x = T(yx);
+      v.y = T(yy);
+      v.z = T(yz);
+      v.w = T(q);
+      sh.ys[lane] = v;
+      if (SPLIT)
+        sh.yl[lane] = make_float4(float(yx - double(float(yx))), float(yy - double(float(yy))),
+                                  float(yz - double(float(yz))), 0.0f);
+    }
+    __syncthreads();
+  };
+  // The near row is walked in chunks of up to 64 entries.  The own leaf's sources are
+  // computed apart (r^2 == 0 select); the other entries' sources form one stream, cut
+  // into full tiles of 64 whatever the leaf sizes, each lane staging a source of the
+  // entry its stream position falls in (frames and prefix sums in LDS).
+  for (uint32_t cb = e0; cb < e1; cb += TILE) {
+    const int nce = int((e1 - cb) < uint32_t(TILE) ? (e1 - cb) : uint32_t(TILE));
+    uint32_t st = 0, cnt = 0;
+    bool own = false;
+    double c[3] = {0.0, 0.0, 0.0}, r = 1.0;
+    if (lane < nce) {
+      const uint32_t sl = near_ent[cb + lane];
+      st = src_start[sl];
+      cnt = src_start[sl + 1] - st;
+      own = sl == lf;
+      if (own) cnt = 0;
+      relative_frame<double>(leaf_cell + 4 * size_t(sl), ct, c, r);
+    }
+    uint32_t inc = cnt;  // inclusive prefix sum over the lanes
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t v = __shfl_up(inc, off);
+      if (lane >= off) inc += v;
+    }
+    const uint32_t total = __shfl(inc, 63);
+    const bool has_own = __ballot(own) != 0;
+    __syncthreads();  // the previous chunk's tiles are done with the entry table
+    sh.fr[lane][0] = c[0];
+    sh.fr[lane][1] = c[1];
+    sh.fr[lane][2] = c[2];
+    sh.fr[lane][3] = r;
+    sh.fstart[lane] = st;
+    sh.fcum[lane + 1] = inc;
+    if (lane == 0) sh.fcum[0] = 0;
+    if (has_own) {
+      // the own leaf: y = u_s; coincident points add nothing
+      const uint32_t s0 = src_start[lf], s1 = src_start[lf + 1];
+      for (uint32_t sb = s0; sb < s1; sb += uint32_t(tsz)) {
+        const int cn = int((s1 - sb) < uint32_t(tsz) ? (s1 - sb) : uint32_t(tsz));
+        const int steps = (cn + phases - 1) / phases;
+        const uint32_t s = sb + uint32_t(lane);
+        const bool valid = s < s1;
+        stage(cn, steps, valid, valid ? sx[s] : 0.0, valid ? sy[s] : 0.0, valid ? sz[s] : 0.0,
+              valid ? sq[s] : 0.0);
+        for (int k2 = 0; k2 < steps; ++k2) step(phase + k2 * phases, std::true_type{});
+        flush();
+      }
+    } else {
+      __syncthreads();  // the entry table is visible to every lane
+    }
+    // stream position f of lane: entry e with fcum[e] <= f < fcum[e + 1]
+    uint32_t ea = 0;  // first entry of the current tile (uniform)
+    uint32_t pe = 0;
+    bool pvalid = false;
+    double px = 0.0, py = 0.0, pz = 0.0, pq = 0.0;
+    auto prefetch = [&](uint32_t base) {
+      while (sh.fcum[ea + 1] <= base) ++ea;
+      const uint32_t f = base + uint32_t(lane);
+      pvalid = f < total;
+      if (pvalid) {
+        uint32_t e = ea;
+        while (sh.fcum[e + 1] <= f) ++e;
+        pe = e;
+        const uint32_t s = sh.fstart[e] + (f - sh.fcum[e]);
+        px = sx[s];
+        py = sy[s];
+        pz = sz[s];
+        pq = sq[s];
+      }
+    };
+    if (total > 0) prefetch(0);
+    for (uint32_t base = 0; base < total; base += uint32_t(tsz)) {
+      const int cn = int((total - base) < uint32_t(tsz) ? (total - base) : uint32_t(tsz));
+      const int steps = (cn + phases - 1) / phases;
+      double yx = 0.0, yy = 0.0, yz = 0.0;
+      if (pvalid) {
+        yx = fma(sh.fr[pe][3], px, sh.fr[pe][0]);
+        yy = fma(sh.fr[pe][3], py, sh.fr[pe][1]);
+        yz = fma(sh.fr[pe][3], pz, sh.fr[pe][2]);
+      }
+      stage(cn, steps, pvalid, yx, yy, yz, pq);
+      // start the next tile's loads before computing this one
+      if (base + uint32_t(tsz) < total) prefetch(base + uint32_t(tsz));
+      int k2 = 0;
+      for (; k2 + 2 <= steps; k2 += 2) {
+        step(phase + k2 * phases, std::false_type{});
+        step(phase + (k2 + 1) * phases, std::false_type{});
+      }
+      if (k2 < steps) step(phase + k2 * phases, std::false_type{});
+      flush();
+    }
+  }
+  if (!SPLIT) {
+#pragma unroll
+    for (int a = 0; a < A; ++a) {
+      cp[a] = double(ap[a]);
+      cx[a] = double(ax[a]);
+      cy[a] = double(ay[a]);
+      cz[a] = double(az[a]);
+    }
+  }
+  // add the phases' partial sums (lanes slot + np f share their targets) in phase order,
+  // through the frame table's LDS (free once the row's tiles are done)
+  if (phases > 1) {
+#pragma unroll
+    for (int a = 0; a < A; ++a) {
+      __syncthreads();
+      sh.fr[lane][0] = cp[a];
+      sh.fr[lane][1] = cx[a];
+      sh.fr[lane][2] = cy[a];
+      sh.fr[lane][3] = cz[a];
+      __syncthreads();
+      if (phase == 0)
+        for (int f = 1; f < phases; ++f) {
+          const int o = f * np + slot;
+          cp[a] += sh.fr[o][0];
+          if (GRAD) {
+            cx[a] += sh.fr[o][1];
+            cy[a] += sh.fr[o][2];
+            cz[a] += sh.fr[o][3];
+          }
+        }
+    }
+    __syncthreads();  // the next chunk writes the frame table again
+  }
+#pragma unroll
+  for (int a = 0; a < A; ++a) {
+    const uint32_t i = tb + uint32_t(slot + a * np);
+    if (ok[a] && phase == 0) {
+      phi[i] += cp[a];
+      if (GRAD) {
+        grad[3 * size_t(i) + 0] += cx[a];
+        grad[3 * size_t(i) + 1] += cy[a];
+        grad[3 * size_t(i) + 2] += cz[a];
+      }
+    }
+  }
+}
+
 template <typename T, bool GRAD>
 __global__ __launch_bounds__(64) void k_p2p(uint32_t leaf_first, uint32_t count, uint32_t umin,
                                             const uint32_t *__restrict__ near_off,
@@ -421,29 +685,16 @@ __global__ __launch_bounds__(64) void k_p2p(uint32_t leaf_first, uint32_t count,
                                             const double *__restrict__ tx, const double *__restrict__ ty,
                                             const double *__restrict__ tz, double *__restrict__ phi,
                                             double *__restrict__ grad) {
-  constexpr bool SPLIT = sizeof(T) == 4;
-  constexpr int TILE = 64;
-  constexpr T TINY = sizeof(T) == 4 ? T(1.17549435e-38f) : T(2.2250738585072014e-308);
-  constexpr double FAR = 1024.0;  // padding position, in target-leaf units
-  // a source in LDS: (x, y, z, q) and, for the split form, (x_lo, y_lo, z_lo, 0), so a
-  // lane reads it with one or two 16-byte loads
-  using V4 = typename std::conditional<SPLIT, float4, double4>::type;
-  __shared__ V4 ys[TILE];
-  __shared__ float4 yl[SPLIT ? TILE : 1];
-  __shared__ double fr[TILE][4];       // frame (c, r) of each entry of a chunk of the near row
-  __shared__ uint32_t fstart[TILE];    // first source of each entry
-  __shared__ uint32_t fcum[TILE + 1];  // exclusive prefix sums of the entries' source counts
-  const int lane = threadIdx.x;
+  __shared__ P2pStage<T> sh;
   const uint32_t li = xcd_index(count);
   if (li >= count) return;
   const uint32_t lf = leaf_first + li;
   const uint32_t t0 = tgt_start[lf], t1 = tgt_start[lf + 1];
   if (t0 == t1) return;
-  const uint32_t *ct = leaf_cell + 4 * size_t(lf);
   const uint32_t e0 = near_off[lf], e1 = near_off[lf + 1];
   for (uint32_t tb = t0; tb < t1; tb += 128) {
     const uint32_t n = (t1 - tb) < 128u ? (t1 - tb) : 128u;
-    if (SPLIT && n >= umin) {
+    if (sizeof(T) == 4 && n >= umin) {
       if (n > 64)
         p2p_uniform<GRAD, true>(lf, tb, n, e0, e1, near_ent, leaf_cell, src_start, rec, near_close, sx, sy, sz, tx,
                                 ty, tz, phi, grad);
@@ -452,233 +703,16 @@ __global__ __launch_bounds__(64) void k_p2p(uint32_t leaf_first, uint32_t count,
                                  ty, tz, phi, grad);
       continue;
     }
-    // np = n lanes per phase and floor(64 / n) phases (a chunk of 17..21 targets runs 3
-    // phases, where the next power of two would allow 2); lanes past np x phases idle
-    int np = 64, phases = 1;
-    if (n <= 64) {
-      np = int(n);
-      phases = 64 / np;
-    }
-    const int tsz = phases * (64 / phases);  // sources per tile: a multiple of the phases
-    const bool lane_ok = lane < np * phases;
-    const int slot = lane % np, phase = lane_ok ? lane / np : 0;
-    const bool two = n > 64;
-    T ux[2], uy[2], uz[2], lx[2], ly[2], lz[2], ap[2], ax[2], ay[2], az[2];
-    bool ok[2];
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-      const uint32_t i = tb + slot + a * 64;
-      ok[a] = lane_ok && ((a == 0) ? (uint32_t(slot) < n) : (two && uint32_t(slot + 64) < n));
-      const double x = ok[a] ? tx[i] : 0.0, y = ok[a] ? ty[i] : 0.0, z = ok[a] ? tz[i] : 0.0;
-      ux[a] = T(x);
-      uy[a] = T(y);
-      uz[a] = T(z);
-      lx[a] = T(x - double(ux[a]));
-      ly[a] = T(y - double(uy[a]));
-      lz[a] = T(z - double(uz[a]));
-      ap[a] = ax[a] = ay[a] = az[a] = T(0);
-    }
-    // f32 sums are per tile (at most 64 terms) and go into f64 after each tile, so long
-    // near rows do not lose digits to one growing f32 sum
-    double cp[2] = {0.0, 0.0}, cx[2] = {0.0, 0.0}, cy[2] = {0.0, 0.0}, cz[2] = {0.0, 0.0};
-    auto flush = [&]() {
-      if (SPLIT) {
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-          cp[a] += double(ap[a]);
-          cx[a] += double(ax[a]);
-          cy[a] += double(ay[a]);
-          cz[a] += double(az[a]);
-          ap[a] = ax[a] = ay[a] = az[a] = T(0);
-        }
-      }
-    };
-    // one source j of the tile against the lane's targets
-    auto step = [&](int j, bool check) {
-      const V4 v = ys[j];
-      const T yx = v.x, yy = v.y, yz = v.z, q = v.w;
-      T yxl = T(0), yyl = T(0), yzl = T(0);
-      if (SPLIT) {
-        const float4 w = yl[j];
-        yxl = w.x;
-        yyl = w.y;
-        yzl = w.z;
-      }
-#pragma unroll
-      for (int a = 0; a < 2; ++a) {
-        if (a == 1 && !two) break;
-        T dx = ux[a] - yx, dy = uy[a] - yy, dz = uz[a] - yz;
-        if (SPLIT) {
-          dx += lx[a] - yxl;
-          dy += ly[a] - yyl;
-          dz += lz[a] - yzl;
-        }
-        const T r2 = dx * dx + dy * dy + dz * dz;
-        const T inv = check ? (r2 == T(0) ? T(0) : rsqrt_t<T>(r2)) : rsqrt_t<T>(r2 > TINY ? r2 : TINY);
-        const T qi = q * inv;
-        ap[a] += qi;
-        if (GRAD) {
-          const T qi3 = qi * (inv * inv);
-          ax[a] -= qi3 * dx;
-          ay[a] -= qi3 * dy;
-          az[a] -= qi3 * dz;
-        }
-      }
-    };
-    // stage one tile: lane < cnt holds the source (x, y, z, q) in the target frame;
-    // lanes cnt .. steps * phases - 1 hold zero charges far away
-    auto stage = [&](int cnt, int steps, bool valid, double yx, double yy, double yz, double q) {
-      __syncthreads();
-      if (lane < steps * phases) {
-        if (!(valid && lane < cnt)) {
-          yx = yy = yz = FAR;
-          q = 0.0;
-        }
-        V4 v;
-        v.x = T(yx);
-        v.y = T(yy);
-        v.z = T(yz);
-        v.w = T(q);
-        ys[lane] = v;
-        if (SPLIT)
-          yl[lane] = make_float4(float(yx - double(float(yx))), float(yy - double(float(yy))),
-                                 float(yz - double(float(yz))), 0.0f);
-      }
-      __syncthreads();
-    };
-    // The near row is walked in chunks of up to 64 entries.  The own leaf's sources are
-    // computed apart (r^2 == 0 select); the other entries' sources form one stream, cut
-    // into full tiles of 64 whatever the leaf sizes, each lane staging a source of the
-    // entry its stream position falls in (frames and prefix sums in LDS).
-    for (uint32_t cb = e0; cb < e1; cb += TILE) {
-      const int nce = int((e1 - cb) < uint32_t(TILE) ? (e1 - cb) : uint32_t(TILE));
-      uint32_t st = 0, cnt = 0;
-      bool own = false;
-      double c[3] = {0.0, 0.0, 0.0}, r = 1.0;
-      if (lane < nce) {
-        const uint32_t sl = near_ent[cb + lane];
-        st = src_start[sl];
-        cnt = src_start[sl + 1] - st;
-        own = sl == lf;
-        if (own) cnt = 0;
-        relative_frame<double>(leaf_cell + 4 * size_t(sl), ct, c, r);
-      }
-      uint32_t inc = cnt;  // inclusive prefix sum over the lanes
-#pragma unroll
-      for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t v = __shfl_up(inc, off);
-        if (lane >= off) inc += v;
-      }
-      const uint32_t total = __shfl(inc, 63);
-      const bool has_own = __ballot(own) != 0;
-      __syncthreads();  // the previous chunk's tiles are done with the entry table
-      fr[lane][0] = c[0];
-      fr[lane][1] = c[1];
-      fr[lane][2] = c[2];
-      fr[lane][3] = r;
-      fstart[lane] = st;
-      fcum[lane + 1] = inc;
-      if (lane == 0) fcum[0] = 0;
-      if (has_own) {
-        // the own leaf: y = u_s; coincident points add nothing
-        const uint32_t s0 = src_start[lf], s1 = src_start[lf + 1];
-        for (uint32_t sb = s0; sb < s1; sb += uint32_t(tsz)) {
-          const int cn = int((s1 - sb) < uint32_t(tsz) ? (s1 - sb) : uint32_t(tsz));
-          const int steps = (cn + phases - 1) / phases;
-          const uint32_t s = sb + uint32_t(lane);
-          const bool valid = s < s1;
-          stage(cn, steps, valid, valid ? sx[s] : 0.0, valid ? sy[s] : 0.0, valid ? sz[s] : 0.0,
-                valid ? sq[s] : 0.0);
-          for (int k2 = 0; k2 < steps; ++k2) step(phase + k2 * phases, true);
-          flush();
-        }
-      } else {
-        __syncthreads();  // the entry table is visible to every lane
-      }
-      // stream position f of lane: entry e with fcum[e] <= f < fcum[e + 1]
-      uint32_t ea = 0;  // first entry of the current tile (uniform)
-      uint32_t pe = 0;
-      bool pvalid = false;
-      double px = 0.0, py = 0.0, pz = 0.0, pq = 0.0;
-      auto prefetch = [&](uint32_t base) {
-        while (fcum[ea + 1] <= base) ++ea;
-        const uint32_t f = base + uint32_t(lane);
-        pvalid = f < total;
-        if (pvalid) {
-          uint32_t e = ea;
-          while (fcum[e + 1] <= f) ++e;
-          pe = e;
-          const uint32_t s = fstart[e] + (f - fcum[e]);
-          px = sx[s];
-          py = sy[s];
-          pz = sz[s];
-          pq = sq[s];
-        }
-      };
-      if (total > 0) prefetch(0);
-      for (uint32_t base = 0; base < total; base += uint32_t(tsz)) {
-        const int cn = int((total - base) < uint32_t(tsz) ? (total - base) : uint32_t(tsz));
-        const int steps = (cn + phases - 1) / phases;
-        double yx = 0.0, yy = 0.0, yz = 0.0;
-        if (pvalid) {
-          yx = fma(fr[pe][3], px, fr[pe][0]);
-          yy = fma(fr[pe][3], py, fr[pe][1]);
-          yz = fma(fr[pe][3], pz, fr[pe][2]);
-        }
-        stage(cn, steps, pvalid, yx, yy, yz, pq);
-        // start the next tile's loads before computing this one
-        if (base + uint32_t(tsz) < total) prefetch(base + uint32_t(tsz));
-        int k2 = 0;
-        for (; k2 + 2 <= steps; k2 += 2) {
-          step(phase + k2 * phases, false);
-          step(phase + (k2 + 1) * phases, false);
-        }
-        if (k2 < steps) step(phase + k2 * phases, false);
-        flush();
-      }
-    }
-    if (!SPLIT) {
-#pragma unroll
-      for (int a = 0; a < 2; ++a) {
-        cp[a] = double(ap[a]);
-        cx[a] = double(ax[a]);
-        cy[a] = double(ay[a]);
-        cz[a] = double(az[a]);
-      }
-    }
-    // add the phases' partial sums (lanes slot + np f share a target) in phase order,
-    // through the frame table's LDS (free once the row's tiles are done)
-    if (phases > 1) {
-      __syncthreads();
-      fr[lane][0] = cp[0];
-      fr[lane][1] = cx[0];
-      fr[lane][2] = cy[0];
-      fr[lane][3] = cz[0];
-      __syncthreads();
-      if (phase == 0)
-        for (int f = 1; f < phases; ++f) {
-          const int o = f * np + slot;
-          cp[0] += fr[o][0];
-          if (GRAD) {
-            cx[0] += fr[o][1];
-            cy[0] += fr[o][2];
-            cz[0] += fr[o][3];
-          }
-        }
-      __syncthreads();  // the next chunk writes the frame table again
-    }
-#pragma unroll
-    for (int a = 0; a < 2; ++a) {
-      const uint32_t i = tb + slot + a * 64;
-      if (ok[a] && phase == 0) {
-        phi[i] += cp[a];
-        if (GRAD) {
-          grad[3 * size_t(i) + 0] += cx[a];
-          grad[3 * size_t(i) + 1] += cy[a];
-          grad[3 * size_t(i) + 2] += cz[a];
-        }
-      }
-    }
+    // two targets per lane unless one fills more of the lanes' target slots: 18 targets are
+    // 3 phases of 18 lanes (54 of 64 slots) or 7 phases of 9 lanes (126 of 128), and two
+    // targets share each source's LDS reads
+    const int slots1 = n <= 64 ? int(n) * (64 / int(n)) : 0, slots2 = int(n) * (64 / staged_lanes(n, 2));
+    if (2 * slots1 > slots2)
+      p2p_staged<T, GRAD, 1>(sh, lf, tb, n, e0, e1, near_ent, leaf_cell, src_start, sx, sy, sz, sq, tx, ty, tz, phi,
+                             grad);
+    else
+      p2p_staged<T, GRAD, 2>(sh, lf, tb, n, e0, e1, near_ent, leaf_cell, src_start, sx, sy, sz, sq, tx, ty, tz, phi,
+                             grad);
   }
 }
 
@@ -1033,7 +1067,7 @@ __device__ __forceinline__ void wave_sync() {
 }
 
 template <bool GRAD>
-__global__ __launch_bounds__(512) void k_m2p(int p, int wave_doubles, uint32_t rows, const uint32_t *row_leaf,
+__global__ __launch_bounds__(512, 4) void k_m2p(int p, int wave_doubles, uint32_t rows, const uint32_t *row_leaf,
                                              const uint32_t *row_off, const uint32_t *row_box,
                                              const uint32_t *box_cell, const uint32_t *leaf_cell,
                                              const uint32_t *tgt_start, const double *tx, const double *ty,
@@ -1041,7 +1075,7 @@ __global__ __launch_bounds__(512) void k_m2p(int p, int wave_doubles, uint32_t r
   extern __shared__ __align__(16) double eval_smem[];
   constexpr int ED = GRAD ? 8 : 2;  // doubles per entry
   constexpr int ME = (kMaxDegree + 2) * (kMaxDegree + 3) / 2;
-  constexpr int EL = (ME + 63) / 64;  // entries per lane
+  __shared__ uint8_t en[ME], em[ME];  // (n, m) of the entries
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, W = blockDim.x >> 6;
   const int nc = (p + 1) * (p + 1), ptop = GRAD ? p + 1 : p;
   const int ne = (ptop + 1) * (ptop + 2) / 2;
@@ -1051,18 +1085,17 @@ __global__ __launch_bounds__(512) void k_m2p(int p, int wave_doubles, uint32_t r
   const uint32_t t0 = tgt_start[lf], t1 = tgt_start[lf + 1];
   if (t0 == t1) return;
   double *E = eval_smem + size_t(wave) * wave_doubles;
-  // (n, m) of the entries this lane fills: columns m = 0 .. ptop, each n = m .. ptop
-  int en[EL], em[EL];
-#pragma unroll
-  for (int k = 0; k < EL; ++k) {
-    int t = lane + 64 * k, m = 0;
-    while (m <= ptop && t >= ptop + 1 - m) {
+  // columns m = 0 .. ptop, each n = m .. ptop
+  for (int k = int(threadIdx.x); k < ne; k += int(blockDim.x)) {
+    int t = k, m = 0;
+    while (t >= ptop + 1 - m) {
       t -= ptop + 1 - m;
       ++m;
     }
-    en[k] = m + t;
-    em[k] = m;
+    en[k] = uint8_t(m + t);
+    em[k] = uint8_t(m);
   }
+  __syncthreads();
   const uint32_t nt = t1 - t0;
   const int L = sub_lanes(nt);
   const int per = 64 / L;  // targets per pass
@@ -1080,29 +1113,27 @@ __global__ __launch_bounds__(512) void k_m2p(int p, int wave_doubles, uint32_t r
       relative_frame<double>(box_cell + 4 * size_t(box), leaf_cell + 4 * size_t(lf), c, r);
       const double *M = coeffs + size_t(box) * nc;
       wave_sync();  // the previous box's entries are read
-#pragma unroll
-      for (int k = 0; k < EL; ++k)
-        if (lane + 64 * k < ne) {
-          const int n = en[k], m = em[k];
-          const double w = m == 0 ? 1.0 : 2.0;
-          double *o = E + (lane + 64 * k) * ED;
-          double cr, ci;
-          read_order(M, n, m, p, cr, ci);
-          o[0] = w * cr;
-          o[1] = w * ci;
-          if (GRAD) {
-            double ar, ai, br, bi, zr, zi;
-            read_order(M, n - 1, m + 1, p, ar, ai);
-            read_order(M, n - 1, m - 1, p, br, bi);
-            read_order(M, n - 1, m, p, zr, zi);
-            o[2] = 0.5 * w * (ar - br);
-            o[3] = m > 0 ? 0.5 * w * (ai - bi) : 0.0;
-            o[4] = -0.5 * w * (ai + bi);
-            o[5] = m > 0 ? 0.5 * w * (ar + br) : 0.0;
-            o[6] = -w * zr;
-            o[7] = m > 0 ? -w * zi : 0.0;
-          }
+      for (int k = lane; k < ne; k += 64) {
+        const int n = en[k], m = em[k];
+        const double w = m == 0 ? 1.0 : 2.0;
+        double *o = E + k * ED;
+        double cr, ci;
+        read_order(M, n, m, p, cr, ci);
+        o[0] = w * cr;
+        o[1] = w * ci;
+        if (GRAD) {
+          double ar, ai, br, bi, zr, zi;
+          read_order(M, n - 1, m + 1, p, ar, ai);
+          read_order(M, n - 1, m - 1, p, br, bi);
+          read_order(M, n - 1, m, p, zr, zi);
+          o[2] = 0.5 * w * (ar - br);
+          o[3] = m > 0 ? 0.5 * w * (ai - bi) : 0.0;
+          o[4] = -0.5 * w * (ai + bi);
+          o[5] = m > 0 ? 0.5 * w * (ar + br) : 0.0;
+          o[6] = -w * zr;
+          o[7] = m > 0 ? -w * zi : 0.0;
         }
+      }
       wave_sync();
       if (valid) {
         const double inv_r = 1.0 / r;  // a power of two
