@@ -85,6 +85,8 @@ __host__ __device__ static inline void split3(double x, uint16_t &hi, uint16_t &
   lo = bf16_bits(float(r2));
 }
 
+void split_bf16x3(double x, uint16_t s[3]) { split3(x, s[0], s[1], s[2]); }
+
 // [ks][plane][mt][lane][e]: row = 16 mt + lane % 16, k = 32 ks + 8 (lane / 16) + e
 void swizzle_table_bf16(int p, const double *a, uint16_t *out) {
   const int nc = (p + 1) * (p + 1), MT = m_tiles(p), KS = k_steps16(p);

@@ -175,6 +175,8 @@ size_t swizzled_table_size_bf16(int p);
 size_t split_expansion_size(int p);
 void swizzle_table(int p, const double *table_colmajor, double *out);
 void swizzle_table_bf16(int p, const double *table_colmajor, uint16_t *out);
+// x = s[0] + s[1] + s[2] in bf16 (24 bits)
+void split_bf16x3(double x, uint16_t s[3]);
 
 }  // namespace dev
 }  // namespace fmmh

@@ -17,6 +17,7 @@
 
 #include "plan.hpp"
 #include "pwkernels.hpp"
+#include "reflect.hpp"
 
 namespace fmmh {
 
@@ -162,8 +163,10 @@ class DeviceOperator {
   // the bf16x3 M2L's pipeline stage shape (Tuning::m2l_stage), from the next launch
   void set_m2l_stage(int stage) { opt_.tuning.m2l_stage = stage; }
   int p2p_uniform_min() const { return opt_.tuning.p2p_uniform_min > 0 ? opt_.tuning.p2p_uniform_min : 33; }
-  // the M2L mode each level's schedule took: 0 none, 1 box mode, 2 clustered mode
+  // the M2L mode each level's schedule took: 0 none or by reflection classes, 1 box mode,
+  // 2 clustered mode
   int m2l_mode_of(int level) const { return level >= 0 && level < kTuneLevels ? m2l_mode_taken_[level] : 0; }
+  bool m2l_reflected(int level) const { return level + 1 < int(rf_level_task_.size()) && rf_level_task_[level + 1] > rf_level_task_[level]; }
   int l2l_width_of(int level) const { return level >= 0 && level < int(l2l_.size()) ? l2l_[level].width : 0; }
 
   int nlevels() const { return nlevels_; }
@@ -173,15 +176,17 @@ class DeviceOperator {
   const OperatorOptions &options() const { return opt_; }
   // statistics for reports and the roofline
   uint64_t p2p_pairs() const { return p2p_pairs_; }
-  uint64_t m2l_pairs() const { return m2l_.pairs; }
-  uint64_t m2l_slots() const { return m2l_.slots; }
+  uint64_t m2l_pairs() const { return m2l_.pairs + rf_pairs_; }
+  uint64_t m2l_slots() const { return m2l_.slots + rf_slots_issued_; }
   size_t device_bytes() const;
   double *device_locals() const { return loc_.ptr; }
   double *device_multipoles() const { return mult_.ptr; }
   size_t nboxes_total() const { return nbox_total_; }
 
  private:
-  void build_schedules(const Plan &plan);
+  void build_schedules(const Plan &plan, const std::vector<char> &reflected);
+  std::vector<char> reflected_levels(const Plan &plan) const;
+  void build_reflect(const Plan &plan, const std::vector<char> &levels, const std::vector<double> &m2l);
   template <class F>
   void timed(int kind, F &&f);
   void collect_timings();
@@ -273,6 +278,20 @@ class DeviceOperator {
   std::vector<uint32_t> m2l_level_task_;                     // task range per level
   Rows m2l_red_;                                             // clustered-mode reductions
   std::vector<uint32_t> m2l_red_level_;
+
+  // M2L by reflection classes (reflect.hpp): the levels that take it, their target rows
+  // and tasks (by level), the class tables and the multipoles sorted by parity
+  dev::ReflectArgs rf_{};
+  DevBuf<uint32_t> rf_first_, rf_row_box_, rf_src_;
+  DevBuf<uint16_t> rf_tables16_;
+  DevBuf<uint64_t> rf_kmask_;
+  DevBuf<uint8_t> rf_parity_, rf_tile_class_, rf_row_flip_;
+  DevBuf<int32_t> rf_perm_, rf_tile_row_;
+  DevBuf<dev::ReflectTask> rf_tasks_;
+  DevBuf<double> rf_tables_, rf_sorted_, rf_scratch_;
+  std::vector<uint32_t> rf_level_task_, rf_red_level_;
+  Rows rf_red_;
+  uint64_t rf_pairs_ = 0, rf_slots_issued_ = 0;
 };
 
 // Compensated f64 direct sum on the device (unscaled sums q / r and their gradient):

@@ -10,7 +10,8 @@
 //   - P2P (mixed precision): the chunk size from which targets read their sources by
 //     uniform loads instead of LDS tiles with phases: 33 (static), 17, 49, 65, never;
 //   - M2L per level: box mode (tiles of 128 targets of one octant walking their offsets)
-//     or clustered mode (scratch rows per target and parent-level neighbour);
+//     or clustered mode (scratch rows per target and parent-level neighbour), and where the
+//     static rule takes the reflection classes, those (decision 0) or clustered mode;
 //   - L2L per level: 16, 64 or 128 columns per task;
 //   - M2M per parent level: the per-tile form or the split form;
 //   - the bf16x3 M2L's pipeline stage: one k-step per stage (ring of three) or two (ring
@@ -141,7 +142,7 @@ void autotune(const Plan &plan, const OperatorOptions &options, double budget_s,
   OperatorOptions ob = oa, oc = oa, od = oa;
   for (int l = 0; l < std::min(L, kTuneLevels); ++l) {
     const int m = A->m2l_mode_of(l);
-    ob.tuning.m2l_mode[l] = m == 1 ? 2 : m == 2 ? 1 : 0;
+    ob.tuning.m2l_mode[l] = m == 1 || A->m2l_reflected(l) ? 2 : m == 2 ? 1 : 0;
     ob.tuning.l2l_width[l] = 16;
     ob.tuning.m2m_form[l] = 1;
     oc.tuning.l2l_width[l] = 64;
@@ -157,7 +158,7 @@ void autotune(const Plan &plan, const OperatorOptions &options, double budget_s,
 
   for (int l = 0; l < std::min(L, kTuneLevels); ++l) {
     // M2L: the static mode (A) against the other (B)
-    if (options.m2l == kM2lDense && ops[0]->m2l_mode_of(l) != 0) {
+    if (options.m2l == kM2lDense && (ops[0]->m2l_mode_of(l) != 0 || ops[0]->m2l_reflected(l))) {
       double best = std::numeric_limits<double>::infinity();
       for (int k = 0; k < 2; ++k) {
         DeviceOperator &op = *ops[k];

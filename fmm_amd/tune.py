@@ -34,7 +34,7 @@ from . import _lib
 
 CACHE_NAME = "fmm_amd_tuning.json"
 # bump when a candidate set or a decision's meaning changes: older files are ignored
-CANDIDATE_SET_VERSION = 1
+CANDIDATE_SET_VERSION = 2
 KINDS = ("p2p", "m2l", "l2l", "m2m", "stage")
 P2P_CANDIDATES = (33, 17, 49, 65, 129)
 

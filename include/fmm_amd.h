@@ -171,7 +171,7 @@ typedef struct {
                               uniform loads, smaller ones through LDS tiles (0: 33) */
   int32_t m2l_stage;       /* mixed dense M2L: 0 or 1 one k-step per pipeline stage, 2 two k-steps
                               in a ring of two LDS buffers (where the table fits) */
-  int32_t m2l_mode[17];    /* dense M2L of the level: 0 static rule, 1 box mode, 2 clustered */
+  int32_t m2l_mode[17];    /* dense M2L of the level: 0 static rule (by density: reflection classes, box or clustered mode), 1 box mode, 2 clustered */
   int32_t l2l_width[17];   /* L2L into the level: 0 static rule, or 16, 64, 128 columns per task */
   int32_t m2m_form[17];    /* M2M into the parents of the level: 0 static, 1 per-tile, 2 split */
 } fmmh_tuning;

@@ -48,3 +48,28 @@ def test_m2p_rows_over_waves(p, leaf, gradients):
     rows = [len(fmm.plan.list("w", level)[1]) for level in range(fmm.plan.nlevels)]
     assert sum(rows) > 0
     _check(fmm, O.Fmm(pts, p=p, leaf_points=leaf, gradients=gradients), q, gradients)
+
+
+@pytest.mark.parametrize("precision,tol", [("f64", 1e-12), ("mixed", 1e-6)])
+@pytest.mark.parametrize("p", [5, 6, 8, 10, 11, 12, 13, 14, 15])
+def test_m2l_reflection_classes(p, precision, tol):
+    """Dense levels at every count of row tiles (8 to 20) and of coefficient chunks, boundary
+    boxes (sources missing at some reflections), target rows that do not fill a workgroup."""
+    _log(f"case M2L reflection p={p} {precision}")
+    rng = O.Rng(91 + p)
+    pts = np.vstack([rng.cube(4500), rng.plummer(1500, (0.4, 0.6, 0.5), 0.03)])
+    q = rng.normals(len(pts))
+    fmm = fmm_amd.FmmBuilder(p).max_points_per_leaf(24).precision(precision).build(pts)
+    _check(fmm, O.Fmm(pts, p=p, leaf_points=24), q, tol=tol)
+
+
+def test_m2l_reflection_level_calls():
+    """The level calls run each level's share of the tasks (whole and split into parts)."""
+    _log("case M2L reflection, level by level")
+    rng = O.Rng(92)
+    pts = rng.cube(60000)
+    q = rng.normals(len(pts))
+    fmm = fmm_amd.FmmBuilder(7).max_points_per_leaf(8).build(pts)
+    a, b = fmm.evaluate(q), fmm.evaluate_levels(q)
+    assert O.error_norms(b.potential, a.potential)[0] < 1e-14
+    assert O.error_norms(b.gradient, a.gradient, True)[0] < 1e-14
