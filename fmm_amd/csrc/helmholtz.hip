@@ -510,25 +510,61 @@ __global__ __launch_bounds__(64) void k_h_evaluate(int p, uint32_t rows, const u
 }
 
 // ---- P2P ---------------------------------------------------------------------------------
-// One wave per target leaf.  Lanes are (phase, target): with n_t <= 32 targets the wave
-// runs 64 / n_t phases that split each source tile; phases are added in order at the end.
-// Every near leaf's sources go through LDS in tiles of 64 with y^ = c^ + r^ u_s formed in
-// f64.  A pair with r^2 == 0 adds nothing (selects, no branch).  T = float: separations
-// from double-float coordinates (hi + lo), the pair arithmetic in f32, each source leaf's
-// f32 sums added to f64 accumulators.
-// Pair kernel pieces per precision.  f64: sqrt, division and sincos of the math library.
-// f32: 1/r from v_rsq_f32 (1 ulp) and r = r^2 / r; sine and cosine from v_sin_f32 and
-// v_cos_f32 of the fraction of x / (2 pi).
+// One workgroup of kP2pWaves waves per target leaf; wave w takes the near entries w, w +
+// kP2pWaves, ... of the leaf's row, and the waves' f64 sums are added in wave order, so a
+// few large leaves do not hold up the launch (80,000 Plummer points: 1,905 leaves, one of
+// them with 30 times the mean's pairs).  Within a wave lanes are (phase, target slot), one
+// or two targets per lane (the fuller use of the lanes), the phases splitting each source
+// tile; phases are added in order at the end.  A near leaf's sources go through the wave's
+// LDS in tiles of 64 with y^ = c^ + r^ u_s formed in f64.  A pair with r^2 == 0 adds nothing
+// (selects, no branch).  T = float: separations from double-float coordinates (hi + lo), the
+// pair arithmetic in f32, each source leaf's f32 sums added to f64 accumulators.
+// Pair kernel pieces per precision.  f64: 1/r by v_rsq_f64 and a third-order step, r = r^2 /
+// r corrected once, sine and cosine as below (300 cycles per 64 pairs against 830 with the
+// math library's sqrt, division and sincos, whose reductions for huge arguments it carries
+// along).  f32: 1/r from v_rsq_f32 (1 ulp) and r = r^2 / r; sine and cosine from v_sin_f32
+// and v_cos_f32 of the fraction of x / (2 pi).
+constexpr int kP2pWaves = 4;
+
 template <typename T>
 struct PairMath;
 
 template <>
 struct PairMath<double> {
   __device__ static __forceinline__ void rinv(double r2, double &r, double &ir) {
-    r = sqrt(r2);
-    ir = r2 == 0.0 ? 0.0 : 1.0 / r;
+    double y = __builtin_amdgcn_rsq(r2);
+    const double e = fma(-r2 * y, y, 1.0);
+    y = fma(y * e, fma(0.375, e, 0.5), y);
+    ir = r2 == 0.0 ? 0.0 : y;
+    r = r2 * ir;
+    r = fma(0.5 * ir, fma(-r, r, r2), r);
   }
-  __device__ static __forceinline__ void sincos(double x, double *s, double *c) { ::sincos(x, s, c); }
+  // x = n pi/2 + t, |t| <= pi/4, with pi/2 as the sum of two doubles (Cody and Waite); sine
+  // and cosine of t by polynomials in t^2 through the Chebyshev points of [0, (pi/4)^2]
+  // (errors 1.8e-17 and 9e-19, below the rounding); the quadrant selects and signs.  For
+  // |x| < 2^31, far beyond any k r of a leaf pair.
+  __device__ static __forceinline__ void sincos(double x, double *s, double *c) {
+    constexpr double kShift = 6755399441055744.0;  // 1.5 2^52: the sum's low bits are rint(x 2/pi)
+    const double m = fma(x, 0.6366197723675814, kShift), n = m - kShift;
+    const int q = __double2loint(m);
+    double t = fma(-n, 1.5707963267948966, x);
+    t = fma(-n, 6.123233995736766e-17, t);
+    const double z = t * t;
+    double ps = fma(z, 1.5918115263265974e-10, -2.505113165023518e-08);
+    ps = fma(z, ps, 2.7557316101617874e-06);
+    ps = fma(z, ps, -0.00019841269836756774);
+    ps = fma(z, ps, 0.008333333333330948);
+    ps = fma(z, ps, -0.16666666666666666);
+    double pc = fma(z, -1.1382623647474604e-11, 2.087614614655861e-09);
+    pc = fma(z, pc, -2.7557317271145144e-07);
+    pc = fma(z, pc, 2.480158729876456e-05);
+    pc = fma(z, pc, -0.0013888888888887398);
+    pc = fma(z, pc, 0.041666666666666664);
+    const double st = fma(t * z, ps, t), ct = fma(z * z, pc, fma(-0.5, z, 1.0));
+    const double sv = (q & 1) ? ct : st, cv = (q & 1) ? st : ct;
+    *s = __hiloint2double(__double2hiint(sv) ^ ((q << 30) & int(0x80000000)), __double2loint(sv));
+    *c = __hiloint2double(__double2hiint(cv) ^ (((q + 1) << 30) & int(0x80000000)), __double2loint(cv));
+  }
 };
 
 template <>
@@ -556,8 +592,25 @@ struct PairMath<float> {
 // e^{i k_t r_t} / r_t = rho e^{i k' r'} / r' and its gradient is rho^2 (i k' r' - 1)
 // e^{i k' r'} d' / r'^3, so an entry's f32 sums (at most 128 sources) go into the f64
 // sums scaled by rho and rho^2 (powers of two).
+//
+// The waves' sums of a chunk meet in red ([wave - 1][sum][lane]) and are added in wave order
+// by wave 0, which keeps them; every wave comes here.
+__device__ __forceinline__ void add_waves(int wave, int lane, double (&acc)[8], double (*red)[8][64]) {
+  __syncthreads();
+  if (wave > 0)
+#pragma unroll
+    for (int q = 0; q < 8; ++q) red[wave - 1][q][lane] = acc[q];
+  __syncthreads();
+  if (wave == 0)
+#pragma unroll
+    for (int w = 0; w < kP2pWaves - 1; ++w)
+#pragma unroll
+      for (int q = 0; q < 8; ++q) acc[q] += red[w][q][lane];
+}
+
 template <bool GRAD, bool DAMP, bool TWO>
-__device__ __forceinline__ void h_p2p_uniform(uint32_t lf, uint32_t tb, uint32_t n, uint32_t e0, uint32_t e1,
+__device__ __forceinline__ void h_p2p_uniform(double (*red)[8][64], uint32_t lf, uint32_t tb, uint32_t n,
+                                              uint32_t e0, uint32_t e1,
                                               const uint32_t *__restrict__ near_ent,
                                               const uint32_t *__restrict__ leaf_cell,
                                               const uint32_t *__restrict__ src_start,
@@ -566,7 +619,7 @@ __device__ __forceinline__ void h_p2p_uniform(uint32_t lf, uint32_t tb, uint32_t
                                               const double *__restrict__ tz, double *__restrict__ phi_hat,
                                               double *__restrict__ grad_hat) {
   constexpr int A = TWO ? 2 : 1;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
   double u[A][3];
   bool ok[A];
 #pragma unroll
@@ -583,7 +636,7 @@ __device__ __forceinline__ void h_p2p_uniform(uint32_t lf, uint32_t tb, uint32_t
 #pragma unroll
     for (int q = 0; q < 8; ++q) acc[a][q] = 0.0;
   const uint32_t *ct = leaf_cell + 4 * size_t(lf);
-  for (uint32_t e = e0; e < e1; ++e) {
+  for (uint32_t e = e0 + uint32_t(wave); e < e1; e += kP2pWaves) {
     const uint32_t sl = near_ent[e];
     const uint32_t s0 = src_start[sl], s1 = src_start[sl + 1];
     if (s0 == s1) continue;
@@ -666,7 +719,8 @@ __device__ __forceinline__ void h_p2p_uniform(uint32_t lf, uint32_t tb, uint32_t
   }
 #pragma unroll
   for (int a = 0; a < A; ++a) {
-    if (!ok[a]) continue;
+    add_waves(wave, lane, acc[a], red);
+    if (wave > 0 || !ok[a]) continue;
     const size_t t = tb + uint32_t(lane + 64 * a);
     phi_hat[2 * t] += acc[a][0];
     phi_hat[2 * t + 1] += acc[a][1];
@@ -676,91 +730,82 @@ __device__ __forceinline__ void h_p2p_uniform(uint32_t lf, uint32_t tb, uint32_t
   }
 }
 
-template <typename T, bool GRAD, bool DAMP>
-__global__ __launch_bounds__(64) void k_h_p2p(uint32_t leaf_first, uint32_t count,
-                                              const uint32_t *__restrict__ near_off,
-                                              const uint32_t *__restrict__ near_ent,
-                                              const uint32_t *__restrict__ leaf_cell,
-                                              const uint32_t *__restrict__ src_start,
-                                              const uint32_t *__restrict__ tgt_start, const double *__restrict__ sx,
-                                              const double *__restrict__ sy, const double *__restrict__ sz,
-                                              const double *__restrict__ qr, const double *__restrict__ qi,
-                                              const float4 *__restrict__ rec, const double *__restrict__ tx,
-                                              const double *__restrict__ ty, const double *__restrict__ tz,
-                                              const double *__restrict__ hlev, double *__restrict__ phi_hat,
-                                              double *__restrict__ grad_hat) {
+template <typename T>
+struct HP2pStage {
+  T ys[kP2pWaves][64][8];  // per wave: y hi (3), y lo (3, f32 only), q re, q im
+  double red[kP2pWaves - 1][8][64];
+};
+
+// A chunk of n targets, A per lane: np = ceil(n / A) lanes per phase, floor(64 / np) phases.
+template <typename T, bool GRAD, bool DAMP, int A>
+__device__ __forceinline__ void h_p2p_staged(HP2pStage<T> &sh, uint32_t lf, uint32_t tb, uint32_t n, uint32_t e0,
+                                             uint32_t e1, T kre, T kim, const uint32_t *__restrict__ near_ent,
+                                             const uint32_t *__restrict__ leaf_cell,
+                                             const uint32_t *__restrict__ src_start, const double *__restrict__ sx,
+                                             const double *__restrict__ sy, const double *__restrict__ sz,
+                                             const double *__restrict__ qr, const double *__restrict__ qi,
+                                             const double *__restrict__ tx, const double *__restrict__ ty,
+                                             const double *__restrict__ tz, double *__restrict__ phi_hat,
+                                             double *__restrict__ grad_hat) {
   constexpr bool F32 = sizeof(T) == 4;
-  __shared__ T ys[64][8];  // y hi (3), y lo (3, f32 only), q re, q im
-  __shared__ double red[64][8];
-  const uint32_t item = xcd_index(count);
-  if (item >= count) return;
-  const uint32_t lf = leaf_first + item;
-  const uint32_t t0 = tgt_start[lf], t1 = tgt_start[lf + 1];
-  if (t1 == t0) return;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  T(*ys)[8] = sh.ys[wave];
   const uint32_t *ct = leaf_cell + 4 * size_t(lf);
-  const int lev = int(ct[0]);
-  const T kre = T(hlev[4 * lev]), kim = T(hlev[4 * lev + 1]);
-  const uint32_t ntl = t1 - t0;
-  if (F32 && ntl > 32) {
-    const uint32_t e0 = near_off[lf], e1 = near_off[lf + 1];
-    for (uint32_t tb = t0; tb < t1; tb += 128) {
-      const uint32_t n = (t1 - tb) < 128u ? (t1 - tb) : 128u;
-      if (n > 64)
-        h_p2p_uniform<GRAD, DAMP, true>(lf, tb, n, e0, e1, near_ent, leaf_cell, src_start, rec, hlev, tx, ty, tz,
-                                        phi_hat, grad_hat);
-      else
-        h_p2p_uniform<GRAD, DAMP, false>(lf, tb, n, e0, e1, near_ent, leaf_cell, src_start, rec, hlev, tx, ty, tz,
-                                         phi_hat, grad_hat);
-    }
-    return;
+  const int np = (int(n) + A - 1) / A, phases = 64 / np;
+  const int slot = lane % np, ph = lane / np;
+  bool ok[A];
+  T xh[A], yh[A], zh[A], xl[A], yl[A], zl[A];
+  double acc[A][8];
+#pragma unroll
+  for (int a = 0; a < A; ++a) {
+    const uint32_t t = tb + uint32_t(slot + a * np);
+    ok[a] = ph < phases && uint32_t(slot + a * np) < n;
+    const double ux = ok[a] ? tx[t] : 0.0, uy = ok[a] ? ty[t] : 0.0, uz = ok[a] ? tz[t] : 0.0;
+    xh[a] = T(ux);
+    yh[a] = T(uy);
+    zh[a] = T(uz);
+    xl[a] = F32 ? T(ux - double(xh[a])) : T(0);
+    yl[a] = F32 ? T(uy - double(yh[a])) : T(0);
+    zl[a] = F32 ? T(uz - double(zh[a])) : T(0);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) acc[a][q] = 0.0;
   }
-  const int phases = ntl >= 64 ? 1 : (ntl > 32 ? 1 : int(64 / ntl));
-  const int span = ntl >= 64 ? 64 : int(ntl);  // targets per chunk
-  for (uint32_t tb = t0; tb < t1; tb += uint32_t(span)) {
-    const int j = lane % span, ph = lane / span;
-    const uint32_t t = tb + uint32_t(j);
-    const bool active = ph < phases && t < t1;
-    double ux = 0.0, uy = 0.0, uz = 0.0;
-    if (active) {
-      ux = tx[t];
-      uy = ty[t];
-      uz = tz[t];
-    }
-    const T xh = T(ux), yh = T(uy), zh = T(uz);
-    const T xl = F32 ? T(ux - double(xh)) : T(0), yl = F32 ? T(uy - double(yh)) : T(0),
-            zl = F32 ? T(uz - double(zh)) : T(0);
-    double acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (uint32_t e = near_off[lf]; e < near_off[lf + 1]; ++e) {
-      const uint32_t sl = near_ent[e];
-      const uint32_t s0 = src_start[sl], s1 = src_start[sl + 1];
-      double c[3] = {0.0, 0.0, 0.0}, r = 1.0;
-      if (sl != lf) cell_frame(leaf_cell + 4 * size_t(sl), ct, c, r);  // c^(s|t), r^(s|t)
-      T loc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-      for (uint32_t sb = s0; sb < s1; sb += 64) {
-        const int cnt = int((s1 - sb) < 64u ? (s1 - sb) : 64u);
-        __syncthreads();
-        if (lane < cnt) {
-          const uint32_t s = sb + lane;
-          const double y0 = fma(r, sx[s], c[0]), y1 = fma(r, sy[s], c[1]), y2 = fma(r, sz[s], c[2]);
-          const T h0 = T(y0), h1 = T(y1), h2 = T(y2);
-          ys[lane][0] = h0;
-          ys[lane][1] = h1;
-          ys[lane][2] = h2;
-          ys[lane][3] = F32 ? T(y0 - double(h0)) : T(0);
-          ys[lane][4] = F32 ? T(y1 - double(h1)) : T(0);
-          ys[lane][5] = F32 ? T(y2 - double(h2)) : T(0);
-          ys[lane][6] = T(qr[s]);
-          ys[lane][7] = T(qi[s]);
-        }
-        __syncthreads();
-        if (active)
-          for (int i = ph; i < cnt; i += phases) {
-            T dx = xh - ys[i][0], dy = yh - ys[i][1], dz = zh - ys[i][2];
+  for (uint32_t e = e0 + uint32_t(wave); e < e1; e += kP2pWaves) {
+    const uint32_t sl = near_ent[e];
+    const uint32_t s0 = src_start[sl], s1 = src_start[sl + 1];
+    double c[3] = {0.0, 0.0, 0.0}, r = 1.0;
+    if (sl != lf) cell_frame(leaf_cell + 4 * size_t(sl), ct, c, r);  // c^(s|t), r^(s|t)
+    T loc[A][8];
+#pragma unroll
+    for (int a = 0; a < A; ++a)
+#pragma unroll
+      for (int q = 0; q < 8; ++q) loc[a][q] = T(0);
+    for (uint32_t sb = s0; sb < s1; sb += 64) {
+      const int cnt = int((s1 - sb) < 64u ? (s1 - sb) : 64u);
+      wave_sync();  // the previous tile is read
+      if (lane < cnt) {
+        const uint32_t s = sb + uint32_t(lane);
+        const double y0 = fma(r, sx[s], c[0]), y1 = fma(r, sy[s], c[1]), y2 = fma(r, sz[s], c[2]);
+        const T h0 = T(y0), h1 = T(y1), h2 = T(y2);
+        ys[lane][0] = h0;
+        ys[lane][1] = h1;
+        ys[lane][2] = h2;
+        ys[lane][3] = F32 ? T(y0 - double(h0)) : T(0);
+        ys[lane][4] = F32 ? T(y1 - double(h1)) : T(0);
+        ys[lane][5] = F32 ? T(y2 - double(h2)) : T(0);
+        ys[lane][6] = T(qr[s]);
+        ys[lane][7] = T(qi[s]);
+      }
+      wave_sync();
+      if (ph < phases)
+        for (int i = ph; i < cnt; i += phases) {
+#pragma unroll
+          for (int a = 0; a < A; ++a) {
+            T dx = xh[a] - ys[i][0], dy = yh[a] - ys[i][1], dz = zh[a] - ys[i][2];
             if (F32) {
-              dx += xl - ys[i][3];
-              dy += yl - ys[i][4];
-              dz += zl - ys[i][5];
+              dx += xl[a] - ys[i][3];
+              dy += yl[a] - ys[i][4];
+              dz += zl[a] - ys[i][5];
             }
             const T r2 = dx * dx + dy * dy + dz * dz;
             T rr, ir;
@@ -770,39 +815,87 @@ __global__ __launch_bounds__(64) void k_h_p2p(uint32_t leaf_first, uint32_t coun
             const T dmp = DAMP ? T(exp(-kim * rr)) : T(1);
             const T er = dmp * cs * ir, ei = dmp * sn * ir;
             const T q0 = ys[i][6], q1 = ys[i][7];
-            loc[0] += q0 * er - q1 * ei;
-            loc[1] += q0 * ei + q1 * er;
+            loc[a][0] += q0 * er - q1 * ei;
+            loc[a][1] += q0 * ei + q1 * er;
             if (GRAD) {
               const T ar = DAMP ? -kim * rr - T(1) : T(-1), ai = kre * rr, ir2 = ir * ir;
               const T gr = (ar * er - ai * ei) * ir2, gi = (ar * ei + ai * er) * ir2;
               const T qgr = q0 * gr - q1 * gi, qgi = q0 * gi + q1 * gr;
-              loc[2] += qgr * dx;
-              loc[3] += qgi * dx;
-              loc[4] += qgr * dy;
-              loc[5] += qgi * dy;
-              loc[6] += qgr * dz;
-              loc[7] += qgi * dz;
+              loc[a][2] += qgr * dx;
+              loc[a][3] += qgi * dx;
+              loc[a][4] += qgr * dy;
+              loc[a][5] += qgi * dy;
+              loc[a][6] += qgr * dz;
+              loc[a][7] += qgi * dz;
             }
           }
-      }
-#pragma unroll
-      for (int q = 0; q < 8; ++q) acc[q] += double(loc[q]);
+        }
     }
-    // phases in order
-    __syncthreads();
 #pragma unroll
-    for (int q = 0; q < 8; ++q) red[lane][q] = acc[q];
-    __syncthreads();
-    if (ph == 0 && active) {
+    for (int a = 0; a < A; ++a)
+#pragma unroll
+      for (int q = 0; q < 8; ++q) acc[a][q] += double(loc[a][q]);
+  }
+#pragma unroll
+  for (int a = 0; a < A; ++a) {
+    // the waves, then the phases, in order
+    add_waves(wave, lane, acc[a], sh.red);
+    if (wave > 0) continue;
+    wave_sync();
+#pragma unroll
+    for (int q = 0; q < 8; ++q) sh.red[0][q][lane] = acc[a][q];
+    wave_sync();
+    if (ph == 0 && ok[a]) {
       for (int h = 1; h < phases; ++h)
 #pragma unroll
-        for (int q = 0; q < 8; ++q) acc[q] += red[h * span + j][q];
-      phi_hat[2 * size_t(t)] += acc[0];
-      phi_hat[2 * size_t(t) + 1] += acc[1];
+        for (int q = 0; q < 8; ++q) acc[a][q] += sh.red[0][q][h * np + slot];
+      const size_t t = tb + uint32_t(slot + a * np);
+      phi_hat[2 * t] += acc[a][0];
+      phi_hat[2 * t + 1] += acc[a][1];
       if (GRAD)
 #pragma unroll
-        for (int q = 0; q < 6; ++q) grad_hat[6 * size_t(t) + q] += acc[2 + q];
+        for (int q = 0; q < 6; ++q) grad_hat[6 * t + q] += acc[a][2 + q];
     }
+  }
+}
+
+template <typename T, bool GRAD, bool DAMP>
+__global__ __launch_bounds__(64 * kP2pWaves) void k_h_p2p(
+    uint32_t leaf_first, uint32_t count, const uint32_t *__restrict__ near_off, const uint32_t *__restrict__ near_ent,
+    const uint32_t *__restrict__ leaf_cell, const uint32_t *__restrict__ src_start,
+    const uint32_t *__restrict__ tgt_start, const double *__restrict__ sx, const double *__restrict__ sy,
+    const double *__restrict__ sz, const double *__restrict__ qr, const double *__restrict__ qi,
+    const float4 *__restrict__ rec, const double *__restrict__ tx, const double *__restrict__ ty,
+    const double *__restrict__ tz, const double *__restrict__ hlev, double *__restrict__ phi_hat,
+    double *__restrict__ grad_hat) {
+  __shared__ HP2pStage<T> sh;
+  const uint32_t item = xcd_index(count);
+  if (item >= count) return;
+  const uint32_t lf = leaf_first + item;
+  const uint32_t t0 = tgt_start[lf], t1 = tgt_start[lf + 1];
+  if (t1 == t0) return;
+  const int lev = int(leaf_cell[4 * size_t(lf)]);
+  const T kre = T(hlev[4 * lev]), kim = T(hlev[4 * lev + 1]);
+  const uint32_t e0 = near_off[lf], e1 = near_off[lf + 1];
+  for (uint32_t tb = t0; tb < t1; tb += 128) {
+    const uint32_t n = (t1 - tb) < 128u ? (t1 - tb) : 128u;
+    if (sizeof(T) == 4 && t1 - t0 > 32) {
+      if (n > 64)
+        h_p2p_uniform<GRAD, DAMP, true>(sh.red, lf, tb, n, e0, e1, near_ent, leaf_cell, src_start, rec, hlev, tx, ty,
+                                        tz, phi_hat, grad_hat);
+      else
+        h_p2p_uniform<GRAD, DAMP, false>(sh.red, lf, tb, n, e0, e1, near_ent, leaf_cell, src_start, rec, hlev, tx, ty,
+                                         tz, phi_hat, grad_hat);
+      continue;
+    }
+    // one target per lane unless two fill more of the lanes' target slots
+    const int slots1 = n <= 64 ? int(n) * (64 / int(n)) : 0, slots2 = int(n) * (64 / ((int(n) + 1) / 2));
+    if (2 * slots1 >= slots2)
+      h_p2p_staged<T, GRAD, DAMP, 1>(sh, lf, tb, n, e0, e1, kre, kim, near_ent, leaf_cell, src_start, sx, sy, sz, qr,
+                                     qi, tx, ty, tz, phi_hat, grad_hat);
+    else
+      h_p2p_staged<T, GRAD, DAMP, 2>(sh, lf, tb, n, e0, e1, kre, kim, near_ent, leaf_cell, src_start, sx, sy, sz, qr,
+                                     qi, tx, ty, tz, phi_hat, grad_hat);
   }
 }
 
@@ -977,7 +1070,7 @@ void h_p2p(hipStream_t s, uint32_t leaf_first, uint32_t count, int gradients, in
   if (count == 0) return;
   const float4 *r4 = reinterpret_cast<const float4 *>(rec);
 #define FMMH_HP2P(G, D)                                                                                         \
-  hipLaunchKernelGGL((k_h_p2p<T, G, D>), dim3(xcd_grid(count)), dim3(64), 0, s, leaf_first, count, near_off,   \
+  hipLaunchKernelGGL((k_h_p2p<T, G, D>), dim3(xcd_grid(count)), dim3(64 * kP2pWaves), 0, s, leaf_first, count, near_off,   \
                      near_ent, leaf_cell, src_start, tgt_start, sx, sy, sz, qr, qi, r4, tx, ty, tz, hlev,       \
                      phi_hat, grad_hat)
   if (gradients) {

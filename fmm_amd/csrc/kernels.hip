@@ -1059,13 +1059,6 @@ static int m2p_waves(int p, int gradients) {
   return w < 8 ? int(w) : 8;
 }
 
-// Ordering of LDS between the lanes of one wave: its LDS operations complete in order, so
-// only the compiler must not move them.
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 template <bool GRAD>
 __global__ __launch_bounds__(512, 4) void k_m2p(int p, int wave_doubles, uint32_t rows, const uint32_t *row_leaf,
                                              const uint32_t *row_off, const uint32_t *row_box,

@@ -47,6 +47,13 @@ __device__ __forceinline__ uint32_t xcd_index(uint32_t n, uint32_t chunk) {
   return ((k / chunk) * kXcds + x) * chunk + k % chunk;
 }
 
+// Ordering of LDS between the lanes of one wave: its LDS operations complete in order, so
+// only the compiler must not move them.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 hipError_t upload_constants();
 
 void fill(hipStream_t s, double *p, size_t n, double v);

@@ -73,3 +73,24 @@ def test_m2l_reflection_level_calls():
     a, b = fmm.evaluate(q), fmm.evaluate_levels(q)
     assert O.error_norms(b.potential, a.potential)[0] < 1e-14
     assert O.error_norms(b.gradient, a.gradient, True)[0] < 1e-14
+
+
+@pytest.mark.parametrize("precision,tol", [("f64", 1e-12), ("mixed", 2e-6)])
+@pytest.mark.parametrize("k,leaf,gradients", [(9.0, 5, True), (2.0 + 0.5j, 40, True), (30.0, 70, False),
+                                              (14.0, 150, True)])
+def test_helmholtz_p2p_rows_over_waves(k, leaf, gradients, precision, tol):
+    """Leaves of one target to several chunks of 128 (one or two targets per lane), rows of one
+    near leaf to many, phases k r of many turns; real and complex wavenumbers."""
+    _log(f"case Helmholtz P2P k={k} leaf={leaf} {precision} gradients={gradients}")
+    rng = O.Rng(55)
+    pts = np.vstack([rng.cube(900), rng.plummer(700, (0.5, 0.5, 0.5), 0.02)])
+    q = rng.normals(len(pts)) + 1j * rng.normals(len(pts))
+    b = fmm_amd.HelmholtzFmmBuilder(k, degree=10).max_points_per_leaf(leaf).gradients(gradients).precision(precision)
+    fmm = b.build(pts)
+    out = fmm.evaluate(q)
+    phi, grad = O.Fmm(pts, p=10, leaf_points=leaf).evaluate_helmholtz(k, q)
+    errs = [np.linalg.norm(out.potential - phi) / np.linalg.norm(phi)]
+    if gradients:
+        errs.append(np.linalg.norm(out.gradient - grad) / np.linalg.norm(grad))
+    _log(f"  errors {errs}")
+    assert max(errs) < tol, errs
