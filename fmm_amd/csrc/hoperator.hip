@@ -466,7 +466,47 @@ HelmholtzOperator::HelmholtzOperator(const Plan &plan, const HelmholtzOptions &o
       upload_rows(rot_red_, red_id, {}, red_off, red_ent);
     }
   }
-  // M2L: per level the offsets present, ids base_l + 2 j + plane; tiles of 64 targets of
+  // dense levels whose M2L runs by reflection classes: the tables of the 56 classes' offsets
+  // alone, their real and imaginary parts as two sets, and each box's re and im expansions
+  // as two rows (Re L += Tr Re M + Ti (-Im M), Im L += Tr Im M + Ti Re M).  Trees of fewer
+  // than 100,000 pairs keep a table per offset: there the per-pair rotation, the form chosen to
+  // hold less memory, would hold more than the classes' tables (3,000 points, p = 10: 94 MB
+  // against 67).
+  std::vector<char> reflected(nlevels_, 0);
+  {
+    std::vector<uint64_t> pairs(nlevels_, 0), boxes(nlevels_, 0);
+    uint64_t total = 0;
+    for (int l = 2; l < nlevels_; ++l)
+      if (dense_level[l]) {
+        total += pairs[l] = plan.v[l].size();
+        boxes[l] = plan.nboxes(l);
+      }
+    if (total >= 100000 && ReflectM2l::fits(p, opt_.precision == kMixed, 3 * nbox_total_))
+      reflected = ReflectM2l::levels(p, pairs, boxes);
+  }
+  if (std::count(reflected.begin(), reflected.end(), char(1)) > 0) {
+    std::vector<size_t> level_vec;
+    for (uint32_t b : box_base_) level_vec.push_back(3 * size_t(b));
+    reflect_.begin(p, opt_.precision == kMixed, level_vec, 2);
+    const std::vector<uint16_t> cls = ReflectM2l::class_offsets();
+    for (int l = 2; l < nlevels_; ++l) {
+      if (!reflected[l]) continue;
+      const Csr &V = plan.v[l];
+      m2l_pairs_ += V.size();
+      std::vector<double> t;
+      h_m2l_tables(p, kh[l], cls, t);
+      const uint32_t tables = reflect_.add_tables([&](int set, int c) { return t.data() + (2 * size_t(c) + set) * n2; });
+      for (uint32_t b = 0; b < plan.nboxes(l); ++b)
+        for (uint32_t im = 0; im < 2 && V.off[b + 1] > V.off[b]; ++im)
+          reflect_.add_row(l, 3 * gid(l, b) + im, octant_of(plan.keys[l][b]), tables, V.aux.data() + V.off[b],
+                           V.off[b + 1] - V.off[b], [&](int set, uint32_t e) {
+                             const uint32_t s = 3 * gid(l, V.ent[V.off[b] + e]);
+                             return set == 0 ? s + im : im ? s : s + 2;
+                           });
+    }
+    reflect_.finish();
+  }
+  // M2L by contraction: per level the offsets present, ids base_l + 2 j + plane; tiles of 64 targets of
   // one octant class, classes interleaved, groups by (parent-level neighbour, octant)
   {
     std::vector<double> m2l_sw;
@@ -477,7 +517,7 @@ HelmholtzOperator::HelmholtzOperator(const Plan &plan, const HelmholtzOptions &o
     uint32_t id_base = 0;
     for (int l = 2; l < nlevels_; ++l) {
       const Csr &V = plan.v[l];
-      if (V.size() == 0 || !dense_level[l]) continue;
+      if (V.size() == 0 || !dense_level[l] || reflected[l]) continue;
       m2l_pairs_ += V.size();
       std::vector<uint16_t> used(V.aux.begin(), V.aux.end());
       std::sort(used.begin(), used.end());
@@ -610,7 +650,7 @@ HelmholtzOperator::HelmholtzOperator(const Plan &plan, const HelmholtzOptions &o
     if (opt_.precision == kMixed) {
       if (m2l16.empty()) m2l16.assign(sw16, 0);
       t_m2l16_.upload(m2l16);
-      mult16_.alloc(3 * nbox_total_ * dev::split_expansion_size(p));
+      if (m2l_.ntasks) mult16_.alloc(3 * nbox_total_ * dev::split_expansion_size(p));
     } else {
       if (m2l_sw.empty()) m2l_sw.assign(sw, 0.0);
       t_m2l_.upload(m2l_sw);
@@ -785,7 +825,7 @@ void HelmholtzOperator::wait_for(hipStream_t producer) {
 }
 
 size_t HelmholtzOperator::device_bytes() const {
-  return mult_.bytes() + loc_.bytes() + t_m2m_.bytes() + t_l2l_.bytes() + t_m2l_.bytes() + t_m2l16_.bytes() +
+  return mult_.bytes() + loc_.bytes() + t_m2m_.bytes() + t_l2l_.bytes() + t_m2l_.bytes() + reflect_.bytes() + t_m2l16_.bytes() +
          mult16_.bytes() + sx_.bytes() * 8 + slots_.bytes() + slots32_.bytes() + rot_fwd_.bytes() +
          rot_coax_.bytes() + rot_slots_.bytes() + pw_tab_.bytes() + pw_shift_.bytes() + pw_waves_.bytes() +
          pw_inc_.bytes();
@@ -909,6 +949,11 @@ void HelmholtzOperator::evaluate() {
       const uint32_t r0 = rot_chunk_row_[c], r1 = rot_chunk_row_[c + 1];
       dev::reduce_slots(stream_, p, r1 - r0, rot_red_.row_id.ptr + r0, rot_red_.row_off.ptr + r0,
                         rot_red_.row_ent.ptr, 0, rot_slots_.ptr, nullptr, loc_.ptr);
+    });
+  if (reflect_.pairs())
+    timed(3, [&] {
+      reflect_.launch(stream_, 2, L, mult_.ptr, loc_.ptr,
+                      [&](const std::function<void()> &f) { timed(kKindM2lContract, f); });
     });
   if (m2l_.ntasks)
     timed(3, [&] {

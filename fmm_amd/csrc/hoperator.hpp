@@ -94,6 +94,7 @@ class HelmholtzOperator {
 
   Rows p2m_rows_, l2p_rows_, m2p_rows_, p2l_rows_;
   std::vector<Schedule> m2m_, l2l_;  // per level (M2M into the parents of level l, L2L into level l)
+  ReflectM2l reflect_;  // dense levels by reflection classes
   Schedule m2l_;
   // sparse M2L levels: scratch rows (ids from 3 nbox_total_ on) of one (target plane,
   // parent-level neighbour) each, and the ordered reduction of a target plane's rows

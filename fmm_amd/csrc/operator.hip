@@ -233,9 +233,31 @@ DeviceOperator::DeviceOperator(const Plan &plan, const OperatorOptions &options)
     upload_rows(p2l_rows_, id, cell, off, ent);
   }
   // the levels whose M2L runs by reflection classes
-  const std::vector<char> reflected = reflected_levels(plan);
+  std::vector<char> reflected(nlevels_, 0);
+  if (opt_.m2l == kM2lDense && ReflectM2l::fits(opt_.p, opt_.precision == kMixed, nbox_total_)) {
+    std::vector<uint64_t> pairs(nlevels_, 0), boxes(nlevels_, 0);
+    for (int l = 2; l < nlevels_; ++l) {
+      if (l < kTuneLevels && opt_.tuning.m2l_mode[l] != 0) continue;
+      pairs[l] = plan.v[l].size();
+      boxes[l] = plan.nboxes(l);
+    }
+    reflected = ReflectM2l::levels(opt_.p, pairs, boxes);
+  }
   build_schedules(plan, reflected);
-  build_reflect(plan, reflected, m2l);
+  if (std::count(reflected.begin(), reflected.end(), char(1)) > 0) {
+    reflect_.begin(opt_.p, opt_.precision == kMixed, std::vector<size_t>(box_base_.begin(), box_base_.end()), 1);
+    const std::vector<uint16_t> cls = ReflectM2l::class_offsets();
+    const size_t n2 = size_t(nc_) * nc_;
+    const uint32_t t = reflect_.add_tables([&](int, int c) { return m2l.data() + n2 * cls[c]; });
+    for (int l = 0; l < nlevels_; ++l) {
+      const Csr &V = plan.v[l];
+      for (uint32_t b = 0; reflected[l] && b < plan.nboxes(l); ++b)
+        if (V.off[b + 1] > V.off[b])
+          reflect_.add_row(l, gid(l, b), octant_of(plan.keys[l][b]), t, V.aux.data() + V.off[b],
+                           V.off[b + 1] - V.off[b], [&](int, uint32_t e) { return gid(l, V.ent[V.off[b] + e]); });
+    }
+    reflect_.finish();
+  }
   if (m2l_.ntasks > 0 && opt_.m2l == kM2lDense) {
     const size_t n2 = size_t(nc_) * nc_, sw = dev::swizzled_table_size(opt_.p);
     if (opt_.precision == kMixed) {
@@ -256,7 +278,7 @@ DeviceOperator::DeviceOperator(const Plan &plan, const OperatorOptions &options)
     slots32_.alloc(nslots_ * nc_);
   else
     slots_.alloc(nslots_ * nc_);
-  if (opt_.precision == kMixed) mult16_.alloc(nbox_total_ * dev::split_expansion_size(opt_.p));
+  if (opt_.precision == kMixed && m2l_.ntasks) mult16_.alloc(nbox_total_ * dev::split_expansion_size(opt_.p));
   if (opt_.precision == kMixed && near_ent_.count > 0) {
     // the near entries whose pairs the fixed-point P2P must test (one pass at build)
     near_close_.alloc(near_ent_.count);
@@ -518,185 +540,6 @@ void DeviceOperator::build_schedules(const Plan &plan, const std::vector<char> &
   upload_rows(m2l_red_, red_id, red_cell, red_off, red_ent);
 }
 
-// The levels whose dense M2L runs by reflection classes (reflect.hpp).
-//
-// Per target a level costs 56 classes of lay.tiles row tiles this way and one product of the
-// (p+1)^2 / 16 row tiles per pair by contraction.  At p = 12 (15 tiles against 11) the two
-// break even near 50 pairs per box: 4M points' level 6 with 49 takes 2.9 ms against 2.0 in
-// bf16x3 and 5.5 against 5.0 in f64, level 5 with 165 takes 1.4 against 2.7 and 3.0 against
-// 8.2.  The levels of up to 512 boxes are short of workgroups by contraction and cost launches
-// of their own (100,000 points, p = 6: 24 us), so they join the deeper ones' launch, or where
-// there are none take the classes from under half of that density on, all of them or none.
-std::vector<char> DeviceOperator::reflected_levels(const Plan &plan) const {
-  std::vector<char> out(nlevels_, 0);
-  const ReflectLayout lay(opt_.p, opt_.precision == kMixed ? dev::kReflectChunk16 : dev::kReflectChunk);
-  // the sources are 32-bit byte offsets
-  if (opt_.m2l != kM2lDense || (nbox_total_ + 1) * size_t(lay.kp) * sizeof(double) > 0xFFFFFFFFu) return out;
-  const double per_pair = double((nc_ + 15) / 16), per_box = double(lay.tiles);
-  bool large = false, any = false;
-  double small_pairs = 0.0, small_boxes = 0.0;
-  std::vector<int> small;
-  for (int l = 2; l < nlevels_; ++l) {
-    const double pairs = double(plan.v[l].size()), boxes = double(plan.nboxes(l));
-    if (pairs == 0.0 || (l < kTuneLevels && opt_.tuning.m2l_mode[l] != 0)) continue;
-    if (boxes <= 512.0) {
-      small.push_back(l);
-      small_pairs += pairs;
-      small_boxes += boxes;
-      continue;
-    }
-    large = true;
-    out[l] = pairs * per_pair >= 37.0 * boxes * per_box;
-    any = any || out[l];
-  }
-  if (any || (!large && small_pairs * per_pair >= 16.0 * small_boxes * per_box))
-    for (int l : small) out[l] = 1;
-  return out;
-}
-
-void DeviceOperator::build_reflect(const Plan &plan, const std::vector<char> &levels,
-                                   const std::vector<double> &m2l) {
-  rf_level_task_.assign(nlevels_ + 1, 0);
-  rf_red_level_.assign(nlevels_ + 1, 0);
-  if (std::count(levels.begin(), levels.end(), char(1)) == 0) return;
-  const ReflectClasses &rc = reflect_classes();
-  const bool mixed = opt_.precision == kMixed;
-  const int chunk = mixed ? dev::kReflectChunk16 : dev::kReflectChunk;
-  const ReflectLayout lay(opt_.p, chunk);
-  // target rows and the source of every reflection position, as the byte offset of its
-  // sorted multipole; a row of zeros after the last box stands for none
-  const size_t row_bytes = size_t(lay.kp) * sizeof(double);
-  int flips[8], where[8][316];
-  for (int o = 0; o < 8; ++o) {
-    // a target at the lower end of its parent has the offsets -3 .. 2 there: reflected
-    flips[o] = 7 & ~o;
-    for (int d = 0; d < 316; ++d) {
-      int dv[3];
-      offset_of_index(d, dv);
-      where[o][d] = -1;
-      bool seen = true;
-      for (int a = 0; a < 3; ++a) seen = seen && dv[a] != (((o >> (2 - a)) & 1) ? -3 : 3);
-      if (seen) where[o][d] = rc.position(dv, flips[o]);
-    }
-  }
-  std::vector<uint32_t> row_box, src;
-  std::vector<uint8_t> row_flip;
-  std::vector<uint32_t> level_row(nlevels_ + 1, 0);
-  for (int l = 0; l < nlevels_; ++l) {
-    const Csr &V = plan.v[l];
-    for (uint32_t b = 0; levels[l] && b < plan.nboxes(l); ++b) {
-      if (V.off[b + 1] == V.off[b]) continue;
-      row_box.push_back(box_base_[l] + b);
-      const int o = octant_of(plan.keys[l][b]);
-      row_flip.push_back(uint8_t(flips[o]));
-      src.resize(kReflectPositions * row_box.size(), uint32_t(nbox_total_ * row_bytes));
-      uint32_t *row = src.data() + kReflectPositions * (row_box.size() - 1);
-      for (uint32_t e = V.off[b]; e < V.off[b + 1]; ++e) {
-        const int at = where[o][V.aux[e]];
-        require(at >= 0, "M2L schedule: V offset outside the parent's neighbours", kUnsupportedLayout);
-        row[at] = uint32_t((box_base_[l] + V.ent[e]) * row_bytes);
-      }
-      rf_pairs_ += V.off[b + 1] - V.off[b];
-    }
-    level_row[l + 1] = static_cast<uint32_t>(row_box.size());
-  }
-  // targets per task, and the tasks that run at once: 2 workgroups of 32 or 4 of 16 per CU
-  const uint32_t width = mixed ? 32 : 16, round = mixed ? 512 : 1024;
-  // A task walks its classes in sequence.  Tasks beyond a whole number of rounds of the
-  // workgroups that run at once would leave most of the GPU idle in the last
-  // round, so their classes are split into parts of about equal cost, as
-  // many parts as fill the round, each part's sums in scratch rows that are added in part
-  // order.
-  uint32_t base_tasks = 0;
-  for (int l = 0; l < nlevels_; ++l) base_tasks += (level_row[l + 1] - level_row[l] + width - 1) / width;
-  const uint32_t whole = base_tasks / round * round;
-  const uint32_t parts =
-      base_tasks == whole ? 1 : std::min<uint32_t>(28, std::max<uint32_t>(1, round / (base_tasks - whole)));
-  // a class costs its products (halved by every component 0) and its butterfly
-  std::vector<uint32_t> cost{0};
-  for (int c = 0; c < kReflectClasses; ++c)
-    cost.push_back(cost.back() + (2u << __builtin_popcount(unsigned(rc.axes[c]))) + uint32_t(rc.first[c + 1] - rc.first[c]));
-  std::vector<int> cut{0};
-  for (uint32_t q = 1; q < parts; ++q) {
-    int c = cut.back() + 1;
-    while (c < kReflectClasses && cost[c] * parts < q * cost.back()) ++c;
-    cut.push_back(c);
-  }
-  cut.push_back(kReflectClasses);
-  std::vector<dev::ReflectTask> tasks;
-  std::vector<uint32_t> red_id, red_off{0}, red_ent;
-  uint32_t nscratch = 0, tasks_seen = 0;
-  for (int l = 0; l < nlevels_; ++l) {
-    for (uint32_t r = level_row[l]; r < level_row[l + 1]; r += width) {
-      const uint32_t n = std::min<uint32_t>(width, level_row[l + 1] - r);
-      if (tasks_seen++ < whole || parts == 1) {
-        tasks.push_back(dev::ReflectTask{r, uint16_t(n), 0, kReflectClasses, kNone, 1});
-        continue;
-      }
-      for (uint32_t q = 0; q < parts; ++q)
-        tasks.push_back(
-            dev::ReflectTask{r, uint16_t(n), uint8_t(cut[q]), uint8_t(cut[q + 1]), nscratch + q, parts});
-      for (uint32_t k = 0; k < n; ++k) {
-        red_id.push_back(row_box[r + k]);
-        for (uint32_t q = 0; q < parts; ++q) red_ent.push_back(nscratch++);
-        red_off.push_back(static_cast<uint32_t>(red_ent.size()));
-      }
-    }
-    rf_level_task_[l + 1] = static_cast<uint32_t>(tasks.size());
-    rf_red_level_[l + 1] = static_cast<uint32_t>(red_id.size());
-  }
-  rf_slots_issued_ = uint64_t(width) * kReflectPositions * base_tasks;
-  upload_rows(rf_red_, red_id, {}, red_off, red_ent);
-  rf_scratch_.alloc(size_t(nscratch) * nc_);
-  rf_tasks_.upload(tasks);
-  rf_row_box_.upload(row_box);
-  rf_src_.upload(src);
-  std::vector<uint32_t> first;
-  for (int c = 0; c <= kReflectClasses; ++c)
-    first.push_back(uint32_t(rc.first[c]) | uint32_t(c < kReflectClasses ? rc.axes[c] : 0) << 16);
-  rf_first_.upload(first);
-  rf_row_flip_.upload(row_flip);
-  std::vector<uint64_t> kmask;
-  for (int axes = 0; axes < 8; ++axes)
-    for (int c = 0; c < 8; ++c) kmask.push_back(lay.steps(axes, c, mixed ? chunk : 4));
-  rf_kmask_.upload(kmask);
-  rf_parity_.upload(lay.parity);
-  rf_tile_class_.upload(lay.tile_class);
-  rf_perm_.upload(lay.perm);
-  rf_tile_row_.upload(lay.tile_row);
-  // (after the last chunk a wave reads, and drops, the next chunk's tiles)
-  const size_t n2 = size_t(nc_) * nc_;
-  auto class_table = [&](int c) {
-    return m2l.data() + n2 * offset_index(rc.offset[c][0], rc.offset[c][1], rc.offset[c][2]);
-  };
-  if (mixed) {
-    const size_t sz = dev::reflect_table_size_bf16(lay);
-    std::vector<uint16_t> tables(sz * kReflectClasses + size_t(lay.tiles + 4) * 1536, 0);
-    for (int c = 0; c < kReflectClasses; ++c) dev::reflect_table_bf16(lay, class_table(c), tables.data() + sz * c);
-    rf_tables16_.upload(tables);
-  } else {
-    const size_t sz = dev::reflect_table_size(lay);
-    std::vector<double> tables(sz * kReflectClasses + size_t(lay.tiles + 4) * 256, 0.0);
-    for (int c = 0; c < kReflectClasses; ++c) dev::reflect_table(lay, class_table(c), tables.data() + sz * c);
-    rf_tables_.upload(tables);
-  }
-  rf_sorted_.alloc((nbox_total_ + 1) * lay.kp);
-  hip_check(hipMemset(rf_sorted_.ptr + nbox_total_ * lay.kp, 0, row_bytes), "reflection zero row");
-  rf_.nc = nc_;
-  rf_.kp = lay.kp;
-  rf_.tiles = lay.tiles;
-  std::copy(rc.run.begin(), rc.run.end(), rf_.run);
-  rf_.first = rf_first_.ptr;
-  rf_.kmask = rf_kmask_.ptr;
-  rf_.parity = rf_parity_.ptr;
-  rf_.tile_row = rf_tile_row_.ptr;
-  rf_.tile_class = rf_tile_class_.ptr;
-  rf_.tasks = rf_tasks_.ptr;
-  rf_.row_box = rf_row_box_.ptr;
-  rf_.row_flip = rf_row_flip_.ptr;
-  rf_.src = rf_src_.ptr;
-}
-
 // Plane-wave M2L by merge and shift (fmm-kernels/src/plane_wave.rs:1-60,
 // fmm-tables/src/plane_wave/geometry.rs): the quadrature of degree p, the accumulators and
 // shifts (the same for every parent), and per level the parents of its boxes with their
@@ -891,7 +734,7 @@ void DeviceOperator::build_rotation(const Plan &plan) {
 size_t DeviceOperator::device_bytes() const {
   return mult_.bytes() + loc_.bytes() + slots_.bytes() + slots32_.bytes() + t_m2l_.bytes() + t_m2m_.bytes() +
          t_l2l_.bytes() + sx_.bytes() * 8 + src_rec_.bytes() + rot_slots_.bytes() + rot_slots32_.bytes() +
-         mult32_.bytes() + rf_tables_.bytes() + rf_tables16_.bytes() + rf_src_.bytes() + rf_sorted_.bytes() + rf_scratch_.bytes() + pw_waves_.bytes() + pw_inc_.bytes() + pw_src_shift_.bytes() + pw_child_shift_.bytes();
+         mult32_.bytes() + reflect_.bytes() + pw_waves_.bytes() + pw_inc_.bytes() + pw_src_shift_.bytes() + pw_child_shift_.bytes();
 }
 
 void DeviceOperator::launch_contract(const Schedule &s, uint32_t task_first, uint32_t ntasks, const double *X,
@@ -946,28 +789,8 @@ void DeviceOperator::launch_m2l(int level_first, int level_last) {
     }
     return;
   }
-  const uint32_t f0 = rf_level_task_[level_first], f1 = rf_level_task_[level_last + 1];
-  if (f1 > f0) {
-    // the multipoles of the levels that take it, sorted; their tasks; the parts' sums
-    int a = level_first, b = level_last;
-    while (rf_level_task_[a + 1] == f0) ++a;
-    while (rf_level_task_[b] == f1) --b;
-    const size_t x0 = box_base_[a], x1 = box_base_[b + 1];
-    dev::reflect_sort(stream_, nc_, rf_.kp, x1 - x0, rf_perm_.ptr, mult_.ptr + x0 * nc_,
-                      rf_sorted_.ptr + x0 * rf_.kp);
-    dev::ReflectArgs args = rf_;
-    args.tasks += f0;
-    timed(kKindM2lContract, [&] {
-      if (opt_.precision == kMixed)
-        dev::m2l_reflect_bf16(stream_, args, f1 - f0, rf_tables16_.ptr, rf_sorted_.ptr, loc_.ptr, rf_scratch_.ptr);
-      else
-        dev::m2l_reflect_f64(stream_, args, f1 - f0, rf_tables_.ptr, rf_sorted_.ptr, loc_.ptr, rf_scratch_.ptr);
-    });
-    const uint32_t w0 = rf_red_level_[level_first], w1 = rf_red_level_[level_last + 1];
-    if (w1 > w0)
-      dev::reduce_slots(stream_, opt_.p, w1 - w0, rf_red_.row_id.ptr + w0, rf_red_.row_off.ptr + w0,
-                        rf_red_.row_ent.ptr, 0, rf_scratch_.ptr, nullptr, loc_.ptr);
-  }
+  reflect_.launch(stream_, level_first, level_last, mult_.ptr, loc_.ptr,
+                  [&](const std::function<void()> &f) { timed(kKindM2lContract, f); });
   const uint32_t t0 = m2l_level_task_[level_first], t1 = m2l_level_task_[level_last + 1];
   if (t1 > t0) {
     if (opt_.precision == kMixed) {

@@ -15,6 +15,7 @@
 #include <string>
 #include <vector>
 
+#include "devbuf.hpp"
 #include "plan.hpp"
 #include "pwkernels.hpp"
 #include "reflect.hpp"
@@ -31,47 +32,6 @@ enum Precision : int {
   kMixed = 1,     // P2P in f32 (double-float separations), M2L in bf16x3 on MFMA
 };
 
-void hip_check(hipError_t e, const char *what);
-
-template <typename T>
-struct DevBuf {
-  T *ptr = nullptr;
-  size_t count = 0;
-  DevBuf() = default;
-  DevBuf(const DevBuf &) = delete;
-  DevBuf &operator=(const DevBuf &) = delete;
-  DevBuf(DevBuf &&o) noexcept : ptr(o.ptr), count(o.count) {
-    o.ptr = nullptr;
-    o.count = 0;
-  }
-  DevBuf &operator=(DevBuf &&o) noexcept {
-    if (this != &o) {
-      release();
-      ptr = o.ptr;
-      count = o.count;
-      o.ptr = nullptr;
-      o.count = 0;
-    }
-    return *this;
-  }
-  ~DevBuf() { release(); }
-  void release() {
-    if (ptr) (void)hipFree(ptr);
-    ptr = nullptr;
-    count = 0;
-  }
-  void alloc(size_t n) {
-    release();
-    count = n;
-    if (n) hip_check(hipMalloc(&ptr, n * sizeof(T)), "hipMalloc");
-  }
-  void upload(const std::vector<T> &v) {
-    alloc(v.size());
-    if (!v.empty()) hip_check(hipMemcpy(ptr, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice), "upload");
-  }
-  size_t bytes() const { return count * sizeof(T); }
-};
-
 // One contraction launch: tasks of COLS output columns, groups of (table, sources).
 struct Schedule {
   int width = 128;  // columns per task
@@ -80,12 +40,6 @@ struct Schedule {
   uint64_t slots = 0;  // columns x groups issued
   DevBuf<uint32_t> task_group_off, group_src, col_out;
   DevBuf<uint16_t> group_table;
-};
-
-// A row list for the leaf kernels: rows with an output (box or leaf) and CSR entries.
-struct Rows {
-  uint32_t rows = 0;
-  DevBuf<uint32_t> row_id, row_cell, row_off, row_ent;
 };
 
 enum M2lMethod : int {
@@ -166,7 +120,7 @@ class DeviceOperator {
   // the M2L mode each level's schedule took: 0 none or by reflection classes, 1 box mode,
   // 2 clustered mode
   int m2l_mode_of(int level) const { return level >= 0 && level < kTuneLevels ? m2l_mode_taken_[level] : 0; }
-  bool m2l_reflected(int level) const { return level + 1 < int(rf_level_task_.size()) && rf_level_task_[level + 1] > rf_level_task_[level]; }
+  bool m2l_reflected(int level) const { return reflect_.has(level); }
   int l2l_width_of(int level) const { return level >= 0 && level < int(l2l_.size()) ? l2l_[level].width : 0; }
 
   int nlevels() const { return nlevels_; }
@@ -176,8 +130,8 @@ class DeviceOperator {
   const OperatorOptions &options() const { return opt_; }
   // statistics for reports and the roofline
   uint64_t p2p_pairs() const { return p2p_pairs_; }
-  uint64_t m2l_pairs() const { return m2l_.pairs + rf_pairs_; }
-  uint64_t m2l_slots() const { return m2l_.slots + rf_slots_issued_; }
+  uint64_t m2l_pairs() const { return m2l_.pairs + reflect_.pairs(); }
+  uint64_t m2l_slots() const { return m2l_.slots + reflect_.slots(); }
   size_t device_bytes() const;
   double *device_locals() const { return loc_.ptr; }
   double *device_multipoles() const { return mult_.ptr; }
@@ -185,8 +139,6 @@ class DeviceOperator {
 
  private:
   void build_schedules(const Plan &plan, const std::vector<char> &reflected);
-  std::vector<char> reflected_levels(const Plan &plan) const;
-  void build_reflect(const Plan &plan, const std::vector<char> &levels, const std::vector<double> &m2l);
   template <class F>
   void timed(int kind, F &&f);
   void collect_timings();
@@ -279,19 +231,7 @@ class DeviceOperator {
   Rows m2l_red_;                                             // clustered-mode reductions
   std::vector<uint32_t> m2l_red_level_;
 
-  // M2L by reflection classes (reflect.hpp): the levels that take it, their target rows
-  // and tasks (by level), the class tables and the multipoles sorted by parity
-  dev::ReflectArgs rf_{};
-  DevBuf<uint32_t> rf_first_, rf_row_box_, rf_src_;
-  DevBuf<uint16_t> rf_tables16_;
-  DevBuf<uint64_t> rf_kmask_;
-  DevBuf<uint8_t> rf_parity_, rf_tile_class_, rf_row_flip_;
-  DevBuf<int32_t> rf_perm_, rf_tile_row_;
-  DevBuf<dev::ReflectTask> rf_tasks_;
-  DevBuf<double> rf_tables_, rf_sorted_, rf_scratch_;
-  std::vector<uint32_t> rf_level_task_, rf_red_level_;
-  Rows rf_red_;
-  uint64_t rf_pairs_ = 0, rf_slots_issued_ = 0;
+  ReflectM2l reflect_;  // the levels whose dense M2L runs by reflection classes
 };
 
 // Compensated f64 direct sum on the device (unscaled sums q / r and their gradient):

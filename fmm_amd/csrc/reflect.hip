@@ -147,6 +147,14 @@ __device__ __forceinline__ uint32_t flip_of(uint32_t sign, uint32_t flip) {
   return x ^ (x << 1) ^ (x << 2);
 }
 
+// Units of 64 lanes in one set of the class tables (16 bytes per lane).
+__device__ __forceinline__ size_t table_set(const ReflectArgs &a) {
+  return size_t(kReflectClasses) * (a.kp / kReflectChunk) * a.tiles * 2;
+}
+__device__ __forceinline__ size_t table_set16(const ReflectArgs &a) {
+  return size_t(kReflectClasses) * (a.kp / kReflectChunk16) * a.tiles * 3;
+}
+
 // Small read-only tables through the scalar cache.
 template <typename T>
 __device__ __forceinline__ T scalar_read(const T *p) {
@@ -294,7 +302,7 @@ __global__ __launch_bounds__(256, 4) void k_m2l_reflect_f64(ReflectArgs a, uint3
   for (int k = tid; k < a.kp; k += 256) sh.sign[k] = uint32_t(a.parity[k]) << 29;
   // the sources of this thread's target (a row past the task's last takes the last row's)
   const uint32_t mine = task.row0 + min(uint32_t(tid) >> 4, uint32_t(task.nrows) - 1u);
-  const uint32_t *ids = a.src + size_t(mine) * kReflectPositions;
+  const uint32_t *ids = a.src + (size_t(mine) * a.sets + task.set) * kReflectPositions;
   const uint32_t flip = uint32_t(a.row_flip[mine]) << 29;
   d4 acc[TPW];
   int tcls[TPW];
@@ -306,7 +314,7 @@ __global__ __launch_bounds__(256, 4) void k_m2l_reflect_f64(ReflectArgs a, uint3
   }
   const int nt = __builtin_amdgcn_readfirstlane(wave < a.tiles ? (a.tiles - wave + 3) / 4 : 0);
   __syncthreads();
-  const d2 *t2 = reinterpret_cast<const d2 *>(tables);
+  const d2 *t2 = reinterpret_cast<const d2 *>(tables) + size_t(task.table) * table_set(a) * 64;
   const char *x = reinterpret_cast<const char *>(Xs);
   int buf = 0;
 #define FMMH_RUN(P)                                                                         \
@@ -327,7 +335,7 @@ __global__ __launch_bounds__(256, 4) void k_m2l_reflect_f64(ReflectArgs a, uint3
   const uint32_t r = lane & 15;
   if (r >= task.nrows) return;
   const bool slot = task.slot != kNone;
-  double *y = slot ? S + size_t(task.slot + r * task.stride) * a.nc : Y + size_t(a.row_box[task.row0 + r]) * a.nc;
+  double *y = slot ? S + size_t(task.slot + r * task.stride) * a.nc : Y + size_t(a.row_out[task.row0 + r]) * a.nc;
   const uint32_t out_flip = uint32_t(a.row_flip[task.row0 + r]) << 29;
 #pragma unroll
   for (int i = 0; i < TPW; ++i) {
@@ -536,7 +544,7 @@ __global__ __launch_bounds__(512, TPW <= 2 ? 4 : 2) void k_m2l_reflect_bf16(Refl
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   for (int k = tid; k < a.kp; k += 512) sh.sign[k] = uint32_t(a.parity[k]) << 29;
   const uint32_t mine = task.row0 + min(uint32_t(tid) >> 4, uint32_t(task.nrows) - 1u);
-  const uint32_t *ids = a.src + size_t(mine) * kReflectPositions;
+  const uint32_t *ids = a.src + (size_t(mine) * a.sets + task.set) * kReflectPositions;
   const uint32_t flip = uint32_t(a.row_flip[mine]) << 29;
   const int t0 = __builtin_amdgcn_readfirstlane(wave * TPW);
   const int nt = __builtin_amdgcn_readfirstlane(max(0, min(TPW, a.tiles - t0)));
@@ -552,11 +560,12 @@ __global__ __launch_bounds__(512, TPW <= 2 ? 4 : 2) void k_m2l_reflect_bf16(Refl
   }
   __syncthreads();
   const char *x = reinterpret_cast<const char *>(Xs);
-#define FMMH_RUN(P)                                                                                              \
-  {                                                                                                              \
-    const int c0 = max(int(task.first), a.run[P]), c1 = min(int(task.last), a.run[P + 1]);                       \
-    if (c0 < c1)                                                                                                 \
-      reflect_run16<P, TPW>(sh, a, ids, flip, c0, c1, tables, x, min(t0, a.tiles - 1), nt, tcls, sum);            \
+  const u4 *t4 = tables + size_t(task.table) * table_set16(a) * 64;
+#define FMMH_RUN(P)                                                                                   \
+  {                                                                                                   \
+    const int c0 = max(int(task.first), a.run[P]), c1 = min(int(task.last), a.run[P + 1]);            \
+    if (c0 < c1)                                                                                      \
+      reflect_run16<P, TPW>(sh, a, ids, flip, c0, c1, t4, x, min(t0, a.tiles - 1), nt, tcls, sum);     \
   }
   FMMH_RUN(0)
   FMMH_RUN(1)
@@ -573,7 +582,7 @@ __global__ __launch_bounds__(512, TPW <= 2 ? 4 : 2) void k_m2l_reflect_bf16(Refl
     const uint32_t r = (lane & 15) + 16 * n;
     if (r >= task.nrows) continue;
     const bool slot = task.slot != kNone;
-    double *y = slot ? S + size_t(task.slot + r * task.stride) * a.nc : Y + size_t(a.row_box[task.row0 + r]) * a.nc;
+    double *y = slot ? S + size_t(task.slot + r * task.stride) * a.nc : Y + size_t(a.row_out[task.row0 + r]) * a.nc;
     const uint32_t out_flip = uint32_t(a.row_flip[task.row0 + r]) << 29;
 #pragma unroll
     for (int i = 0; i < TPW; ++i) {
@@ -607,4 +616,245 @@ void m2l_reflect_bf16(hipStream_t s, const ReflectArgs &a, uint32_t ntasks, cons
 }
 
 }  // namespace dev
+// ---- the operator's side ---------------------------------------------------------------------
+
+// Per target a level costs 56 classes of `tiles` row tiles this way and one product of the
+// (p+1)^2 / 16 row tiles per pair by contraction.  At p = 12 (15 tiles against 11) the two
+// break even near 50 pairs per box: 4M points' level 6 with 49 takes 2.9 ms against 2.0 in
+// bf16x3 and 5.5 against 5.0 in f64, level 5 with 165 takes 1.4 against 2.7 and 3.0 against
+// 8.2.  The levels of up to 512 boxes are short of workgroups by contraction and cost launches
+// of their own (100,000 points, p = 6: 24 us), so they join the deeper ones' launch, or where
+// there are none take the classes from under half of that density on, all of them or none.
+std::vector<char> ReflectM2l::levels(int p, const std::vector<uint64_t> &pairs, const std::vector<uint64_t> &boxes) {
+  std::vector<char> out(pairs.size(), 0);
+  const double per_pair = double(((p + 1) * (p + 1) + 15) / 16), per_box = double(ReflectLayout(p, 16).tiles);
+  bool large = false, any = false;
+  double small_pairs = 0.0, small_boxes = 0.0;
+  std::vector<size_t> small;
+  for (size_t l = 0; l < pairs.size(); ++l) {
+    if (pairs[l] == 0) continue;
+    if (boxes[l] <= 512) {
+      small.push_back(l);
+      small_pairs += double(pairs[l]);
+      small_boxes += double(boxes[l]);
+      continue;
+    }
+    large = true;
+    out[l] = double(pairs[l]) * per_pair >= 37.0 * double(boxes[l]) * per_box;
+    any = any || out[l];
+  }
+  if (any || (!large && small_pairs * per_pair >= 16.0 * small_boxes * per_box))
+    for (size_t l : small) out[l] = 1;
+  return out;
+}
+
+bool ReflectM2l::fits(int p, bool mixed, size_t nvec) {
+  const ReflectLayout lay(p, mixed ? dev::kReflectChunk16 : dev::kReflectChunk);
+  return (nvec + 1) * size_t(lay.kp) * sizeof(double) <= 0xFFFFFFFFu;
+}
+
+std::vector<uint16_t> ReflectM2l::class_offsets() {
+  std::vector<uint16_t> out;
+  for (const auto &d : reflect_classes().offset) out.push_back(uint16_t(offset_index(d[0], d[1], d[2])));
+  return out;
+}
+
+void ReflectM2l::begin(int p, bool mixed, const std::vector<size_t> &level_vec, int sets) {
+  p_ = p;
+  mixed_ = mixed;
+  level_vec_ = level_vec;
+  nvec_ = level_vec.back();
+  nlevels_ = int(level_vec.size()) - 1;
+  sets_ = sets;
+  lay_ = ReflectLayout(p, mixed ? dev::kReflectChunk16 : dev::kReflectChunk);
+  level_row_.assign(nlevels_ + 1, 0);
+}
+
+uint32_t ReflectM2l::add_tables(const std::function<const double *(int, int)> &table) {
+  const size_t sz = mixed_ ? dev::reflect_table_size_bf16(lay_) : dev::reflect_table_size(lay_);
+  size_t at = sz * kReflectClasses * ntables_;
+  if (mixed_)
+    tables16_h_.resize(at + sz * kReflectClasses * sets_);
+  else
+    tables_h_.resize(at + sz * kReflectClasses * sets_);
+  for (int s = 0; s < sets_; ++s)
+    for (int c = 0; c < kReflectClasses; ++c, at += sz) {
+      if (mixed_)
+        dev::reflect_table_bf16(lay_, table(s, c), tables16_h_.data() + at);
+      else
+        dev::reflect_table(lay_, table(s, c), tables_h_.data() + at);
+    }
+  const uint32_t id = ntables_;
+  ntables_ += uint32_t(sets_);
+  return id;
+}
+
+void ReflectM2l::add_row(int level, uint32_t out, int octant, uint32_t tables, const uint16_t *aux, uint32_t n,
+                         const std::function<uint32_t(int, uint32_t)> &source) {
+  // a target at the lower end of its parent has the offsets -3 .. 2 there: reflected
+  static const std::vector<int> where = [] {
+    std::vector<int> w(8 * 316, -1);
+    for (int o = 0; o < 8; ++o)
+      for (int d = 0; d < 316; ++d) {
+        int dv[3];
+        offset_of_index(d, dv);
+        bool seen = true;
+        for (int a = 0; a < 3; ++a) seen = seen && dv[a] != (((o >> (2 - a)) & 1) ? -3 : 3);
+        if (seen) w[316 * o + d] = reflect_classes().position(dv, 7 & ~o);
+      }
+    return w;
+  }();
+  // a row of zeros after the last expansion stands for a source that is not there
+  const size_t row_bytes = size_t(lay_.kp) * sizeof(double);
+  row_out_h_.push_back(out);
+  row_flip_h_.push_back(uint8_t(7 & ~octant));
+  row_table_h_.push_back(tables);
+  const size_t at = src_h_.size();
+  src_h_.resize(at + size_t(sets_) * kReflectPositions, uint32_t(nvec_ * row_bytes));
+  for (int s = 0; s < sets_; ++s)
+    for (uint32_t e = 0; e < n; ++e) {
+      const int pos = where[316 * octant + aux[e]];
+      require(pos >= 0, "M2L schedule: V offset outside the parent's neighbours", kUnsupportedLayout);
+      src_h_[at + size_t(s) * kReflectPositions + pos] = uint32_t(source(s, e) * row_bytes);
+    }
+  pairs_ += uint64_t(sets_) * n;
+  for (int l = level + 1; l <= nlevels_; ++l) level_row_[l] = static_cast<uint32_t>(row_out_h_.size());
+}
+
+void ReflectM2l::finish() {
+  const ReflectClasses &rc = reflect_classes();
+  // targets per task, and the tasks that run at once: 2 workgroups of 32 or 4 of 16 per CU
+  const uint32_t width = mixed_ ? 32 : 16, round = mixed_ ? 512 : 1024;
+  // A task walks its classes in sequence.  Tasks beyond a whole number of rounds of the
+  // workgroups that run at once would leave most of the GPU idle in the last round, so their
+  // classes are split into parts of about equal cost, as many parts as fill the round.  The
+  // parts of a row, and its sets, leave their sums in scratch rows that are added in order.
+  uint32_t base_tasks = 0;
+  for (int l = 0; l < nlevels_; ++l) base_tasks += (level_row_[l + 1] - level_row_[l] + width - 1) / width * uint32_t(sets_);
+  const uint32_t whole = base_tasks / round * round;
+  const uint32_t parts =
+      base_tasks == whole ? 1 : std::min<uint32_t>(28, std::max<uint32_t>(1, round / (base_tasks - whole)));
+  // a class costs its products (halved by every component 0) and its butterfly
+  std::vector<uint32_t> cost{0};
+  for (int c = 0; c < kReflectClasses; ++c)
+    cost.push_back(cost.back() + (2u << __builtin_popcount(unsigned(rc.axes[c]))) +
+                   uint32_t(rc.first[c + 1] - rc.first[c]));
+  std::vector<int> cut{0};
+  for (uint32_t q = 1; q < parts; ++q) {
+    int c = cut.back() + 1;
+    while (c < kReflectClasses && cost[c] * parts < q * cost.back()) ++c;
+    cut.push_back(c);
+  }
+  cut.push_back(kReflectClasses);
+  std::vector<dev::ReflectTask> tasks;
+  std::vector<uint32_t> red_id, red_off{0}, red_ent;
+  uint32_t nscratch = 0, seen = 0;
+  level_task_.assign(nlevels_ + 1, 0);
+  red_level_.assign(nlevels_ + 1, 0);
+  for (int l = 0; l < nlevels_; ++l) {
+    for (uint32_t r = level_row_[l]; r < level_row_[l + 1]; r += width) {
+      const uint32_t n = std::min<uint32_t>(width, level_row_[l + 1] - r), t = row_table_h_[r];
+      const uint32_t np = seen < whole ? 1 : parts, stride = np * uint32_t(sets_);
+      seen += uint32_t(sets_);
+      if (stride == 1) {
+        tasks.push_back(dev::ReflectTask{r, uint16_t(n), 0, kReflectClasses, kNone, 1, t, 0});
+        continue;
+      }
+      for (uint32_t q = 0; q < stride; ++q) {
+        const uint32_t set = q / np, part = q % np;
+        const int c0 = np == 1 ? 0 : cut[part], c1 = np == 1 ? kReflectClasses : cut[part + 1];
+        tasks.push_back(
+            dev::ReflectTask{r, uint16_t(n), uint8_t(c0), uint8_t(c1), nscratch + q, stride, t + set, set});
+      }
+      for (uint32_t k = 0; k < n; ++k) {
+        red_id.push_back(row_out_h_[r + k]);
+        for (uint32_t q = 0; q < stride; ++q) red_ent.push_back(nscratch++);
+        red_off.push_back(static_cast<uint32_t>(red_ent.size()));
+      }
+    }
+    level_task_[l + 1] = static_cast<uint32_t>(tasks.size());
+    red_level_[l + 1] = static_cast<uint32_t>(red_id.size());
+  }
+  slots_ = uint64_t(width) * kReflectPositions * base_tasks;
+  red_.rows = static_cast<uint32_t>(red_id.size());
+  red_.row_id.upload(red_id);
+  red_.row_off.upload(red_off);
+  red_.row_ent.upload(red_ent);
+  scratch_.alloc(size_t(nscratch) * lay_.nc);
+  tasks_.upload(tasks);
+  row_out_.upload(row_out_h_);
+  row_flip_.upload(row_flip_h_);
+  src_.upload(src_h_);
+  std::vector<uint32_t> first;
+  for (int c = 0; c <= kReflectClasses; ++c)
+    first.push_back(uint32_t(rc.first[c]) | uint32_t(c < kReflectClasses ? rc.axes[c] : 0) << 16);
+  first_.upload(first);
+  std::vector<uint64_t> kmask;
+  for (int axes = 0; axes < 8; ++axes)
+    for (int c = 0; c < 8; ++c) kmask.push_back(lay_.steps(axes, c, mixed_ ? dev::kReflectChunk16 : 4));
+  kmask_.upload(kmask);
+  parity_.upload(lay_.parity);
+  tile_class_.upload(lay_.tile_class);
+  perm_.upload(lay_.perm);
+  tile_row_.upload(lay_.tile_row);
+  // (after the last chunk a wave reads, and drops, the next chunk's tiles)
+  if (mixed_) {
+    tables16_h_.resize(tables16_h_.size() + size_t(lay_.tiles + 4) * 1536);
+    tables16_.upload(tables16_h_);
+  } else {
+    tables_h_.resize(tables_h_.size() + size_t(lay_.tiles + 4) * 256);
+    tables_.upload(tables_h_);
+  }
+  sorted_.alloc((nvec_ + 1) * lay_.kp);
+  hip_check(hipMemset(sorted_.ptr + nvec_ * lay_.kp, 0, size_t(lay_.kp) * sizeof(double)), "reflection zero row");
+  args_.nc = lay_.nc;
+  args_.kp = lay_.kp;
+  args_.tiles = lay_.tiles;
+  std::copy(rc.run.begin(), rc.run.end(), args_.run);
+  args_.first = first_.ptr;
+  args_.kmask = kmask_.ptr;
+  args_.parity = parity_.ptr;
+  args_.tile_row = tile_row_.ptr;
+  args_.tile_class = tile_class_.ptr;
+  args_.tasks = tasks_.ptr;
+  args_.sets = sets_;
+  args_.row_out = row_out_.ptr;
+  args_.row_flip = row_flip_.ptr;
+  args_.src = src_.ptr;
+  std::vector<uint32_t>().swap(row_out_h_);
+  std::vector<uint32_t>().swap(src_h_);
+  std::vector<uint32_t>().swap(row_table_h_);
+  std::vector<uint8_t>().swap(row_flip_h_);
+  std::vector<double>().swap(tables_h_);
+  std::vector<uint16_t>().swap(tables16_h_);
+}
+
+size_t ReflectM2l::bytes() const {
+  return tables_.bytes() + tables16_.bytes() + sorted_.bytes() + scratch_.bytes() + src_.bytes();
+}
+
+void ReflectM2l::launch(hipStream_t s, int first, int last, const double *X, double *Y,
+                        const std::function<void(const std::function<void()> &)> &contract) {
+  if (level_task_.empty()) return;
+  const uint32_t t0 = level_task_[first], t1 = level_task_[last + 1];
+  if (t1 == t0) return;
+  // the sources are of the targets' levels
+  while (!has(first)) ++first;
+  while (!has(last)) --last;
+  const size_t vec0 = level_vec_[first], vec1 = level_vec_[last + 1];
+  dev::reflect_sort(s, lay_.nc, lay_.kp, vec1 - vec0, perm_.ptr, X + vec0 * lay_.nc, sorted_.ptr + vec0 * lay_.kp);
+  dev::ReflectArgs args = args_;
+  args.tasks += t0;
+  contract([&] {
+    if (mixed_)
+      dev::m2l_reflect_bf16(s, args, t1 - t0, tables16_.ptr, sorted_.ptr, Y, scratch_.ptr);
+    else
+      dev::m2l_reflect_f64(s, args, t1 - t0, tables_.ptr, sorted_.ptr, Y, scratch_.ptr);
+  });
+  const uint32_t r0 = red_level_[first], r1 = red_level_[last + 1];
+  if (r1 > r0)
+    dev::reduce_slots(s, p_, r1 - r0, red_.row_id.ptr + r0, red_.row_off.ptr + r0, red_.row_ent.ptr, 0, scratch_.ptr,
+                      nullptr, Y);
+}
+
 }  // namespace fmmh

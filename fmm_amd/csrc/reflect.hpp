@@ -18,7 +18,10 @@
 
 #include <array>
 #include <cstdint>
+#include <functional>
 #include <vector>
+
+#include "devbuf.hpp"
 
 namespace fmmh {
 
@@ -61,6 +64,7 @@ struct ReflectTask {
   uint16_t nrows;
   uint8_t first, last;
   uint32_t slot, stride;
+  uint32_t table, set;  // its class tables, and the set of sources that they take
 };
 
 struct ReflectArgs {
@@ -72,9 +76,10 @@ struct ReflectArgs {
   const int32_t *tile_row;       // tiles x 16
   const uint8_t *tile_class;     // tiles
   const ReflectTask *tasks;
-  const uint32_t *row_box;       // target boxes
+  int sets;                      // sets of sources per row
+  const uint32_t *row_out;       // target expansions
   const uint8_t *row_flip;       // their reflected axes
-  const uint32_t *src;           // rows x 189: byte offset in Xs of the source at every position
+  const uint32_t *src;           // rows x sets x 189: byte offset in Xs of the source at every position
 };
 
 constexpr int kReflectChunk = 16;  // sorted positions per step of the f64 kernel
@@ -98,4 +103,61 @@ void m2l_reflect_bf16(hipStream_t s, const ReflectArgs &a, uint32_t ntasks, cons
                       double *Y, double *S);
 
 }  // namespace dev
+// The levels of an operator whose dense M2L runs by reflection classes.  A row is one real
+// target expansion: it adds, for each of `sets` sets of class tables, the products with the
+// sources that its V list names for that set (the Laplace operator has one set; a complex
+// table is two sets, its real and its imaginary part).
+class ReflectM2l {
+ public:
+  // Which levels take it: V pairs and boxes per level (0 pairs: not asked).
+  static std::vector<char> levels(int p, const std::vector<uint64_t> &pairs, const std::vector<uint64_t> &boxes);
+  // Whether nvec source expansions fit the kernels' 32-bit byte offsets.
+  static bool fits(int p, bool mixed, size_t nvec);
+  // (|dx|, |dy|, |dz|) of the classes as offset indices, in the order of add_tables
+  static std::vector<uint16_t> class_offsets();
+
+  // level_vec: first expansion of every level, and one past the last level's
+  void begin(int p, bool mixed, const std::vector<size_t> &level_vec, int sets);
+  // `sets` sets of tables (column-major (p+1)^2 x (p+1)^2, set s of class c at table(s, c));
+  // returns their index for add_row
+  uint32_t add_tables(const std::function<const double *(int, int)> &table);
+  // rows of one level after another, in ascending levels; source(set, e): expansion of V
+  // entry e (offset indices aux[0 .. n - 1]) of a target of the given octant
+  void add_row(int level, uint32_t out, int octant, uint32_t tables, const uint16_t *aux, uint32_t n,
+               const std::function<uint32_t(int, uint32_t)> &source);
+  void finish();
+
+  bool has(int level) const { return level + 1 < int(level_task_.size()) && level_task_[level + 1] > level_task_[level]; }
+  uint64_t pairs() const { return pairs_; }  // (row, source) pairs, and the column slots issued
+  uint64_t slots() const { return slots_; }
+  size_t bytes() const;
+  // M2L of the levels first .. last: X the multipoles, Y the locals; contract(f) runs the
+  // kernel launch f
+  void launch(hipStream_t s, int first, int last, const double *X, double *Y,
+              const std::function<void(const std::function<void()> &)> &contract);
+
+ private:
+  int p_ = 0, nlevels_ = 0, sets_ = 1;
+  bool mixed_ = false;
+  size_t nvec_ = 0;
+  std::vector<size_t> level_vec_;
+  uint64_t pairs_ = 0, slots_ = 0;
+  ReflectLayout lay_{0, 16};
+  dev::ReflectArgs args_{};
+  std::vector<uint32_t> row_out_h_, src_h_, row_table_h_, level_row_;
+  std::vector<uint8_t> row_flip_h_;
+  std::vector<double> tables_h_;
+  std::vector<uint16_t> tables16_h_;
+  uint32_t ntables_ = 0;
+  DevBuf<uint32_t> first_, row_out_, src_;
+  DevBuf<uint16_t> tables16_;
+  DevBuf<uint64_t> kmask_;
+  DevBuf<uint8_t> parity_, tile_class_, row_flip_;
+  DevBuf<int32_t> perm_, tile_row_;
+  DevBuf<dev::ReflectTask> tasks_;
+  DevBuf<double> tables_, sorted_, scratch_;
+  std::vector<uint32_t> level_task_, red_level_;
+  Rows red_;
+};
+
 }  // namespace fmmh

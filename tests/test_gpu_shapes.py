@@ -94,3 +94,22 @@ def test_helmholtz_p2p_rows_over_waves(k, leaf, gradients, precision, tol):
         errs.append(np.linalg.norm(out.gradient - grad) / np.linalg.norm(grad))
     _log(f"  errors {errs}")
     assert max(errs) < tol, errs
+
+
+@pytest.mark.parametrize("precision,tol", [("f64", 1e-12), ("mixed", 2e-6)])
+@pytest.mark.parametrize("p,k", [(5, 3.0 + 0.2j), (9, 6.0)])
+def test_helmholtz_m2l_reflection_classes(p, k, precision, tol):
+    """Enough pairs for the classes (100,000): complex tables as two sets, a level at a time."""
+    _log(f"case Helmholtz M2L reflection p={p} k={k} {precision}")
+    rng = O.Rng(56)
+    pts = np.vstack([rng.cube(9000), rng.plummer(1000, (0.5, 0.5, 0.5), 0.02)])
+    q = rng.normals(len(pts)) + 1j * rng.normals(len(pts))
+    b = fmm_amd.HelmholtzFmmBuilder(k, degree=p).max_points_per_leaf(10).precision(precision)
+    fmm = b.build(pts)
+    assert sum(len(fmm.plan.list("v", level)[1]) for level in range(2, fmm.plan.nlevels)) >= 100_000
+    out = fmm.evaluate(q)
+    phi, grad = O.Fmm(pts, p=p, leaf_points=10).evaluate_helmholtz(k, q)
+    errs = [np.linalg.norm(out.potential - phi) / np.linalg.norm(phi),
+            np.linalg.norm(out.gradient - grad) / np.linalg.norm(grad)]
+    _log(f"  errors {errs}")
+    assert max(errs) < tol, errs
