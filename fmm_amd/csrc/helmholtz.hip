@@ -285,8 +285,28 @@ __global__ __launch_bounds__(256) void k_h_expand(int p, uint32_t rows, const ui
   }
 }
 
+constexpr int kRowWaves = 4;  // waves that share a target leaf's row (P2P, M2P)
+
+// The waves' sums of a chunk of targets meet in red ([wave - 1][sum][lane]) and are added in
+// wave order by wave 0, which keeps them; every wave comes here.
+__device__ __forceinline__ void add_waves(int wave, int lane, double (&acc)[8], double (*red)[8][64]) {
+  __syncthreads();
+  if (wave > 0)
+#pragma unroll
+    for (int q = 0; q < 8; ++q) red[wave - 1][q][lane] = acc[q];
+  __syncthreads();
+  if (wave == 0)
+#pragma unroll
+    for (int w = 0; w < kRowWaves - 1; ++w)
+#pragma unroll
+      for (int q = 0; q < 8; ++q) acc[q] += red[w][q][lane];
+}
+
 // ---- L2P / M2P ---------------------------------------------------------------------------
-// One wave per target leaf, one target per lane (chunks of 64).  With C the entry box's
+// L2P: one wave per target leaf, one target per lane (chunks of 64).  M2P: kRowWaves waves
+// per leaf and chunk, which take the row's boxes in turn, each with its own coefficients in
+// LDS, their sums added in wave order (rows are few and their boxes many: 80,000 Plummer
+// points, 31 rows: 1.5 -> 0.3 ms).  With C the entry box's
 // coefficients (two planes in LDS) and v the target in the box's units,
 //   F = sum_n c_n sum_m C_n^m S_n^m(v),   grad F = sum_n c_n grad(...) + (sum_n d_n ...) v,
 // L2P: c_n = e^-beta (kh/s)^n g_n, d_n = -kh^2 e^-beta (kh/s)^n g_{n+1};
@@ -303,7 +323,7 @@ __global__ __launch_bounds__(256) void k_h_expand(int p, uint32_t rows, const ui
 // and D_{n-1,+q} = Re(beta_q) / N, D_{n-1,-q} = -Im(beta_q) / N.  Each target then runs the
 // harmonic recursion column by column (orders m, degrees n = m .. p) with scalar state.
 template <bool SING, bool GRAD>
-__global__ __launch_bounds__(64) void k_h_evaluate(int p, uint32_t rows, const uint32_t *__restrict__ row_leaf,
+__global__ __launch_bounds__(SING ? 64 * kRowWaves : 64) void k_h_evaluate(int p, uint32_t rows, const uint32_t *__restrict__ row_leaf,
                                                    const uint32_t *__restrict__ row_off,
                                                    const uint32_t *__restrict__ row_box,
                                                    const uint32_t *__restrict__ box_cell,
@@ -314,23 +334,28 @@ __global__ __launch_bounds__(64) void k_h_evaluate(int p, uint32_t rows, const u
                                                    double *grad_hat) {
   // coefficients scaled by their normalisation, (re, im) planes interleaved: C[t] =
   // N_t (c_re[t], c_im[t]); derivative coefficients likewise, D[q][t] = N_t (D_re, D_im)
-  __shared__ double2 C[kMaxCoef];
-  __shared__ double2 D[3][kMaxCoef];
+  constexpr int W = SING ? kRowWaves : 1;
+  __shared__ double2 Cs[W][kMaxCoef];
+  __shared__ double2 Ds[W][3][kMaxCoef];
+  __shared__ double red[SING ? W - 1 : 1][SING ? 8 : 1][SING ? 64 : 1];
   __shared__ double Nm[kMaxCoef];
   __shared__ double rinv[kMaxDegree + 1][kMaxDegree + 1];  // [n][m]: 1/((n+m)(n-m)), n >= m + 2
   const uint32_t row = xcd_index(rows);
   if (row >= rows) return;
   const int P1 = p + 1, nc = P1 * P1;
-  const int lane = threadIdx.x;
-  for (int t = lane; t < nc; t += 64) Nm[t] = norm[t];
-  for (int t = lane; t < (kMaxDegree + 1) * (kMaxDegree + 1); t += 64) {
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  double2 *C = Cs[wave];
+  double2(*D)[kMaxCoef] = Ds[wave];
+  for (int t = int(threadIdx.x); t < nc; t += 64 * W) Nm[t] = norm[t];
+  for (int t = int(threadIdx.x); t < (kMaxDegree + 1) * (kMaxDegree + 1); t += 64 * W) {
     const int n = t / (kMaxDegree + 1), m = t % (kMaxDegree + 1);
     rinv[n][m] = n > m ? 1.0 / double((n + m) * (n - m)) : 0.0;
   }
   const uint32_t lf = row_leaf[row];
   const uint32_t t0 = tgt_start[lf], t1 = tgt_start[lf + 1];
   const uint32_t *lcell = leaf_cell + 4 * size_t(lf);
-  for (uint32_t tb = t0; tb < t1; tb += 64) {
+  __syncthreads();
+  for (uint32_t tb = t0 + 64 * blockIdx.y; tb < t1; tb += 64 * gridDim.y) {
     const uint32_t t = tb + lane;
     const bool active = t < t1;
     double u[3] = {0.0, 0.0, 0.0};
@@ -340,13 +365,13 @@ __global__ __launch_bounds__(64) void k_h_evaluate(int p, uint32_t rows, const u
       u[2] = tz[t];
     }
     cx phi = {0.0, 0.0}, g[3] = {{0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}};
-    for (uint32_t e = row_off[row]; e < row_off[row + 1]; ++e) {
+    for (uint32_t e = row_off[row] + uint32_t(wave); e < row_off[row + 1]; e += W) {
       const uint32_t box = row_box[e];
-      __syncthreads();
+      wave_sync();
       for (int i = lane; i < nc; i += 64)
         C[i] = make_double2(Nm[i] * coeffs[(3 * size_t(box)) * nc + i],
                             Nm[i] * coeffs[(3 * size_t(box) + 1) * nc + i]);
-      __syncthreads();
+      wave_sync();
       if (GRAD)
         for (int i = lane; i < p * p; i += 64) {
           // derivative coefficient slot i = (n', m') of degree n' = n - 1
@@ -442,7 +467,7 @@ __global__ __launch_bounds__(64) void k_h_evaluate(int p, uint32_t rows, const u
         }
         cn[kMaxDegree + 1] = {0.0, 0.0};
       }
-      __syncthreads();
+      wave_sync();
       cx f = {0.0, 0.0}, rad = {0.0, 0.0}, gr[3] = {{0.0, 0.0}, {0.0, 0.0}, {0.0, 0.0}};
       double dr = 1.0, di = 0.0;  // R_m^m
       for (int m = 0; m <= p; ++m) {
@@ -496,6 +521,15 @@ __global__ __launch_bounds__(64) void k_h_evaluate(int p, uint32_t rows, const u
         for (int q = 0; q < 3; ++q) g[q] = cadd(g[q], cscale(cadd(gr[q], cscale(rad, vv[q])), s2));
       }
     }
+    if constexpr (SING) {
+      double acc[8] = {phi.re, phi.im, g[0].re, g[0].im, g[1].re, g[1].im, g[2].re, g[2].im};
+      add_waves(wave, lane, acc, red);
+      if (wave > 0) continue;
+      phi = {acc[0], acc[1]};
+      g[0] = {acc[2], acc[3]};
+      g[1] = {acc[4], acc[5]};
+      g[2] = {acc[6], acc[7]};
+    }
     if (active) {
       phi_hat[2 * size_t(t)] += phi.re;
       phi_hat[2 * size_t(t) + 1] += phi.im;
@@ -510,8 +544,8 @@ __global__ __launch_bounds__(64) void k_h_evaluate(int p, uint32_t rows, const u
 }
 
 // ---- P2P ---------------------------------------------------------------------------------
-// One workgroup of kP2pWaves waves per target leaf; wave w takes the near entries w, w +
-// kP2pWaves, ... of the leaf's row, and the waves' f64 sums are added in wave order, so a
+// One workgroup of kRowWaves waves per target leaf; wave w takes the near entries w, w +
+// kRowWaves, ... of the leaf's row, and the waves' f64 sums are added in wave order, so a
 // few large leaves do not hold up the launch (80,000 Plummer points: 1,905 leaves, one of
 // them with 30 times the mean's pairs).  Within a wave lanes are (phase, target slot), one
 // or two targets per lane (the fuller use of the lanes), the phases splitting each source
@@ -524,8 +558,6 @@ __global__ __launch_bounds__(64) void k_h_evaluate(int p, uint32_t rows, const u
 // math library's sqrt, division and sincos, whose reductions for huge arguments it carries
 // along).  f32: 1/r from v_rsq_f32 (1 ulp) and r = r^2 / r; sine and cosine from v_sin_f32
 // and v_cos_f32 of the fraction of x / (2 pi).
-constexpr int kP2pWaves = 4;
-
 template <typename T>
 struct PairMath;
 
@@ -592,22 +624,6 @@ struct PairMath<float> {
 // e^{i k_t r_t} / r_t = rho e^{i k' r'} / r' and its gradient is rho^2 (i k' r' - 1)
 // e^{i k' r'} d' / r'^3, so an entry's f32 sums (at most 128 sources) go into the f64
 // sums scaled by rho and rho^2 (powers of two).
-//
-// The waves' sums of a chunk meet in red ([wave - 1][sum][lane]) and are added in wave order
-// by wave 0, which keeps them; every wave comes here.
-__device__ __forceinline__ void add_waves(int wave, int lane, double (&acc)[8], double (*red)[8][64]) {
-  __syncthreads();
-  if (wave > 0)
-#pragma unroll
-    for (int q = 0; q < 8; ++q) red[wave - 1][q][lane] = acc[q];
-  __syncthreads();
-  if (wave == 0)
-#pragma unroll
-    for (int w = 0; w < kP2pWaves - 1; ++w)
-#pragma unroll
-      for (int q = 0; q < 8; ++q) acc[q] += red[w][q][lane];
-}
-
 template <bool GRAD, bool DAMP, bool TWO>
 __device__ __forceinline__ void h_p2p_uniform(double (*red)[8][64], uint32_t lf, uint32_t tb, uint32_t n,
                                               uint32_t e0, uint32_t e1,
@@ -636,7 +652,7 @@ __device__ __forceinline__ void h_p2p_uniform(double (*red)[8][64], uint32_t lf,
 #pragma unroll
     for (int q = 0; q < 8; ++q) acc[a][q] = 0.0;
   const uint32_t *ct = leaf_cell + 4 * size_t(lf);
-  for (uint32_t e = e0 + uint32_t(wave); e < e1; e += kP2pWaves) {
+  for (uint32_t e = e0 + uint32_t(wave); e < e1; e += kRowWaves) {
     const uint32_t sl = near_ent[e];
     const uint32_t s0 = src_start[sl], s1 = src_start[sl + 1];
     if (s0 == s1) continue;
@@ -732,8 +748,8 @@ __device__ __forceinline__ void h_p2p_uniform(double (*red)[8][64], uint32_t lf,
 
 template <typename T>
 struct HP2pStage {
-  T ys[kP2pWaves][64][8];  // per wave: y hi (3), y lo (3, f32 only), q re, q im
-  double red[kP2pWaves - 1][8][64];
+  T ys[kRowWaves][64][8];  // per wave: y hi (3), y lo (3, f32 only), q re, q im
+  double red[kRowWaves - 1][8][64];
 };
 
 // A chunk of n targets, A per lane: np = ceil(n / A) lanes per phase, floor(64 / np) phases.
@@ -770,7 +786,7 @@ __device__ __forceinline__ void h_p2p_staged(HP2pStage<T> &sh, uint32_t lf, uint
 #pragma unroll
     for (int q = 0; q < 8; ++q) acc[a][q] = 0.0;
   }
-  for (uint32_t e = e0 + uint32_t(wave); e < e1; e += kP2pWaves) {
+  for (uint32_t e = e0 + uint32_t(wave); e < e1; e += kRowWaves) {
     const uint32_t sl = near_ent[e];
     const uint32_t s0 = src_start[sl], s1 = src_start[sl + 1];
     double c[3] = {0.0, 0.0, 0.0}, r = 1.0;
@@ -860,7 +876,7 @@ __device__ __forceinline__ void h_p2p_staged(HP2pStage<T> &sh, uint32_t lf, uint
 }
 
 template <typename T, bool GRAD, bool DAMP>
-__global__ __launch_bounds__(64 * kP2pWaves) void k_h_p2p(
+__global__ __launch_bounds__(64 * kRowWaves) void k_h_p2p(
     uint32_t leaf_first, uint32_t count, const uint32_t *__restrict__ near_off, const uint32_t *__restrict__ near_ent,
     const uint32_t *__restrict__ leaf_cell, const uint32_t *__restrict__ src_start,
     const uint32_t *__restrict__ tgt_start, const double *__restrict__ sx, const double *__restrict__ sy,
@@ -1045,7 +1061,7 @@ void h_evaluate(hipStream_t s, int p, int singular, int gradients, uint32_t rows
                 double *grad_hat) {
   if (rows == 0) return;
 #define FMMH_HEVAL(S, G)                                                                                        \
-  hipLaunchKernelGGL((k_h_evaluate<S, G>), dim3(xcd_grid(rows)), dim3(64), 0, s, p, rows, row_leaf, row_off,   \
+  hipLaunchKernelGGL((k_h_evaluate<S, G>), dim3(xcd_grid(rows), S ? 4 : 1), dim3(S ? 64 * kRowWaves : 64), 0, s, p, rows, row_leaf, row_off,   \
                      row_box, box_cell, leaf_cell, tgt_start, tx, ty, tz, hlev, norm, coeffs, phi_hat, grad_hat)
   if (singular) {
     if (gradients)
@@ -1070,7 +1086,7 @@ void h_p2p(hipStream_t s, uint32_t leaf_first, uint32_t count, int gradients, in
   if (count == 0) return;
   const float4 *r4 = reinterpret_cast<const float4 *>(rec);
 #define FMMH_HP2P(G, D)                                                                                         \
-  hipLaunchKernelGGL((k_h_p2p<T, G, D>), dim3(xcd_grid(count)), dim3(64 * kP2pWaves), 0, s, leaf_first, count, near_off,   \
+  hipLaunchKernelGGL((k_h_p2p<T, G, D>), dim3(xcd_grid(count)), dim3(64 * kRowWaves), 0, s, leaf_first, count, near_off,   \
                      near_ent, leaf_cell, src_start, tgt_start, sx, sy, sz, qr, qi, r4, tx, ty, tz, hlev,       \
                      phi_hat, grad_hat)
   if (gradients) {
