@@ -73,6 +73,10 @@ HelmholtzOperator::HelmholtzOperator(const Plan &plan, const HelmholtzOptions &o
   ns_ = plan.ns;
   nt_ = plan.nt;
   nleaves_ = plan.nleaves();
+  // the first level whose locals can receive anything but their parents'
+  first_local_ = nlevels_;
+  for (int l = nlevels_ - 1; l >= 0; --l)
+    if (plan.v[l].size() > 0 || plan.x[l].size() > 0) first_local_ = l;
   box_base_.assign(nlevels_ + 1, 0);
   for (int l = 0; l < nlevels_; ++l) box_base_[l + 1] = box_base_[l] + plan.nboxes(l);
   nbox_total_ = box_base_[nlevels_];
@@ -891,10 +895,8 @@ void HelmholtzOperator::load_charges(const double *charges, bool on_device) {
 }
 
 void HelmholtzOperator::reset() {
-  dev::fill(stream_, mult_.ptr, mult_.count, 0.0);
-  dev::fill(stream_, loc_.ptr, loc_.count, 0.0);
-  dev::fill(stream_, phi_hat_.ptr, phi_hat_.count, 0.0);
-  dev::fill(stream_, grad_hat_.ptr, grad_hat_.count, 0.0);
+  dev::clear(stream_, dev::ClearList{{mult_.ptr, loc_.ptr, phi_hat_.ptr, grad_hat_.ptr},
+                                     {mult_.count, loc_.count, phi_hat_.count, grad_hat_.count}});
 }
 
 void HelmholtzOperator::launch_p2p() {
@@ -983,8 +985,8 @@ void HelmholtzOperator::evaluate() {
                     p2l_rows_.row_off.ptr, p2l_rows_.row_ent.ptr, leaf_cell_.ptr, src_start_.ptr, sx_.ptr, sy_.ptr,
                     sz_.ptr, qr_.ptr, qi_.ptr, hlev_.ptr, norm_.ptr, loc_.ptr);
     });
-  // downward: L2L from the root
-  for (int l = 1; l <= L; ++l)
+  // downward: L2L from the first level with an M2L or P2L row (the locals above are zero)
+  for (int l = first_local_ + 1; l <= L; ++l)
     timed(2, [&] {
       if (m2m_complex_) dev::h_negate(stream_, p, box_base_[l - 1], box_base_[l], loc_.ptr);
       const Schedule &s = l2l_[l];

@@ -73,7 +73,7 @@ class HelmholtzOperator {
   void launch_p2p();
 
   HelmholtzOptions opt_;
-  int nlevels_ = 0, nc_ = 0;
+  int nlevels_ = 0, nc_ = 0, first_local_ = 0;
   bool m2m_complex_ = true;  // M2M / L2L tables have an imaginary part (not for real k)
   hipStream_t stream_ = nullptr;
   hipEvent_t order_event_ = nullptr;  // wait_for: a caller's stream before this one

@@ -57,6 +57,11 @@ __device__ __forceinline__ void wave_sync() {
 hipError_t upload_constants();
 
 void fill(hipStream_t s, double *p, size_t n, double v);
+struct ClearList {
+  double *p[4];
+  size_t n[4];
+};
+void clear(hipStream_t s, const ClearList &c);  // zeros into p[k][0 .. n[k])
 // q64[j] = q[order[j]]; with rec set, also rec[8 j + 3] = f32 of it (the charge slot of
 // the mixed-precision P2P source records)
 void gather_charges(hipStream_t s, const double *q, const uint32_t *order, size_t n, double *q64, float *rec);

@@ -144,6 +144,11 @@ DeviceOperator::DeviceOperator(const Plan &plan, const OperatorOptions &options)
     }
   }
 
+  // the first level whose locals can receive anything but their parents'
+  first_local_ = nlevels_;
+  for (int l = nlevels_ - 1; l >= 0; --l)
+    if (plan.v[l].size() > 0 || plan.x[l].size() > 0) first_local_ = l;
+
   // expansions and outputs (the clustered-mode scratch rows are sized in build_schedules)
   // 64 doubles past the last box: the per-M-tile M2M reads a source expansion as four
   // runs of 4 ceil(nc / 16) values (at most 15 past its end) and masks the tail
@@ -831,10 +836,8 @@ void DeviceOperator::load_charges(const double *charges, bool on_device) {
 }
 
 void DeviceOperator::reset() {
-  dev::fill(stream_, mult_.ptr, mult_.count, 0.0);
-  dev::fill(stream_, loc_.ptr, loc_.count, 0.0);
-  dev::fill(stream_, phi_hat_.ptr, phi_hat_.count, 0.0);
-  dev::fill(stream_, grad_hat_.ptr, grad_hat_.count, 0.0);
+  dev::clear(stream_, dev::ClearList{{mult_.ptr, loc_.ptr, phi_hat_.ptr, grad_hat_.ptr},
+                                     {mult_.count, loc_.count, phi_hat_.count, grad_hat_.count}});
 }
 
 void DeviceOperator::p2m(int level) {
@@ -931,7 +934,8 @@ void DeviceOperator::evaluate() {
   // local receives its M2L, P2L and L2L terms, each kind in the order of its row.
   if (L >= 2) timed(3, [&] { launch_m2l(2, L); });
   if (L >= 1) timed(4, [&] { launch_p2l(1, L); });
-  for (int l = 1; l <= L; ++l) l2l(l);
+  // (down to the first level with an M2L or P2L row every local is zero)
+  for (int l = first_local_ + 1; l <= L; ++l) l2l(l);
   // leaves: each kind over every level at once; a target still receives L2P, M2P and
   // P2P contributions in that order
   timed(5, [&] {

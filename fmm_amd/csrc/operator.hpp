@@ -149,7 +149,7 @@ class DeviceOperator {
   void launch_p2l(int level_first, int level_last);
 
   OperatorOptions opt_;
-  int nlevels_ = 0, nc_ = 0;
+  int nlevels_ = 0, nc_ = 0, first_local_ = 0;
   hipStream_t stream_ = nullptr;
   hipEvent_t order_event_ = nullptr;  // wait_for: a caller's stream before this one
   int64_t ns_ = 0, nt_ = 0;

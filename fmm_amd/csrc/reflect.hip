@@ -776,27 +776,40 @@ void ReflectM2l::finish() {
     red_level_[l + 1] = static_cast<uint32_t>(red_id.size());
   }
   slots_ = uint64_t(width) * kReflectPositions * base_tasks;
-  red_.rows = static_cast<uint32_t>(red_id.size());
-  red_.row_id.upload(red_id);
-  red_.row_off.upload(red_off);
-  red_.row_ent.upload(red_ent);
-  scratch_.alloc(size_t(nscratch) * lay_.nc);
-  tasks_.upload(tasks);
-  row_out_.upload(row_out_h_);
-  row_flip_.upload(row_flip_h_);
-  src_.upload(src_h_);
   std::vector<uint32_t> first;
   for (int c = 0; c <= kReflectClasses; ++c)
     first.push_back(uint32_t(rc.first[c]) | uint32_t(c < kReflectClasses ? rc.axes[c] : 0) << 16);
-  first_.upload(first);
   std::vector<uint64_t> kmask;
   for (int axes = 0; axes < 8; ++axes)
     for (int c = 0; c < 8; ++c) kmask.push_back(lay_.steps(axes, c, mixed_ ? dev::kReflectChunk16 : 4));
-  kmask_.upload(kmask);
-  parity_.upload(lay_.parity);
-  tile_class_.upload(lay_.tile_class);
-  perm_.upload(lay_.perm);
-  tile_row_.upload(lay_.tile_row);
+  // every index array in one allocation and one copy
+  std::vector<uint8_t> blob;
+  auto put = [&](const auto &v) {
+    const size_t at = (blob.size() + 63) / 64 * 64, n = v.size() * sizeof(v[0]);
+    blob.resize(at + n);
+    if (n) std::memcpy(blob.data() + at, v.data(), n);
+    return at;
+  };
+  const size_t o_first = put(first), o_kmask = put(kmask), o_parity = put(lay_.parity), o_rows = put(lay_.tile_row),
+               o_class = put(lay_.tile_class), o_perm = put(lay_.perm), o_tasks = put(tasks), o_out = put(row_out_h_),
+               o_flip = put(row_flip_h_), o_src = put(src_h_), o_rid = put(red_id), o_roff = put(red_off),
+               o_rent = put(red_ent);
+  index_.upload(blob);
+  auto at = [&](size_t o) { return static_cast<const void *>(index_.ptr + o); };
+  perm_ = static_cast<const int32_t *>(at(o_perm));
+  red_id_ = static_cast<const uint32_t *>(at(o_rid));
+  red_off_ = static_cast<const uint32_t *>(at(o_roff));
+  red_ent_ = static_cast<const uint32_t *>(at(o_rent));
+  args_.first = static_cast<const uint32_t *>(at(o_first));
+  args_.kmask = static_cast<const uint64_t *>(at(o_kmask));
+  args_.parity = static_cast<const uint8_t *>(at(o_parity));
+  args_.tile_row = static_cast<const int32_t *>(at(o_rows));
+  args_.tile_class = static_cast<const uint8_t *>(at(o_class));
+  args_.tasks = static_cast<const dev::ReflectTask *>(at(o_tasks));
+  args_.row_out = static_cast<const uint32_t *>(at(o_out));
+  args_.row_flip = static_cast<const uint8_t *>(at(o_flip));
+  args_.src = static_cast<const uint32_t *>(at(o_src));
+  scratch_.alloc(size_t(nscratch) * lay_.nc);
   // (after the last chunk a wave reads, and drops, the next chunk's tiles)
   if (mixed_) {
     tables16_h_.resize(tables16_h_.size() + size_t(lay_.tiles + 4) * 1536);
@@ -811,16 +824,7 @@ void ReflectM2l::finish() {
   args_.kp = lay_.kp;
   args_.tiles = lay_.tiles;
   std::copy(rc.run.begin(), rc.run.end(), args_.run);
-  args_.first = first_.ptr;
-  args_.kmask = kmask_.ptr;
-  args_.parity = parity_.ptr;
-  args_.tile_row = tile_row_.ptr;
-  args_.tile_class = tile_class_.ptr;
-  args_.tasks = tasks_.ptr;
   args_.sets = sets_;
-  args_.row_out = row_out_.ptr;
-  args_.row_flip = row_flip_.ptr;
-  args_.src = src_.ptr;
   std::vector<uint32_t>().swap(row_out_h_);
   std::vector<uint32_t>().swap(src_h_);
   std::vector<uint32_t>().swap(row_table_h_);
@@ -830,7 +834,7 @@ void ReflectM2l::finish() {
 }
 
 size_t ReflectM2l::bytes() const {
-  return tables_.bytes() + tables16_.bytes() + sorted_.bytes() + scratch_.bytes() + src_.bytes();
+  return tables_.bytes() + tables16_.bytes() + sorted_.bytes() + scratch_.bytes() + index_.bytes();
 }
 
 void ReflectM2l::launch(hipStream_t s, int first, int last, const double *X, double *Y,
@@ -842,7 +846,7 @@ void ReflectM2l::launch(hipStream_t s, int first, int last, const double *X, dou
   while (!has(first)) ++first;
   while (!has(last)) --last;
   const size_t vec0 = level_vec_[first], vec1 = level_vec_[last + 1];
-  dev::reflect_sort(s, lay_.nc, lay_.kp, vec1 - vec0, perm_.ptr, X + vec0 * lay_.nc, sorted_.ptr + vec0 * lay_.kp);
+  dev::reflect_sort(s, lay_.nc, lay_.kp, vec1 - vec0, perm_, X + vec0 * lay_.nc, sorted_.ptr + vec0 * lay_.kp);
   dev::ReflectArgs args = args_;
   args.tasks += t0;
   contract([&] {
@@ -853,7 +857,7 @@ void ReflectM2l::launch(hipStream_t s, int first, int last, const double *X, dou
   });
   const uint32_t r0 = red_level_[first], r1 = red_level_[last + 1];
   if (r1 > r0)
-    dev::reduce_slots(s, p_, r1 - r0, red_.row_id.ptr + r0, red_.row_off.ptr + r0, red_.row_ent.ptr, 0, scratch_.ptr,
+    dev::reduce_slots(s, p_, r1 - r0, red_id_ + r0, red_off_ + r0, red_ent_, 0, scratch_.ptr,
                       nullptr, Y);
 }
 

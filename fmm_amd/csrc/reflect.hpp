@@ -149,15 +149,12 @@ class ReflectM2l {
   std::vector<double> tables_h_;
   std::vector<uint16_t> tables16_h_;
   uint32_t ntables_ = 0;
-  DevBuf<uint32_t> first_, row_out_, src_;
+  DevBuf<uint8_t> index_;  // the index arrays, also those of the scratch rows' reduction
+  const int32_t *perm_ = nullptr;
+  const uint32_t *red_id_ = nullptr, *red_off_ = nullptr, *red_ent_ = nullptr;
   DevBuf<uint16_t> tables16_;
-  DevBuf<uint64_t> kmask_;
-  DevBuf<uint8_t> parity_, tile_class_, row_flip_;
-  DevBuf<int32_t> perm_, tile_row_;
-  DevBuf<dev::ReflectTask> tasks_;
   DevBuf<double> tables_, sorted_, scratch_;
   std::vector<uint32_t> level_task_, red_level_;
-  Rows red_;
 };
 
 }  // namespace fmmh
