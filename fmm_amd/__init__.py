@@ -288,8 +288,8 @@ class Operator:
         _lib.check(_lib.lib().fmmh_evaluate_graph(self._h))
 
     def read_output(self) -> Output:
-        phi = np.zeros(self.ntargets)
-        grad = np.zeros((self.ntargets, 3)) if self.gradients else None
+        phi = np.empty(self.ntargets)
+        grad = np.empty((self.ntargets, 3)) if self.gradients else None
         _lib.check(_lib.lib().fmmh_read_output(self._h, _lib.ptr(phi), _lib.ptr(grad), self.ntargets, 0))
         return Output(phi, grad)
 
@@ -742,8 +742,8 @@ class HelmholtzOperator:
         _lib.check(_lib.lib().fmmh_helmholtz_evaluate(self._h))
 
     def read_output(self) -> Output:
-        phi = np.zeros(2 * self.ntargets)
-        grad = np.zeros(6 * self.ntargets) if self.gradients else None
+        phi = np.empty(2 * self.ntargets)
+        grad = np.empty(6 * self.ntargets) if self.gradients else None
         _lib.check(_lib.lib().fmmh_helmholtz_read_output(self._h, _lib.ptr(phi), _lib.ptr(grad), self.ntargets, 0))
         return Output(phi.view(np.complex128),
                       grad.view(np.complex128).reshape(-1, 3) if self.gradients else None)

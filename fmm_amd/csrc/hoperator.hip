@@ -1014,8 +1014,9 @@ void HelmholtzOperator::read_output(double *phi, double *grad, bool on_device) {
   dev::h_output(stream_, nleaves_, tgt_start_.ptr, leaf_r_.ptr, tgt_order_.ptr, phi_hat_.ptr, grad_hat_.ptr,
                 on_device ? phi : phi_.ptr, on_device ? grad : grad_.ptr, g);
   if (!on_device) {
-    hip_check(hipMemcpyAsync(phi, phi_.ptr, 2 * nt_ * sizeof(double), hipMemcpyDeviceToHost, stream_), "phi");
-    if (g) hip_check(hipMemcpyAsync(grad, grad_.ptr, 6 * nt_ * sizeof(double), hipMemcpyDeviceToHost, stream_), "grad");
+    std::vector<HostCopy> out{{phi, phi_.ptr, 2 * nt_ * sizeof(double)}};
+    if (g) out.push_back({grad, grad_.ptr, 6 * nt_ * sizeof(double)});
+    stage_.download(opt_.device, stream_, out);
   }
   sync();
 }

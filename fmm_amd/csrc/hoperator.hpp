@@ -73,6 +73,7 @@ class HelmholtzOperator {
   void launch_p2p();
 
   HelmholtzOptions opt_;
+  HostStageUser stage_;  // downloads into host arrays
   int nlevels_ = 0, nc_ = 0, first_local_ = 0;
   bool m2m_complex_ = true;  // M2M / L2L tables have an imaginary part (not for real k)
   hipStream_t stream_ = nullptr;

@@ -970,10 +970,9 @@ void DeviceOperator::read_output(double *phi, double *grad, bool on_device) {
                    grad_hat_.ptr, on_device ? phi : phi_.ptr, on_device ? grad : grad_.ptr,
                    opt_.gradients && grad != nullptr);
   if (!on_device) {
-    hip_check(hipMemcpyAsync(phi, phi_.ptr, nt_ * sizeof(double), hipMemcpyDeviceToHost, stream_), "download phi");
-    if (opt_.gradients && grad)
-      hip_check(hipMemcpyAsync(grad, grad_.ptr, 3 * nt_ * sizeof(double), hipMemcpyDeviceToHost, stream_),
-                "download grad");
+    std::vector<HostCopy> out{{phi, phi_.ptr, nt_ * sizeof(double)}};
+    if (opt_.gradients && grad) out.push_back({grad, grad_.ptr, 3 * nt_ * sizeof(double)});
+    stage_.download(opt_.device, stream_, out);
   }
   sync();
 }
@@ -1008,10 +1007,9 @@ void DeviceOperator::vjp(const double *q, const double *g, const double *field, 
                    grad_hat_.ptr, phi_.ptr, grad_.ptr, 1);
   dev::vjp_combine(stream_, n, dq, dg, phi_.ptr, grad_.ptr, df, oq, op);
   if (!on_device) {
-    hip_check(hipMemcpyAsync(grad_q, oq, n * sizeof(double), hipMemcpyDeviceToHost, stream_), "vjp grad_q");
-    if (grad_pos)
-      hip_check(hipMemcpyAsync(grad_pos, op, 3 * n * sizeof(double), hipMemcpyDeviceToHost, stream_),
-                "vjp grad_pos");
+    std::vector<HostCopy> out{{grad_q, oq, n * sizeof(double)}};
+    if (grad_pos) out.push_back({grad_pos, op, 3 * n * sizeof(double)});
+    stage_.download(opt_.device, stream_, out);
   }
   sync();
 }

@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "devbuf.hpp"
+#include "hoststage.hpp"
 #include "plan.hpp"
 #include "pwkernels.hpp"
 #include "reflect.hpp"
@@ -149,6 +150,7 @@ class DeviceOperator {
   void launch_p2l(int level_first, int level_last);
 
   OperatorOptions opt_;
+  HostStageUser stage_;  // downloads into host arrays
   int nlevels_ = 0, nc_ = 0, first_local_ = 0;
   hipStream_t stream_ = nullptr;
   hipEvent_t order_event_ = nullptr;  // wait_for: a caller's stream before this one

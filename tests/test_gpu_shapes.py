@@ -113,3 +113,35 @@ def test_helmholtz_m2l_reflection_classes(p, k, precision, tol):
             np.linalg.norm(out.gradient - grad) / np.linalg.norm(grad)]
     _log(f"  errors {errs}")
     assert max(errs) < tol, errs
+
+
+def test_host_downloads_of_every_size():
+    """Host outputs (through the pinned staging, in chunks of both halves, and the small ones
+    past it) against the same evaluation's device outputs, from two threads at once."""
+    import threading
+
+    import torch
+
+    _log("case host downloads")
+    rng = O.Rng(57)
+
+    def one(n, out):
+        pts = rng_pts[n]
+        fmm = fmm_amd.FmmBuilder(3).max_points_per_leaf(64).build(pts)
+        q = np.cos(np.arange(n))
+        host = fmm.evaluate(q)
+        phi = torch.empty(n, dtype=torch.float64, device="cuda")
+        grad = torch.empty(n, 3, dtype=torch.float64, device="cuda")
+        fmm.operator.read_output_device(phi, grad)
+        out[n] = np.array_equal(host.potential, phi.cpu().numpy()) and np.array_equal(host.gradient,
+                                                                                      grad.cpu().numpy())
+
+    sizes = (2, 700, 2049, 9001, 65_536, 400_003)
+    rng_pts = {n: rng.cube(n) for n in sizes}
+    out = {}
+    work = [threading.Thread(target=lambda part=part: [one(n, out) for n in part]) for part in (sizes[::2], sizes[1::2])]
+    for t in work:
+        t.start()
+    for t in work:
+        t.join()
+    assert out == {n: True for n in sizes}
