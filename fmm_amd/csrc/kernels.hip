@@ -221,12 +221,16 @@ __global__ void k_vjp_combine(size_t n, const double *q, const double *g, const 
 // y^ = fma(r^, u_s, c^) formed once per source in f64 (u_s itself for s = t).  A pair adds
 // nothing when r^2 == 0: the select comes before the charge is touched.
 //
-// T = double: every operation in f64.  T = float (mixed precision): coordinates stay
-// f64 in HBM; each is split into hi + lo floats (hi = fl32(u), lo = fl32(u - hi)) and the
-// separation is formed as (t_hi - y_hi) + (t_lo - y_lo), which keeps it accurate to about
-// 2^-24 of |d| even for close pairs (a plain f32 difference loses 2^-24 of |u| >> |d|);
-// r^2, the inverse square root and the sums of a tile (at most 64 sources) are f32; the
-// tile sums are added in f64.  Coincident points give d = 0 exactly in both forms.
+// T = double: every operation in f64.  T = float (mixed precision): coordinates stay f64 in
+// HBM; a staged source's position in the target leaf's frame and the targets' are rounded to
+// 32-bit fixed point (u 2^28; a near pair is within 7 half-widths in either frame, checked at
+// build), so the separation is one exact integer subtraction and one conversion per axis,
+// accurate to 2^-29 half-widths; a pair closer than 2^-4.5 half-widths takes its separation
+// from the f64 positions instead, so every pair keeps about 2^-24 of |d|.  r^2, the inverse
+// square root and the sums of a tile (at most 64 sources) are f32; the tile sums are added
+// in f64.  Coincident points give d = 0 exactly in both forms.  (VALU bound: the fixed point
+// takes the place of a split into hi + lo floats, 6 operations a pair less, and one LDS read
+// a source less; 1M points, p = 8: 689 -> 603 us.)
 
 // Lane mapping (one wave per target leaf, targets processed in chunks of 128): the staged
 // form puts one or two targets in each lane (the fuller use of the lanes), np lanes per
@@ -241,7 +245,7 @@ __global__ void k_vjp_combine(size_t n, const double *q, const double *g, const 
 // leaves): that tile selects 0 for r^2 == 0; other tiles start r^2 from the smallest
 // normal number, which changes nothing for distinct points (r^2 >= 1e-22 in leaf units
 // at the deepest level) and keeps a separation rounded to zero finite.
-// Chunks of at least `umin` targets in the mixed path (33 by the static rule): each lane
+// Chunks of at least `umin` targets in the mixed path (43 by the static rule): each lane
 // holds one target (TWO: two, the second 64 further on) and at every step all lanes take
 // the same source, read from its 16-byte record by uniform loads, so no LDS staging and
 // no lanes split over phases.  A record holds the source's coordinates in its own leaf's
@@ -420,11 +424,11 @@ __device__ __forceinline__ void p2p_uniform(uint32_t lf, uint32_t tb, uint32_t n
 // Shared memory of one wave of the staged form.
 template <typename T>
 struct P2pStage {
-  // a source: (x, y, z, q) and, for the split form, (x_lo, y_lo, z_lo, 0), so a lane reads
-  // it with one or two 16-byte loads
-  using V4 = typename std::conditional<sizeof(T) == 4, float4, double4>::type;
+  // a source in the target leaf's frame: f64 (x, y, z, q), or for T = float fixed point
+  // (u 2^28 in int32) and the charge's f32 bits, 16 bytes, so a lane reads it with one load
+  using V4 = typename std::conditional<sizeof(T) == 4, int4, double4>::type;
   V4 ys[64];
-  float4 yl[sizeof(T) == 4 ? 64 : 1];
+  double yd[sizeof(T) == 4 ? 64 : 1][3];  // T = float: the f64 position (close pairs)
   double fr[64][4];     // frame (c, r) of each entry of a chunk of the near row
   uint32_t fstart[64];  // first source of each entry
   uint32_t fcum[65];    // exclusive prefix sums of the entries' source counts
@@ -443,10 +447,10 @@ __device__ __forceinline__ void p2p_staged(P2pStage<T> &sh, uint32_t lf, uint32_
                                            const double *__restrict__ sq, const double *__restrict__ tx,
                                            const double *__restrict__ ty, const double *__restrict__ tz,
                                            double *__restrict__ phi, double *__restrict__ grad) {
-  constexpr bool SPLIT = sizeof(T) == 4;
+  constexpr bool FIXED = sizeof(T) == 4;
   constexpr int TILE = 64;
   constexpr T TINY = sizeof(T) == 4 ? T(1.17549435e-38f) : T(2.2250738585072014e-308);
-  constexpr double FAR = 1024.0;  // padding position, in target-leaf units
+  constexpr double FAR = FIXED ? 6.0 : 1024.0;  // padding position, in target-leaf units
   using V4 = typename P2pStage<T>::V4;
   const int lane = threadIdx.x;
   const uint32_t *ct = leaf_cell + 4 * size_t(lf);
@@ -454,73 +458,113 @@ __device__ __forceinline__ void p2p_staged(P2pStage<T> &sh, uint32_t lf, uint32_
   const int tsz = phases * (64 / phases);  // sources per tile: a multiple of the phases
   const bool lane_ok = lane < np * phases;
   const int slot = lane % np, phase = lane_ok ? lane / np : 0;
-  T ux[A], uy[A], uz[A], lx[A], ly[A], lz[A], ap[A], ax[A], ay[A], az[A];
+  // the targets, in fixed point for T = float
+  using C = typename std::conditional<FIXED, int, double>::type;
+  C ux[A], uy[A], uz[A];
+  T ap[A], ax[A], ay[A], az[A];
   bool ok[A];
 #pragma unroll
   for (int a = 0; a < A; ++a) {
     const uint32_t i = tb + uint32_t(slot + a * np);
     ok[a] = lane_ok && uint32_t(slot + a * np) < n;
-    const double x = ok[a] ? tx[i] : 0.0, y = ok[a] ? ty[i] : 0.0, z = ok[a] ? tz[i] : 0.0;
-    ux[a] = T(x);
-    uy[a] = T(y);
-    uz[a] = T(z);
-    lx[a] = T(x - double(ux[a]));
-    ly[a] = T(y - double(uy[a]));
-    lz[a] = T(z - double(uz[a]));
+    // (a lane without a target sits where no source comes close, also modulo 2^32)
+    const double idle = FIXED ? -7.9 : 0.0;
+    const double x = ok[a] ? tx[i] : idle, y = ok[a] ? ty[i] : idle, z = ok[a] ? tz[i] : idle;
+    if constexpr (FIXED) {
+      ux[a] = __double2int_rn(x * kP2pFixed);
+      uy[a] = __double2int_rn(y * kP2pFixed);
+      uz[a] = __double2int_rn(z * kP2pFixed);
+    } else {
+      ux[a] = x;
+      uy[a] = y;
+      uz[a] = z;
+    }
     ap[a] = ax[a] = ay[a] = az[a] = T(0);
   }
-  // f32 sums are per tile (at most 64 terms) and go into f64 after each tile, so long
-  // near rows do not lose digits to one growing f32 sum
+  // f32 sums are per tile (at most 64 terms) and go into f64 after each tile,
+  // so long near rows do not lose digits to one growing f32 sum
   double cp[A], cx[A], cy[A], cz[A];
 #pragma unroll
   for (int a = 0; a < A; ++a) cp[a] = cx[a] = cy[a] = cz[a] = 0.0;
   auto flush = [&]() {
-    if (SPLIT) {
+    if (FIXED) {
 #pragma unroll
       for (int a = 0; a < A; ++a) {
-        cp[a] += double(ap[a]);
-        cx[a] += double(ax[a]);
-        cy[a] += double(ay[a]);
-        cz[a] += double(az[a]);
+        cp[a] = fma(double(ap[a]), GRAD ? 1.0 : kP2pFixed, cp[a]);
+        cx[a] = fma(double(ax[a]), 1.0 / kP2pFixed, cx[a]);
+        cy[a] = fma(double(ay[a]), 1.0 / kP2pFixed, cy[a]);
+        cz[a] = fma(double(az[a]), 1.0 / kP2pFixed, cz[a]);
         ap[a] = ax[a] = ay[a] = az[a] = T(0);
       }
     }
   };
-  // one source j of the tile against the lane's targets
-  auto step = [&](int j, auto check) {
-    const V4 v = sh.ys[j];
-    const T yx = v.x, yy = v.y, yz = v.z, q = v.w;
-    T yxl = T(0), yyl = T(0), yzl = T(0);
-    if (SPLIT) {
-      const float4 w = sh.yl[j];
-      yxl = w.x;
-      yyl = w.y;
-      yzl = w.z;
-    }
+  auto minus = [](C a, C b) {
+    if constexpr (FIXED)
+      return float(int(uint32_t(a) - uint32_t(b)));
+    else
+      return a - b;
+  };
+  // the sources j0, j0 + phases, ... (K of them) of the tile against the lane's targets: the
+  // separations and r^2 of every pair first, then for T = float one test for a close pair
+  // among them (its separation again from the f64 positions, rounded once), then the terms
+  auto steps_of = [&](int j0, auto check, auto count) {
+    constexpr int K = decltype(count)::value;
+    T dx[K][A], dy[K][A], dz[K][A], r2[K][A], q[K];
+    T rmin = T(kP2pClose);
 #pragma unroll
-    for (int a = 0; a < A; ++a) {
-      T dx = ux[a] - yx, dy = uy[a] - yy, dz = uz[a] - yz;
-      if (SPLIT) {
-        dx += lx[a] - yxl;
-        dy += ly[a] - yyl;
-        dz += lz[a] - yzl;
-      }
-      T inv;
-      if constexpr (decltype(check)::value) {
-        const T r2 = dx * dx + dy * dy + dz * dz;
-        inv = r2 == T(0) ? T(0) : rsqrt_t<T>(r2);
-      } else {
-        inv = rsqrt_t<T>(fma(dz, dz, fma(dy, dy, fma(dx, dx, TINY))));
-      }
-      const T qi = q * inv;
-      ap[a] += qi;
-      if (GRAD) {
-        const T qi3 = qi * (inv * inv);
-        ax[a] -= qi3 * dx;
-        ay[a] -= qi3 * dy;
-        az[a] -= qi3 * dz;
+    for (int k = 0; k < K; ++k) {
+      const V4 v = sh.ys[j0 + k * phases];
+      if constexpr (FIXED)
+        q[k] = __int_as_float(v.w);
+      else
+        q[k] = v.w;
+#pragma unroll
+      for (int a = 0; a < A; ++a) {
+        dx[k][a] = minus(ux[a], v.x);
+        dy[k][a] = minus(uy[a], v.y);
+        dz[k][a] = minus(uz[a], v.z);
+        r2[k][a] = fma(dz[k][a], dz[k][a],
+                       fma(dy[k][a], dy[k][a], fma(dx[k][a], dx[k][a], FIXED ? T(0.25f) : decltype(check)::value ? T(0) : TINY)));
+        if (FIXED) rmin = fminf(rmin, r2[k][a]);
       }
     }
+    if constexpr (FIXED)
+      if (__any(rmin < kP2pClose)) {
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+#pragma unroll
+          for (int a = 0; a < A; ++a)
+            if (r2[k][a] < kP2pClose && ok[a]) {
+              const double *y = sh.yd[j0 + k * phases];
+              const uint32_t i = tb + uint32_t(slot + a * np);
+              dx[k][a] = float((tx[i] - y[0]) * kP2pFixed);
+              dy[k][a] = float((ty[i] - y[1]) * kP2pFixed);
+              dz[k][a] = float((tz[i] - y[2]) * kP2pFixed);
+              r2[k][a] = fmaf(dz[k][a], dz[k][a],
+                              fmaf(dy[k][a], dy[k][a],
+                                   fmaf(dx[k][a], dx[k][a], decltype(check)::value ? 0.0f : 1.17549435e-38f)));
+            }
+      }
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+#pragma unroll
+      for (int a = 0; a < A; ++a) {
+        T inv;
+        if constexpr (decltype(check)::value)
+          inv = r2[k][a] == T(0) ? T(0) : rsqrt_t<T>(r2[k][a]);
+        else
+          inv = rsqrt_t<T>(r2[k][a]);
+        // (1 / r in leaf units, so that q / r^3 keeps the f32 range of the charges)
+        if (FIXED && GRAD) inv *= T(kP2pFixed);
+        const T qi = q[k] * inv;
+        ap[a] += qi;
+        if (GRAD) {
+          const T qi3 = qi * (inv * inv);
+          ax[a] -= qi3 * dx[k][a];
+          ay[a] -= qi3 * dy[k][a];
+          az[a] -= qi3 * dz[k][a];
+        }
+      }
   };
   // stage one tile: lane < cnt holds the source (x, y, z, q) in the target frame;
   // lanes cnt .. steps * phases - 1 hold zero charges far away
@@ -532,14 +576,19 @@ __device__ __forceinline__ void p2p_staged(P2pStage<T> &sh, uint32_t lf, uint32_
         q = 0.0;
       }
       V4 v;
-      v.x = T(yx);
-      v.y = T(yy);
-      v.z = T(yz);
-      v.w = T(q);
+      if constexpr (FIXED) {
+        v = make_int4(__double2int_rn(yx * kP2pFixed), __double2int_rn(yy * kP2pFixed),
+                      __double2int_rn(yz * kP2pFixed), __float_as_int(float(q)));
+        sh.yd[lane][0] = yx;
+        sh.yd[lane][1] = yy;
+        sh.yd[lane][2] = yz;
+      } else {
+        v.x = yx;
+        v.y = yy;
+        v.z = yz;
+        v.w = q;
+      }
       sh.ys[lane] = v;
-      if (SPLIT)
-        sh.yl[lane] = make_float4(float(yx - double(float(yx))), float(yy - double(float(yy))),
-                                  float(yz - double(float(yz))), 0.0f);
     }
     __syncthreads();
   };
@@ -586,7 +635,7 @@ __device__ __forceinline__ void p2p_staged(P2pStage<T> &sh, uint32_t lf, uint32_
         const bool valid = s < s1;
         stage(cn, steps, valid, valid ? sx[s] : 0.0, valid ? sy[s] : 0.0, valid ? sz[s] : 0.0,
               valid ? sq[s] : 0.0);
-        for (int k2 = 0; k2 < steps; ++k2) step(phase + k2 * phases, std::true_type{});
+        for (int k2 = 0; k2 < steps; ++k2) steps_of(phase + k2 * phases, std::true_type{}, std::integral_constant<int, 1>{});
         flush();
       }
     } else {
@@ -626,15 +675,13 @@ __device__ __forceinline__ void p2p_staged(P2pStage<T> &sh, uint32_t lf, uint32_
       // start the next tile's loads before computing this one
       if (base + uint32_t(tsz) < total) prefetch(base + uint32_t(tsz));
       int k2 = 0;
-      for (; k2 + 2 <= steps; k2 += 2) {
-        step(phase + k2 * phases, std::false_type{});
-        step(phase + (k2 + 1) * phases, std::false_type{});
-      }
-      if (k2 < steps) step(phase + k2 * phases, std::false_type{});
+      for (; k2 + 2 <= steps; k2 += 2)
+        steps_of(phase + k2 * phases, std::false_type{}, std::integral_constant<int, 2>{});
+      if (k2 < steps) steps_of(phase + k2 * phases, std::false_type{}, std::integral_constant<int, 1>{});
       flush();
     }
   }
-  if (!SPLIT) {
+  if (!FIXED) {
 #pragma unroll
     for (int a = 0; a < A; ++a) {
       cp[a] = double(ap[a]);

@@ -50,12 +50,18 @@ enum M2lMethod : int {
                      // approximate to the quadrature's tolerance)
 };
 
+// Chunks of 33 to 42 targets fill 77 to 98% of the staged form's lanes (three phases of two
+// targets per lane) and 52 to 66% of the uniform one's; from 43 on both fill as much, and the
+// uniform form takes fewer instructions.  (P2P with 33 and with 43: 1M points, leaves of 22 to
+// 40, 626 and 539 us; 1.5M, 35 to 57, 1265 and 1130; 156k, 28 to 49, 150 and 154.  49 gains
+// another 3% at 1.5M and loses 9% at 156k to 188k.)
+constexpr int kP2pUniformMin = 43;
 constexpr int kTuneLevels = 17;  // levels 0..16
 
 // Launch-shape decisions an autotuner may take (tune.hip); 0 everywhere is the static rule.
 struct Tuning {
   int p2p_uniform_min = 0;                  // mixed P2P: chunks of at least this many targets read
-                                            // sources by uniform loads (0: 33)
+                                            // sources by uniform loads (0: kP2pUniformMin)
   int m2l_stage = 0;                        // bf16x3 M2L: 0/1 one k-step per pipeline stage,
                                             // 2 two k-steps in a ring of two buffers
   std::array<int, kTuneLevels> m2l_mode{};  // per level: 0 static, 1 box mode, 2 clustered mode
@@ -117,7 +123,7 @@ class DeviceOperator {
   void set_p2p_uniform_min(int n) { opt_.tuning.p2p_uniform_min = n; }
   // the bf16x3 M2L's pipeline stage shape (Tuning::m2l_stage), from the next launch
   void set_m2l_stage(int stage) { opt_.tuning.m2l_stage = stage; }
-  int p2p_uniform_min() const { return opt_.tuning.p2p_uniform_min > 0 ? opt_.tuning.p2p_uniform_min : 33; }
+  int p2p_uniform_min() const { return opt_.tuning.p2p_uniform_min > 0 ? opt_.tuning.p2p_uniform_min : kP2pUniformMin; }
   // the M2L mode each level's schedule took: 0 none or by reflection classes, 1 box mode,
   // 2 clustered mode
   int m2l_mode_of(int level) const { return level >= 0 && level < kTuneLevels ? m2l_mode_taken_[level] : 0; }

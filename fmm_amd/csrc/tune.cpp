@@ -6,9 +6,10 @@
 // the GEMM of each translation kind per pair bucket and the P2P layout per
 // points-per-leaf bucket on the Fmm's own levels, keeps the winners in a cache file and
 // falls back to a static rule where nothing was tuned.  This tuner takes the decisions of
-// this path's kernels (the static rule's candidate first, so a cut budget keeps it):
+// this path's kernels (the first candidate is kept by a cut budget):
 //   - P2P (mixed precision): the chunk size from which targets read their sources by
-//     uniform loads instead of LDS tiles with phases: 33 (static), 17, 49, 65, never;
+//     uniform loads instead of LDS tiles with phases: 33, 17, 49, 65, never (the static
+//     43 chooses as 33 or as 49 for every leaf but those of 33 to 48);
 //   - M2L per level: box mode (tiles of 128 targets of one octant walking their offsets)
 //     or clustered mode (scratch rows per target and parent-level neighbour), and where the
 //     static rule takes the reflection classes, those (decision 0) or clustered mode;

@@ -10,7 +10,7 @@ boxes (L2L), the child level's boxes (M2M into the level), and the mean points p
 static rule applies (0 in the tuning).
 
 Decisions (the static rule's candidate is timed first and wins ties):
-  p2p  the mixed P2P's uniform-source threshold: 33 (static), 17, 49, 65, 129 (never)
+  p2p  the mixed P2P's uniform-source threshold: 33, 17, 49, 65, 129 (never); untuned 43
   m2l  per level: box mode (1) or clustered mode (2)
   l2l  per level: 16, 64 or 128 columns per task
   m2m  per parent level: per-tile form (1) or split form (2)
