@@ -254,8 +254,8 @@ __global__ void k_vjp_combine(size_t n, const double *q, const double *g, const 
 // (c'' = (C_t - C_s) / r_s, rho = r_t / r_s), and rounded to the same fixed point: in a
 // 2:1-balanced tree a near leaf (U list, or W/X pairs moved to P2P by the near rule) has
 // |x'| <= 1 + 2 rho + 2 <= 7 per axis, so |x' 2^28| < 2^31 and the separation
-// d' = x' - u_s is one exact integer subtraction per axis, then one conversion to f32
-// (relative rounding 2^-24).  The coordinates' quantisation, 2^-29 source-leaf units,
+// d' = x' - u_s, within 8 half-widths (less one unit, p2p_fixed), is one exact integer
+// subtraction per axis, then one conversion to f32 (relative rounding 2^-24).  The coordinates' quantisation, 2^-29 source-leaf units,
 // bounds the error of a pair at 2^-29 / |d'| relative: below 1e-7 from |d'| = 2^-4.5
 // half-widths on; a closer pair (r^2 under 2^47 integer units, rare: one in ~10^6 pairs
 // of a uniform leaf) forms d' again from the f64 coordinates, x' - u_s, scaled and
@@ -265,6 +265,15 @@ __global__ void k_vjp_combine(size_t n, const double *q, const double *g, const 
 // since q / |d| = rho q / |d'| and q d / |d|^3 = rho^2 q d' / |d'|^3 in target units.
 // Off the own leaf r^2 starts from 1/4 (integer units) in the quantised form and from the
 // smallest normal float in the f64 form: distinct points keep a finite r^2.
+// A position up to 7 half-widths out, seen from the other leaf of a near pair, in the fixed
+// point.  One unit is kept from the ends: 7 half-widths against a coordinate of 1 on the other
+// side would be 2^31, past an int32.
+__device__ __forceinline__ int p2p_fixed(double u) {
+  constexpr int kReach = 7 * (1 << 28) - 1;
+  const int v = __double2int_rn(u * kP2pFixed);
+  return v > kReach ? kReach : v < -kReach ? -kReach : v;
+}
+
 template <bool GRAD, bool TWO>
 __device__ __forceinline__ void p2p_uniform(uint32_t lf, uint32_t tb, uint32_t n, uint32_t e0, uint32_t e1,
                                             const uint32_t *__restrict__ near_ent,
@@ -303,7 +312,7 @@ __device__ __forceinline__ void p2p_uniform(uint32_t lf, uint32_t tb, uint32_t n
 #pragma unroll
     for (int a = 0; a < A; ++a)
 #pragma unroll
-      for (int k = 0; k < 3; ++k) xi[a][k] = __double2int_rn(fma(rho, u[a][k], c[k]) * kP2pFixed);
+      for (int k = 0; k < 3; ++k) xi[a][k] = p2p_fixed(fma(rho, u[a][k], c[k]));
     const bool own = sl == lf;
     // entries flagged at build (a pair of the entry closer than the threshold) and the
     // own leaf test their pairs; the others run the separations unchecked
@@ -577,8 +586,7 @@ __device__ __forceinline__ void p2p_staged(P2pStage<T> &sh, uint32_t lf, uint32_
       }
       V4 v;
       if constexpr (FIXED) {
-        v = make_int4(__double2int_rn(yx * kP2pFixed), __double2int_rn(yy * kP2pFixed),
-                      __double2int_rn(yz * kP2pFixed), __float_as_int(float(q)));
+        v = make_int4(p2p_fixed(yx), p2p_fixed(yy), p2p_fixed(yz), __float_as_int(float(q)));
         sh.yd[lane][0] = yx;
         sh.yd[lane][1] = yy;
         sh.yd[lane][2] = yz;
@@ -1411,9 +1419,9 @@ __global__ __launch_bounds__(64) void k_p2p_close_flags(uint32_t count, const ui
     for (uint32_t tb = t0; tb < t1; tb += 64) {
       const uint32_t i = tb + uint32_t(lane);
       if (i >= t1) break;
-      const int xi0 = __double2int_rn(fma(rho, tx[i], c[0]) * kP2pFixed);
-      const int xi1 = __double2int_rn(fma(rho, ty[i], c[1]) * kP2pFixed);
-      const int xi2 = __double2int_rn(fma(rho, tz[i], c[2]) * kP2pFixed);
+      const int xi0 = p2p_fixed(fma(rho, tx[i], c[0]));
+      const int xi1 = p2p_fixed(fma(rho, ty[i], c[1]));
+      const int xi2 = p2p_fixed(fma(rho, tz[i], c[2]));
       for (uint32_t j = s0; j < s1; ++j) {
         const int4 h = rec[j];
         const float dx = float(xi0 - h.x), dy = float(xi1 - h.y), dz = float(xi2 - h.z);

@@ -193,3 +193,55 @@ def test_mixed_near_field_of_close_pairs(leaf, scale):
             worst = max(worst, e.max(initial=0.0), g.max(initial=0.0))
     _log(f"  worst error over its bound {worst:.2f}")
     assert worst < 1.0
+
+
+def _near_field(plan, q, precision, gradients=True):
+    op = fmm_amd.Operator(plan, 3, precision, gradients, 0)
+    op.load_charges(q)
+    op.reset()
+    for level in range(plan.nlevels):
+        op.call("p2p", level)
+    return op.read_output()
+
+
+def _eight_half_widths_apart(coarse, fine, mirror):
+    """Points whose first two are 8 half-widths of the finer one's leaf apart in x, each at the
+    outer face of its leaf to 2^-36 of the domain: A in a leaf of `coarse` points, B in one half
+    its size with `fine` points, two cells further."""
+    corners = np.array([[0.0, 0.0, 0.0], [1.0, 1.0, 1.0]])
+    box, side = fmm_amd.Plan(corners, leaf_points=1).domain()
+    rng = O.Rng(64)
+    a = np.vstack([[0.25 + 2.0**-36, 0.3, 0.3], 0.26 + 0.22 * rng.cube(coarse - 1)])
+    b = np.vstack([[0.75 - 2.0**-36, 0.3, 0.3], [0.63, 0.26, 0.26] + 0.11 * rng.cube(fine - 1)])
+    rest = [0.51, 0.26, 0.26] + 0.22 * rng.cube(400)
+    rest = rest[~((rest[:, 0] > 0.62) & (rest[:, 1] < 0.38) & (rest[:, 2] < 0.38))]
+    pts = np.vstack([box[:3] + side * np.vstack([a[:1], b[:1], a[1:], b[1:], rest]), corners])
+    if mirror:
+        pts[:, 0] = (box[0] + box[3]) - pts[:, 0]
+    return pts
+
+
+@pytest.mark.parametrize("mirror", [False, True])
+@pytest.mark.parametrize("coarse,fine", [(3, 4), (30, 30), (50, 50), (3, 50), (50, 4)])
+def test_mixed_near_field_at_eight_half_widths(coarse, fine, mirror):
+    """The largest separation of a near pair, 8 half-widths (W and X entries moved to the near
+    rows, both points on the outer faces of their leaves), is one unit past an int32 in the
+    fixed point: the force of the pair alone, in both forms and both directions."""
+    _log(f"case mixed eight half-widths coarse={coarse} fine={fine} mirror={mirror}")
+    pts = _eight_half_widths_apart(coarse, fine, mirror)
+    plan = fmm_amd.Plan(pts, leaf_points=64, near_rule=(300, 300))
+    leaves, cells = plan.point_leaves().astype(int), plan.leaf_cells().astype(int)
+    u, order = plan.leaf_coordinates()
+    at = np.argsort(order)
+    la, lb = leaves[0], leaves[1]
+    assert cells[la][0] + 1 == cells[lb][0]
+    assert (leaves == la).sum() == coarse and (leaves == lb).sum() == fine
+    assert abs(u[at[0], 0] - u[at[1], 0]) == pytest.approx(2.0, abs=2.0**-28)
+    for source, target in ((0, 1), (1, 0)):
+        q = np.zeros(len(pts))
+        q[source] = 1.0
+        mixed, f64 = _near_field(plan, q, "mixed"), _near_field(plan, q, "f64")
+        assert f64.potential[target] > 0  # a near pair
+        assert abs(mixed.potential[target] / f64.potential[target] - 1) < 1e-6
+        size = np.linalg.norm(f64.gradient[target])
+        assert np.abs(mixed.gradient[target] - f64.gradient[target]).max() < 1e-6 * size
