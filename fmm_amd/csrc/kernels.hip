@@ -491,7 +491,9 @@ __device__ __forceinline__ void p2p_staged(P2pStage<T> &sh, uint32_t lf, uint32_
     ap[a] = ax[a] = ay[a] = az[a] = T(0);
   }
   // f32 sums are per tile (at most 64 terms) and go into f64 after each tile,
-  // so long near rows do not lose digits to one growing f32 sum
+  // so long near rows do not lose digits to one growing f32 sum; `unit` is what the tile's sums
+  // of charges are counted in
+  double unit = 1.0;
   double cp[A], cx[A], cy[A], cz[A];
 #pragma unroll
   for (int a = 0; a < A; ++a) cp[a] = cx[a] = cy[a] = cz[a] = 0.0;
@@ -499,10 +501,10 @@ __device__ __forceinline__ void p2p_staged(P2pStage<T> &sh, uint32_t lf, uint32_
     if (FIXED) {
 #pragma unroll
       for (int a = 0; a < A; ++a) {
-        cp[a] = fma(double(ap[a]), GRAD ? 1.0 : kP2pFixed, cp[a]);
-        cx[a] = fma(double(ax[a]), 1.0 / kP2pFixed, cx[a]);
-        cy[a] = fma(double(ay[a]), 1.0 / kP2pFixed, cy[a]);
-        cz[a] = fma(double(az[a]), 1.0 / kP2pFixed, cz[a]);
+        cp[a] = fma(double(ap[a]), unit, cp[a]);
+        cx[a] = fma(double(ax[a]), unit / kP2pFixed, cx[a]);
+        cy[a] = fma(double(ay[a]), unit / kP2pFixed, cy[a]);
+        cz[a] = fma(double(az[a]), unit / kP2pFixed, cz[a]);
         ap[a] = ax[a] = ay[a] = az[a] = T(0);
       }
     }
@@ -563,7 +565,7 @@ __device__ __forceinline__ void p2p_staged(P2pStage<T> &sh, uint32_t lf, uint32_
           inv = r2[k][a] == T(0) ? T(0) : rsqrt_t<T>(r2[k][a]);
         else
           inv = rsqrt_t<T>(r2[k][a]);
-        // (1 / r in leaf units, so that q / r^3 keeps the f32 range of the charges)
+        // (1 / r in leaf units, so that q / r^3 stays in range for small charges)
         if (FIXED && GRAD) inv *= T(kP2pFixed);
         const T qi = q[k] * inv;
         ap[a] += qi;
@@ -578,6 +580,17 @@ __device__ __forceinline__ void p2p_staged(P2pStage<T> &sh, uint32_t lf, uint32_
   // stage one tile: lane < cnt holds the source (x, y, z, q) in the target frame;
   // lanes cnt .. steps * phases - 1 hold zero charges far away
   auto stage = [&](int cnt, int steps, bool valid, double yx, double yy, double yz, double q) {
+    // The f32 terms carry powers of two: with gradients the force's separation is in units of
+    // 2^-28, and without them 1/r is in units of 2^28, which the charge takes up.  A tile with a
+    // charge beyond 2^38 counts in larger units, so that neither leaves f32 where the plain
+    // q / r^3 and q / r would not; what a small charge of such a tile loses is far below the
+    // rounding of the large one's term (at most 8 sqrt 3 half-widths away).
+    double per_unit = 1.0;
+    if constexpr (FIXED) {
+      const bool large = __any(valid && fabs(q) > 0x1p38);
+      unit = large ? (GRAD ? 0x1p30 : kP2pFixed) : 1.0;
+      per_unit = large ? (GRAD ? 0x1p-30 : 1.0) : (GRAD ? 1.0 : kP2pFixed);
+    }
     __syncthreads();
     if (lane < steps * phases) {
       if (!(valid && lane < cnt)) {
@@ -586,7 +599,8 @@ __device__ __forceinline__ void p2p_staged(P2pStage<T> &sh, uint32_t lf, uint32_
       }
       V4 v;
       if constexpr (FIXED) {
-        v = make_int4(p2p_fixed(yx), p2p_fixed(yy), p2p_fixed(yz), __float_as_int(float(q)));
+        v = make_int4(p2p_fixed(yx), p2p_fixed(yy), p2p_fixed(yz),
+                      __float_as_int(float(q * per_unit)));
         sh.yd[lane][0] = yx;
         sh.yd[lane][1] = yy;
         sh.yd[lane][2] = yz;

@@ -204,6 +204,43 @@ def _near_field(plan, q, precision, gradients=True):
     return op.read_output()
 
 
+def _near_error(plan, pts, q, out):
+    """The largest error of potential and gradient over a bound of the mixed near field.  Each
+    f32 operation of a pair's term and of its tile's sum is within 2^-24, and a separation on
+    each axis within 2^-28 half-widths from 2^-4.5 on: 1e-6 of the summed magnitudes.  The f64
+    positions carry two roundings of 2^-53 of the domain each, 2^(level - 51) half-widths, so both
+    of a pair at distance d on three axes move its potential by up to 2^(level - 49) / d of it
+    and its force by three times that."""
+    leaves, cells = plan.point_leaves().astype(int), plan.leaf_cells()
+    counts = np.concatenate([[0], np.cumsum(np.bincount(cells[:, 0], minlength=plan.nlevels))])
+    side = plan.domain()[1]
+    order = np.argsort(leaves, kind="stable")
+    start = np.searchsorted(leaves[order], np.arange(plan.nleaves + 1))
+    worst = 0.0
+    for level in range(plan.nlevels):
+        off, ent = plan.list("near", level)
+        half = 0.5 * side / 2.0 ** level
+        for r in range(len(off) - 1):
+            leaf = counts[level] + r
+            t = order[start[leaf]:start[leaf + 1]]
+            s = np.concatenate([order[start[e]:start[e + 1]] for e in ent[off[r]:off[r + 1]]])
+            d = (pts[t][:, None] - pts[s][None]) / half
+            r2 = (d * d).sum(-1)
+            with np.errstate(divide="ignore"):
+                inv = np.where(r2 == 0, 0.0, 1 / np.sqrt(r2))
+            tol = 1e-6 + 2.0 ** (level - 49) * inv
+            terms = q[s] * inv
+            e = np.abs(out.potential[t] * (4 * np.pi * half) - terms.sum(1)) / ((np.abs(terms) * tol).sum(1) + 1e-60)
+            worst = max(worst, e.max(initial=0.0))
+            if out.gradient is None:
+                continue
+            force = -(q[s] * inv**3)[..., None] * d
+            size = (np.sqrt((force * force).sum(-1)) * 3 * tol).sum(1) + 1e-60
+            g = np.abs(out.gradient[t] * (4 * np.pi * half**2) - force.sum(1)).max(-1) / size
+            worst = max(worst, g.max(initial=0.0))
+    return worst
+
+
 def _eight_half_widths_apart(coarse, fine, mirror):
     """Points whose first two are 8 half-widths of the finer one's leaf apart in x, each at the
     outer face of its leaf to 2^-36 of the domain: A in a leaf of `coarse` points, B in one half
@@ -245,3 +282,17 @@ def test_mixed_near_field_at_eight_half_widths(coarse, fine, mirror):
         assert abs(mixed.potential[target] / f64.potential[target] - 1) < 1e-6
         size = np.linalg.norm(f64.gradient[target])
         assert np.abs(mixed.gradient[target] - f64.gradient[target]).max() < 1e-6 * size
+
+
+@pytest.mark.parametrize("leaf", [1, 9, 20, 42])
+@pytest.mark.parametrize("scale,gradients", [(1e30, True), (1e-34, True), (1e30, False), (1e-34, False)])
+def test_mixed_near_field_charge_range(leaf, scale, gradients):
+    """The staged form over the f32 range of the charges (and of q / r^3 in leaf units)."""
+    _log(f"case mixed charge range leaf={leaf} scale={scale} gradients={gradients}")
+    rng = O.Rng(65)
+    pts = (np.stack(np.meshgrid(*[np.arange(12.0)] * 3), -1).reshape(-1, 3) + 0.5 * rng.cube(12**3)) / 12
+    q = rng.normals(len(pts)) * scale
+    plan = fmm_amd.Plan(pts, leaf_points=leaf)
+    worst = _near_error(plan, pts, q, _near_field(plan, q, "mixed", gradients))
+    _log(f"  worst error over its bound {worst:.2f}")
+    assert worst < 1.0
