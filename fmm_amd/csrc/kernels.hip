@@ -225,12 +225,15 @@ __global__ void k_vjp_combine(size_t n, const double *q, const double *g, const 
 // HBM; a staged source's position in the target leaf's frame and the targets' are rounded to
 // 32-bit fixed point (u 2^28; a near pair is within 7 half-widths in either frame, checked at
 // build), so the separation is one exact integer subtraction and one conversion per axis,
-// accurate to 2^-29 half-widths; a pair closer than 2^-4.5 half-widths takes its separation
-// from the f64 positions instead, so every pair keeps about 2^-24 of |d|.  r^2, the inverse
-// square root and the sums of a tile (at most 64 sources) are f32; the tile sums are added
-// in f64.  Coincident points give d = 0 exactly in both forms.  (VALU bound: the fixed point
-// takes the place of a split into hi + lo floats, 6 operations a pair less, and one LDS read
-// a source less; 1M points, p = 8: 689 -> 603 us.)
+// accurate to 2^-28 half-widths (each end is rounded by up to half a unit); a pair closer than
+// 2^-4.5 half-widths takes its separation from the f64 positions instead, so every pair keeps
+// 2^-23.5 of |d| or better.  r^2, the inverse square root and the sums of a tile (at most 64
+// sources) are f32; the tile sums are added in f64.  (Errors against f64 over 8 distributions
+// and leaves of 8 to 64: potential 5.5e-9 to 1.1e-8 rms of the summed magnitudes and force 1.1e-7
+// to 1.2e-7 in the median, with hi + lo floats 6.5e-9 to 1.2e-8 and 1.1e-7 to 1.3e-7.)
+// Coincident points give d = 0 exactly in both forms.  (VALU bound: the fixed point takes the
+// place of a split into hi + lo floats, 6 operations a pair less, and one LDS read a source
+// less; 1M points, p = 8: 689 -> 603 us.)
 
 // Lane mapping (one wave per target leaf, targets processed in chunks of 128): the staged
 // form puts one or two targets in each lane (the fuller use of the lanes), np lanes per
@@ -255,9 +258,9 @@ __global__ void k_vjp_combine(size_t n, const double *q, const double *g, const 
 // 2:1-balanced tree a near leaf (U list, or W/X pairs moved to P2P by the near rule) has
 // |x'| <= 1 + 2 rho + 2 <= 7 per axis, so |x' 2^28| < 2^31 and the separation
 // d' = x' - u_s, within 8 half-widths (less one unit, p2p_fixed), is one exact integer
-// subtraction per axis, then one conversion to f32 (relative rounding 2^-24).  The coordinates' quantisation, 2^-29 source-leaf units,
-// bounds the error of a pair at 2^-29 / |d'| relative: below 1e-7 from |d'| = 2^-4.5
-// half-widths on; a closer pair (r^2 under 2^47 integer units, rare: one in ~10^6 pairs
+// subtraction per axis, then one conversion to f32 (relative rounding 2^-24).  The
+// coordinates' quantisation, 2^-29 source-leaf units at either end, bounds the error of a
+// pair at 2^-28 / |d'| per axis: 2^-23.5 from |d'| = 2^-4.5 half-widths on; a closer pair (r^2 under 2^47 integer units, rare: one in ~10^6 pairs
 // of a uniform leaf) forms d' again from the f64 coordinates, x' - u_s, scaled and
 // rounded once, so close pairs keep 2^-24 of |d'| as in the double-float form.
 // In integer units r^2 = |d'|^2 2^56: the f32 sums of an entry (at most 128 sources) are

@@ -67,8 +67,8 @@ void clear(hipStream_t s, const ClearList &c);  // zeros into p[k][0 .. n[k])
 void gather_charges(hipStream_t s, const double *q, const uint32_t *order, size_t n, double *q64, float *rec);
 // Fixed-point scale of the mixed P2P's source records: 2^28 per leaf half-width.
 constexpr double kP2pFixed = 268435456.0;
-// r^2 (integer units) below which a pair's quantised separation would cost more than 1e-7
-// of its terms (|d| < 2^23.5 units, 0.044 half-widths): 2^47
+// r^2 (integer units) below which a pair's quantised separation would cost more than 2^-23.5
+// of it on an axis (|d| < 2^23.5 units, 0.044 half-widths): 2^47
 constexpr float kP2pClose = 140737488355328.0f;
 // Mixed-precision P2P source records, 4 words per source in leaf order: the source's
 // own-leaf coordinates u (|u| <= 1) as round(u 2^28) in int32, then the charge's f32

@@ -147,54 +147,6 @@ def test_host_downloads_of_every_size():
     assert out == {n: True for n in sizes}
 
 
-@pytest.mark.parametrize("leaf,scale", [(2, 1.0), (9, 1e-25), (32, 1.0), (43, 1.0), (70, 1.0)])
-def test_mixed_near_field_of_close_pairs(leaf, scale):
-    """The mixed near field alone (fixed-point separations, close pairs from f64) at chunks
-    below and above the uniform form's threshold: coincident points, pairs 1e-2 to 1e-12 apart
-    inside a leaf and across the faces of boxes, charges over the f32 range.  Each f32
-    operation of a pair's term and of its tile's sum is within 2^-24: 1e-6 of the summed
-    magnitudes at every target, and the f64 positions in leaf units carry 2^-53 each, which a
-    pair d apart feels as 2^-51 / d of its term (three times that in its force)."""
-    _log(f"case mixed close pairs leaf={leaf} scale={scale}")
-    rng = O.Rng(63)
-    base = rng.cube(2400)
-    gaps = 10.0 ** -np.linspace(2, 12, 300)[:, None]
-    faces = np.round(rng.cube(200) * 8) / 8 * 0.998 + 0.001
-    pts = np.vstack([base, base[:100], base[300:600] + gaps * (rng.cube(300) - 0.5), faces,
-                     faces + 1e-9 * (rng.cube(200) - 0.5), [[0.0, 0.0, 0.0], [1.0, 1.0, 1.0]]])
-    pts = np.clip(pts, 0.0, 1.0)
-    q = rng.normals(len(pts)) * scale
-    fmm = fmm_amd.FmmBuilder(3).precision("mixed").max_points_per_leaf(leaf).build(pts)
-    op = fmm.operator
-    op.load_charges(q)
-    op.reset()
-    plan = fmm.plan
-    for level in range(plan.nlevels):
-        op.call("p2p", level)
-    out = op.read_output()
-    leaves = plan.point_leaves().astype(int)
-    levels = (plan.leaf_keys() & np.uint64(0x7FFF)).astype(int)
-    offsets = np.concatenate([[0], np.cumsum(np.bincount(levels, minlength=plan.nlevels))])
-    worst = 0.0
-    for level in range(plan.nlevels):
-        off, ent = plan.list("near", level)
-        for r in range(len(off) - 1):
-            t = np.flatnonzero(leaves == offsets[level] + r)
-            s = np.flatnonzero(np.isin(leaves, ent[off[r]:off[r + 1]]))
-            d = pts[t][:, None] - pts[s][None]
-            r2 = (d * d).sum(-1)
-            with np.errstate(divide="ignore"):
-                inv = np.where(r2 == 0, 0.0, 1 / np.sqrt(r2)) / (4 * np.pi) ** (1 / 3)
-            c = (4 * np.pi) ** (-2 / 3)
-            terms = q[s] * inv * c
-            force = -(q[s] * inv**3)[..., None] * d
-            e = np.abs(out.potential[t] - terms.sum(1)) / (np.abs(terms).sum(1) + 1e-300)
-            g = np.abs(out.gradient[t] - force.sum(1)).max(-1) / (np.abs(force).max(-1).sum(1) + 1e-300)
-            worst = max(worst, e.max(initial=0.0), g.max(initial=0.0))
-    _log(f"  worst error over its bound {worst:.2f}")
-    assert worst < 1.0
-
-
 def _near_field(plan, q, precision, gradients=True):
     op = fmm_amd.Operator(plan, 3, precision, gradients, 0)
     op.load_charges(q)
@@ -239,6 +191,27 @@ def _near_error(plan, pts, q, out):
             g = np.abs(out.gradient[t] * (4 * np.pi * half**2) - force.sum(1)).max(-1) / size
             worst = max(worst, g.max(initial=0.0))
     return worst
+
+
+@pytest.mark.parametrize("gradients", [True, False])
+@pytest.mark.parametrize("leaf,scale", [(2, 1.0), (9, 1e-25), (32, 1.0), (43, 1.0), (70, 1.0)])
+def test_mixed_near_field_of_close_pairs(leaf, scale, gradients):
+    """The mixed near field alone (fixed-point separations, close pairs from f64) at chunks
+    below and above the uniform form's threshold: coincident points, pairs 1e-2 to 1e-12 apart
+    inside a leaf and across the faces of boxes."""
+    _log(f"case mixed close pairs leaf={leaf} scale={scale} gradients={gradients}")
+    rng = O.Rng(63)
+    base = rng.cube(2400)
+    gaps = 10.0 ** -np.linspace(2, 12, 300)[:, None]
+    faces = np.round(rng.cube(200) * 8) / 8 * 0.998 + 0.001
+    pts = np.vstack([base, base[:100], base[300:600] + gaps * (rng.cube(300) - 0.5), faces,
+                     faces + 1e-9 * (rng.cube(200) - 0.5), [[0.0, 0.0, 0.0], [1.0, 1.0, 1.0]]])
+    pts = np.clip(pts, 0.0, 1.0)
+    q = rng.normals(len(pts)) * scale
+    plan = fmm_amd.Plan(pts, leaf_points=leaf)
+    worst = _near_error(plan, pts, q, _near_field(plan, q, "mixed", gradients))
+    _log(f"  worst error over its bound {worst:.2f}")
+    assert worst < 1.0
 
 
 def _eight_half_widths_apart(coarse, fine, mirror):
