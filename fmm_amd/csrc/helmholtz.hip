@@ -21,6 +21,7 @@
 
 #include "hkernels.hpp"
 #include "kernels.hpp"
+#include "sincos.hpp"
 
 namespace fmmh {
 namespace dev {
@@ -554,9 +555,9 @@ __global__ __launch_bounds__(SING ? 64 * kRowWaves : 64) void k_h_evaluate(int p
 // (selects, no branch).  T = float: separations from double-float coordinates (hi + lo), the
 // pair arithmetic in f32, each source leaf's f32 sums added to f64 accumulators.
 // Pair kernel pieces per precision.  f64: 1/r by v_rsq_f64 and a third-order step, r = r^2 /
-// r corrected once, sine and cosine as below (300 cycles per 64 pairs against 830 with the
-// math library's sqrt, division and sincos, whose reductions for huge arguments it carries
-// along).  f32: 1/r from v_rsq_f32 (1 ulp) and r = r^2 / r; sine and cosine from v_sin_f32
+// r corrected once (the bits of sqrt; 1/r within 0.99 ulp, rms 5.2e-17, where 1 / sqrt rounds
+// twice: 1.49 and 6.7e-17), sine and cosine by sincos_f64 (about 345 cycles per 64 pairs against 830
+// with the math library's, whose reductions for huge arguments they carry along).  f32: 1/r from v_rsq_f32 (1 ulp) and r = r^2 / r; sine and cosine from v_sin_f32
 // and v_cos_f32 of the fraction of x / (2 pi).
 template <typename T>
 struct PairMath;
@@ -571,32 +572,7 @@ struct PairMath<double> {
     r = r2 * ir;
     r = fma(0.5 * ir, fma(-r, r, r2), r);
   }
-  // x = n pi/2 + t, |t| <= pi/4, with pi/2 as the sum of two doubles (Cody and Waite); sine
-  // and cosine of t by polynomials in t^2 through the Chebyshev points of [0, (pi/4)^2]
-  // (errors 1.8e-17 and 9e-19, below the rounding); the quadrant selects and signs.  For
-  // |x| < 2^31, far beyond any k r of a leaf pair.
-  __device__ static __forceinline__ void sincos(double x, double *s, double *c) {
-    constexpr double kShift = 6755399441055744.0;  // 1.5 2^52: the sum's low bits are rint(x 2/pi)
-    const double m = fma(x, 0.6366197723675814, kShift), n = m - kShift;
-    const int q = __double2loint(m);
-    double t = fma(-n, 1.5707963267948966, x);
-    t = fma(-n, 6.123233995736766e-17, t);
-    const double z = t * t;
-    double ps = fma(z, 1.5918115263265974e-10, -2.505113165023518e-08);
-    ps = fma(z, ps, 2.7557316101617874e-06);
-    ps = fma(z, ps, -0.00019841269836756774);
-    ps = fma(z, ps, 0.008333333333330948);
-    ps = fma(z, ps, -0.16666666666666666);
-    double pc = fma(z, -1.1382623647474604e-11, 2.087614614655861e-09);
-    pc = fma(z, pc, -2.7557317271145144e-07);
-    pc = fma(z, pc, 2.480158729876456e-05);
-    pc = fma(z, pc, -0.0013888888888887398);
-    pc = fma(z, pc, 0.041666666666666664);
-    const double st = fma(t * z, ps, t), ct = fma(z * z, pc, fma(-0.5, z, 1.0));
-    const double sv = (q & 1) ? ct : st, cv = (q & 1) ? st : ct;
-    *s = __hiloint2double(__double2hiint(sv) ^ ((q << 30) & int(0x80000000)), __double2loint(sv));
-    *c = __hiloint2double(__double2hiint(cv) ^ (((q + 1) << 30) & int(0x80000000)), __double2loint(cv));
-  }
+  __device__ static __forceinline__ void sincos(double x, double *s, double *c) { sincos_f64(x, s, c); }
 };
 
 template <>
@@ -829,14 +805,13 @@ __device__ __forceinline__ void h_p2p_staged(HP2pStage<T> &sh, uint32_t lf, uint
             T sn, cs;
             PairMath<T>::sincos(kre * rr, &sn, &cs);
             const T dmp = DAMP ? T(exp(-kim * rr)) : T(1);
-            const T er = dmp * cs * ir, ei = dmp * sn * ir;
-            const T q0 = ys[i][6], q1 = ys[i][7];
-            loc[a][0] += q0 * er - q1 * ei;
-            loc[a][1] += q0 * ei + q1 * er;
+            const T q0 = ys[i][6], q1 = ys[i][7], es = DAMP ? dmp * ir : ir;
+            const T pr = (q0 * cs - q1 * sn) * es, pi = (q0 * sn + q1 * cs) * es;  // q e^{ikr} / r
+            loc[a][0] += pr;
+            loc[a][1] += pi;
             if (GRAD) {
               const T ar = DAMP ? -kim * rr - T(1) : T(-1), ai = kre * rr, ir2 = ir * ir;
-              const T gr = (ar * er - ai * ei) * ir2, gi = (ar * ei + ai * er) * ir2;
-              const T qgr = q0 * gr - q1 * gi, qgi = q0 * gi + q1 * gr;
+              const T qgr = (ar * pr - ai * pi) * ir2, qgi = (ar * pi + ai * pr) * ir2;
               loc[a][2] += qgr * dx;
               loc[a][3] += qgi * dx;
               loc[a][4] += qgr * dy;
