@@ -22,7 +22,7 @@ namespace {
 constexpr size_t kHalf = size_t(4) << 20;   // bytes per half
 constexpr size_t kSlice = size_t(128) << 10;  // bytes per host thread at least
 constexpr int kThreads = 16;
-constexpr size_t kKeep = 4;                 // idle buffers kept
+constexpr size_t kKeep = 8;                 // idle buffers kept (one for each GPU of a node)
 
 struct Stage {
   int device = 0;
@@ -40,7 +40,8 @@ void destroy(Stage &t) {
   if (t.buf) (void)hipHostFree(t.buf);
 }
 
-// An idle buffer of the device, or a new one; false when none can be had.
+// An idle buffer of the device, or a new one (the calling thread's current device must be it:
+// the events belong to that one); false when none can be had.
 bool take(int device, Stage &t) {
   {
     std::lock_guard<std::mutex> lock(g_mu);
@@ -75,6 +76,23 @@ void give(Stage &t) {
   destroy(t);
 }
 
+// The thread's current device is `device` while this lives.
+class OnDevice {
+ public:
+  explicit OnDevice(int device) {
+    hip_check(hipGetDevice(&before_), "hipGetDevice");
+    if (before_ != device) hip_check(hipSetDevice(device), "hipSetDevice");
+    moved_ = before_ != device;
+  }
+  ~OnDevice() {
+    if (moved_) (void)hipSetDevice(before_);
+  }
+
+ private:
+  int before_ = 0;
+  bool moved_ = false;
+};
+
 void host_copy(char *dst, const char *src, size_t bytes) {
   const int n = int(std::min<size_t>(size_t(std::min(kThreads, omp_get_max_threads())), bytes / kSlice));
   if (n <= 1) {
@@ -93,6 +111,7 @@ void host_copy(char *dst, const char *src, size_t bytes) {
 
 HostStageUser::HostStageUser() {
   std::lock_guard<std::mutex> lock(g_mu);
+  g_idle.reserve(kKeep);  // giving a buffer back cannot fail
   ++g_users;
 }
 
@@ -109,6 +128,14 @@ void HostStageUser::download(int device, hipStream_t s, const std::vector<HostCo
   size_t total = 0;
   for (const HostCopy &c : copies) total += c.bytes;
   if (total == 0) return;
+  const OnDevice on(device);
+  // chunks of a quarter of the whole, so that copying starts early, within the halves' size
+  const size_t most = std::min(kHalf, std::max<size_t>(size_t(256) << 10, (total / 4 + 4095) / 4096 * 4096));
+  std::vector<HostCopy> chunks;
+  for (const HostCopy &c : copies)
+    for (size_t at = 0; at < c.bytes; at += most)
+      chunks.push_back({static_cast<char *>(c.dst) + at, static_cast<const char *>(c.src) + at,
+                        std::min(most, c.bytes - at)});
   Stage t;
   // (a few kilobytes arrive sooner through the runtime's own staging)
   if (total < (size_t(64) << 10) || !take(device, t)) {
@@ -117,13 +144,6 @@ void HostStageUser::download(int device, hipStream_t s, const std::vector<HostCo
     hip_check(hipStreamSynchronize(s), "download");
     return;
   }
-  // chunks of a quarter of the whole, so that copying starts early, within the halves' size
-  const size_t most = std::min(kHalf, std::max<size_t>(size_t(256) << 10, (total / 4 + 4095) / 4096 * 4096));
-  std::vector<HostCopy> chunks;
-  for (const HostCopy &c : copies)
-    for (size_t at = 0; at < c.bytes; at += most)
-      chunks.push_back({static_cast<char *>(c.dst) + at, static_cast<const char *>(c.src) + at,
-                        std::min(most, c.bytes - at)});
   const auto send = [&](size_t i) {
     const HostCopy &c = chunks[i];
     const hipError_t e = hipMemcpyAsync(t.buf + (i & 1) * kHalf, c.src, c.bytes, hipMemcpyDeviceToHost, s);
