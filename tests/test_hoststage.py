@@ -28,6 +28,9 @@ void hip_check(hipError_t e, const char *what) {
 }  // namespace fmmh
 
 static thread_local int g_device = 0;
+static std::atomic<const void *> g_pinned{nullptr};
+static std::atomic<bool> g_refuse_unknown{false};
+static std::atomic<int> g_direct{0};
 static std::atomic<int> g_buffers{0}, g_events{0}, g_fail_after{1 << 30};
 struct Event { int device; };
 
@@ -51,8 +54,17 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p) {
+  if (p == g_pinned) {
+    a->type = hipMemoryTypeHost;
+    return hipSuccess;
+  }
+  a->type = hipMemoryTypeUnregistered;
+  return g_refuse_unknown ? hipErrorInvalidValue : hipSuccess;
+}
 hipError_t hipMemcpyAsync(void *dst, const void *src, size_t n, hipMemcpyKind, hipStream_t) {
   if (--g_fail_after < 0) return hipErrorUnknown;
+  if (dst == g_pinned) ++g_direct;
   std::memcpy(dst, src, n);
   return hipSuccess;
 }
@@ -113,6 +125,23 @@ int main() {
 }
 """
 
+PINNED = r"""
+int main() {
+  int bad = 0;
+  fmmh::HostStageUser user;
+  std::vector<char> a(3000000, 5), x(a.size());
+  g_pinned = x.data();
+  user.download(0, stream_of(0), {{x.data(), a.data(), a.size()}});
+  bad += check(a == x && g_direct == 1 && g_buffers == 0, "memory the runtime knows takes one copy");
+  g_pinned = nullptr;
+  for (bool refuse : {false, true}) {
+    g_refuse_unknown = refuse;
+    bad += check(round_trip(user, 0, 3000000) && g_buffers == 1, "other memory is staged");
+  }
+  return bad;
+}
+"""
+
 
 def _build(tmp_path, main):
     if shutil.which("g++") is None:
@@ -134,3 +163,7 @@ def _run(exe, **env):
 
 def test_downloads_of_several_devices(tmp_path):
     _run(_build(tmp_path, DEVICES))
+
+
+def test_downloads_into_pinned_memory(tmp_path):
+    _run(_build(tmp_path, PINNED))
