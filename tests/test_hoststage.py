@@ -142,6 +142,57 @@ int main() {
 }
 """
 
+THREADS = r"""
+#include <chrono>
+#include <condition_variable>
+#include <dirent.h>
+#include <mutex>
+static int threads() {
+  int n = 0;
+  DIR *d = opendir("/proc/self/task");
+  while (dirent *e = readdir(d)) n += e->d_name[0] != '.';
+  closedir(d);
+  return n;
+}
+int main() {
+  int bad = 0;
+  const int before = threads();
+  {
+    fmmh::HostStageUser user;
+    // callers that have downloaded and live on: at most four have kept threads of their own
+    std::mutex mu;
+    std::condition_variable cv;
+    bool stop = false;
+    int ready = 0;
+    std::atomic<int> wrong{0};
+    std::vector<std::thread> work;
+    for (int k = 0; k < 20; ++k)
+      work.emplace_back([&, k] {
+        for (size_t n : {3000000u, 100000u, 9000001u}) wrong += !round_trip(user, k & 1, n + k);
+        std::unique_lock<std::mutex> lock(mu);
+        ++ready;
+        cv.notify_all();
+        cv.wait(lock, [&] { return stop; });
+      });
+    {
+      std::unique_lock<std::mutex> lock(mu);
+      cv.wait(lock, [&] { return ready == 20; });
+      bad += check(threads() <= before + 20 + 4 * 7, "threads that stay");
+      stop = true;
+    }
+    cv.notify_all();
+    for (auto &t : work) t.join();
+    bad += check(wrong == 0, "many threads");
+  }
+  for (int k = 0; k < 200 && threads() > before; ++k) std::this_thread::sleep_for(std::chrono::milliseconds(10));
+  bad += check(threads() == before, "threads given back with the callers'");
+  // and others may have them now
+  fmmh::HostStageUser user;
+  bad += check(round_trip(user, 0, 9000001), "another user");
+  return bad;
+}
+"""
+
 
 def _build(tmp_path, main):
     if shutil.which("g++") is None:
@@ -167,3 +218,9 @@ def test_downloads_of_several_devices(tmp_path):
 
 def test_downloads_into_pinned_memory(tmp_path):
     _run(_build(tmp_path, PINNED))
+
+
+def test_copying_threads_are_bounded(tmp_path):
+    exe = _build(tmp_path, THREADS)
+    _run(exe, OMP_NUM_THREADS="8")
+    _run(exe, OMP_NUM_THREADS="1")
