@@ -48,6 +48,7 @@ EXPORTS = [
     "fmmh_helmholtz_plane_wave_merge",
     "fmmh_stream_wait", "fmmh_helmholtz_stream_wait",
     "fmmh_direct_sum_noalloc", "fmmh_operator_create_tuned", "fmmh_autotune", "fmmh_inject_error",
+    "fmmh_m2l_class_levels",
     "fmmh_set_table_cache", "fmmh_table_cache_stats",
 ]
 
@@ -174,6 +175,7 @@ def lib():
     L.fmmh_operator_create.argtypes = [vp, C.POINTER(OperatorOptions), C.POINTER(vp)]
     L.fmmh_operator_create_tuned.argtypes = [vp, C.POINTER(OperatorOptions), C.POINTER(Tuning), C.POINTER(vp)]
     L.fmmh_autotune.argtypes = [vp, C.POINTER(OperatorOptions), dbl, C.POINTER(Tuning), vp]
+    L.fmmh_m2l_class_levels.argtypes = [vp, C.POINTER(OperatorOptions), vp]
     L.fmmh_inject_error.argtypes = [vp]
     L.fmmh_operator_free.argtypes = [vp]
     L.fmmh_operator_free.restype = None

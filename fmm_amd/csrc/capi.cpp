@@ -576,6 +576,15 @@ int32_t fmmh_operator_create_tuned(const fmmh_plan *plan, const fmmh_operator_op
   });
 }
 
+int32_t fmmh_m2l_class_levels(const fmmh_plan *plan, const fmmh_operator_options *options, int32_t *out) {
+  return guard([&] {
+    need(plan && options && out, "fmmh_m2l_class_levels: NULL argument");
+    need(options->p >= 0 && options->p <= fmmh::dev::kMaxDegree, "fmmh_m2l_class_levels: 0 <= p <= 15");
+    const std::vector<char> levels = fmmh::m2l_class_levels(plan->plan, options_of(options, nullptr));
+    std::copy(levels.begin(), levels.end(), out);
+  });
+}
+
 void fmmh_operator_free(fmmh_operator *op) { delete op; }
 
 int32_t fmmh_autotune(const fmmh_plan *plan, const fmmh_operator_options *options, double budget_seconds,

@@ -21,6 +21,22 @@ void hip_check(hipError_t e, const char *what) {
   throw Error(s, std::string(what) + ": " + hipGetErrorString(e));
 }
 
+std::vector<char> m2l_class_levels(const Plan &plan, const OperatorOptions &options) {
+  std::vector<char> out(plan.nlevels, 0);
+  size_t nboxes = 0;
+  for (int l = 0; l < plan.nlevels; ++l) nboxes += plan.nboxes(l);
+  if (options.m2l != kM2lDense || !ReflectM2l::fits(options.p, options.precision == kMixed, nboxes)) return out;
+  std::vector<uint64_t> pairs(plan.nlevels, 0), boxes(plan.nlevels, 0);
+  for (int l = 2; l < plan.nlevels; ++l) {
+    pairs[l] = plan.v[l].size();
+    boxes[l] = plan.nboxes(l);
+  }
+  out = ReflectM2l::levels(options.p, pairs, boxes);
+  for (int l = 2; l < std::min(plan.nlevels, kTuneLevels); ++l)
+    if (options.tuning.m2l_mode[l] != 0) out[l] = 0;
+  return out;
+}
+
 DeviceOperator::DeviceOperator(const Plan &plan, const OperatorOptions &options) : opt_(options) {
   require(opt_.p >= 0 && opt_.p <= dev::kMaxDegree, "the device path supports 0 <= p <= 15", kUnsupportedLayout);
   require(opt_.precision == kPlainF64 || opt_.precision == kMixed, "unknown precision", kUnsupportedPrecision);
@@ -237,17 +253,7 @@ DeviceOperator::DeviceOperator(const Plan &plan, const OperatorOptions &options)
     }
     upload_rows(p2l_rows_, id, cell, off, ent);
   }
-  // the levels whose M2L runs by reflection classes
-  std::vector<char> reflected(nlevels_, 0);
-  if (opt_.m2l == kM2lDense && ReflectM2l::fits(opt_.p, opt_.precision == kMixed, nbox_total_)) {
-    std::vector<uint64_t> pairs(nlevels_, 0), boxes(nlevels_, 0);
-    for (int l = 2; l < nlevels_; ++l) {
-      if (l < kTuneLevels && opt_.tuning.m2l_mode[l] != 0) continue;
-      pairs[l] = plan.v[l].size();
-      boxes[l] = plan.nboxes(l);
-    }
-    reflected = ReflectM2l::levels(opt_.p, pairs, boxes);
-  }
+  const std::vector<char> reflected = m2l_class_levels(plan, opt_);
   build_schedules(plan, reflected);
   if (std::count(reflected.begin(), reflected.end(), char(1)) > 0) {
     reflect_.begin(opt_.p, opt_.precision == kMixed, std::vector<size_t>(box_base_.begin(), box_base_.end()), 1);

@@ -78,6 +78,10 @@ struct OperatorOptions {
   Tuning tuning;
 };
 
+// The levels whose dense M2L runs by reflection classes: the static rule's (ReflectM2l::levels), but
+// those that the tuning gives another mode.
+std::vector<char> m2l_class_levels(const Plan &plan, const OperatorOptions &options);
+
 class DeviceOperator {
  public:
   DeviceOperator(const Plan &plan, const OperatorOptions &options);

@@ -6,13 +6,15 @@
 // the GEMM of each translation kind per pair bucket and the P2P layout per
 // points-per-leaf bucket on the Fmm's own levels, keeps the winners in a cache file and
 // falls back to a static rule where nothing was tuned.  This tuner takes the decisions of
-// this path's kernels (the first candidate is kept by a cut budget):
+// this path's kernels (the static rule's candidate first, so a cut budget keeps it):
 //   - P2P (mixed precision): the chunk size from which targets read their sources by
-//     uniform loads instead of LDS tiles with phases: 33, 17, 49, 65, never (the static
-//     43 chooses as 33 or as 49 for every leaf but those of 33 to 48);
-//   - M2L per level: box mode (tiles of 128 targets of one octant walking their offsets)
-//     or clustered mode (scratch rows per target and parent-level neighbour), and where the
-//     static rule takes the reflection classes, those (decision 0) or clustered mode;
+//     uniform loads instead of LDS tiles with phases: 43 (static), 17, 33, 65, never;
+//   - M2L per level that does not run by reflection classes: box mode (tiles of 128 targets of
+//     one octant walking their offsets) or clustered mode (scratch rows per target and
+//     parent-level neighbour).  The levels by classes share one launch, and the small ones join it
+//     because alone they are slow, so a level's own time says nothing about them: they are not
+//     timed (4M points, p = 12: timed alone, levels 2 to 4 went to clustered mode, M2L 3.8 ms
+//     against 3.5);
 //   - L2L per level: 16, 64 or 128 columns per task;
 //   - M2M per parent level: the per-tile form or the split form;
 //   - the bf16x3 M2L's pipeline stage: one k-step per stage (ring of three) or two (ring
@@ -104,7 +106,7 @@ void autotune(const Plan &plan, const OperatorOptions &options, double budget_s,
 
   // P2P form (the mixed path only has two forms)
   if (options.precision == kMixed) {
-    const int cand[kTuneCandidates] = {33, 17, 49, 65, 129};
+    const int cand[kTuneCandidates] = {kP2pUniformMin, 17, 33, 65, 129};
     double best = std::numeric_limits<double>::infinity();
     for (int c = 0; c < kTuneCandidates; ++c) {
       A->set_p2p_uniform_min(cand[c]);
@@ -143,7 +145,7 @@ void autotune(const Plan &plan, const OperatorOptions &options, double budget_s,
   OperatorOptions ob = oa, oc = oa, od = oa;
   for (int l = 0; l < std::min(L, kTuneLevels); ++l) {
     const int m = A->m2l_mode_of(l);
-    ob.tuning.m2l_mode[l] = m == 1 || A->m2l_reflected(l) ? 2 : m == 2 ? 1 : 0;
+    ob.tuning.m2l_mode[l] = m == 1 ? 2 : m == 2 ? 1 : 0;
     ob.tuning.l2l_width[l] = 16;
     ob.tuning.m2m_form[l] = 1;
     oc.tuning.l2l_width[l] = 64;
@@ -159,7 +161,7 @@ void autotune(const Plan &plan, const OperatorOptions &options, double budget_s,
 
   for (int l = 0; l < std::min(L, kTuneLevels); ++l) {
     // M2L: the static mode (A) against the other (B)
-    if (options.m2l == kM2lDense && (ops[0]->m2l_mode_of(l) != 0 || ops[0]->m2l_reflected(l))) {
+    if (options.m2l == kM2lDense && ops[0]->m2l_mode_of(l) != 0) {
       double best = std::numeric_limits<double>::infinity();
       for (int k = 0; k < 2; ++k) {
         DeviceOperator &op = *ops[k];

@@ -11,7 +11,8 @@ constexpr int kTuneCandidates = 5;  // at most per decision
 enum TuneKind : int { kTuneP2p = 0, kTuneM2l = 1, kTuneL2l = 2, kTuneM2m = 3, kTuneStage = 4 };
 
 // ms per call of every candidate timed, NaN where not timed: [kind][level][candidate]
-// (P2P: level 0, candidates 33, 17, 49, 65, never; M2L: the static mode, the other; L2L:
+// (P2P: level 0, candidates 43 (the static rule's), 17, 33, 65, never; M2L: the static mode, the
+// other, on the levels that do not run by reflection classes; L2L:
 // the static width, 16, 64, 128; M2M: static, per-tile, split; M2L stage: level 0, one
 // k-step per stage, two k-steps in a ring of two).
 struct TuneReport {

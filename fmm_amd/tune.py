@@ -10,8 +10,9 @@ boxes (L2L), the child level's boxes (M2M into the level), and the mean points p
 static rule applies (0 in the tuning).
 
 Decisions (the static rule's candidate is timed first and wins ties):
-  p2p  the mixed P2P's uniform-source threshold: 33, 17, 49, 65, 129 (never); untuned 43
-  m2l  per level: box mode (1) or clustered mode (2)
+  p2p  the mixed P2P's uniform-source threshold: 43 (static), 17, 33, 65, 129 (never)
+  m2l  per level that the static rule does not run by reflection classes: box mode (1) or
+       clustered mode (2)
   l2l  per level: 16, 64 or 128 columns per task
   m2m  per parent level: per-tile form (1) or split form (2)
   stage the mixed dense M2L's pipeline: one k-step per stage (0) or two in a ring of two
@@ -34,9 +35,9 @@ from . import _lib
 
 CACHE_NAME = "fmm_amd_tuning.json"
 # bump when a candidate set or a decision's meaning changes: older files are ignored
-CANDIDATE_SET_VERSION = 2
+CANDIDATE_SET_VERSION = 3
 KINDS = ("p2p", "m2l", "l2l", "m2m", "stage")
-P2P_CANDIDATES = (33, 17, 49, 65, 129)
+P2P_CANDIDATES = (43, 17, 33, 65, 129)  # the static rule's first
 
 
 def bucket(n: float) -> int:
@@ -57,8 +58,19 @@ def cache_key(p, precision, gradients, m2l, device=0) -> str:
     return f"{device_name(device)}|p{int(p)}|{precision}|g{int(bool(gradients))}|{m2l}"
 
 
-def level_buckets(plan) -> dict:
-    """The bucket of every decision of this plan: {kind: {level: bucket}}."""
+def m2l_class_levels(plan, p, precision, m2l="dense") -> list:
+    """The levels whose dense M2L the static rule runs by reflection classes."""
+    from . import M2L_METHODS, PRECISIONS
+
+    o = _lib.OperatorOptions(int(p), PRECISIONS[precision], 1, 0, M2L_METHODS[m2l])
+    out = np.zeros(max(plan.nlevels, 1), np.int32)
+    _lib.check(_lib.lib().fmmh_m2l_class_levels(plan.handle, C.byref(o), _lib.ptr(out)))
+    return [l for l in range(plan.nlevels) if out[l]]
+
+
+def level_buckets(plan, classes=()) -> dict:
+    """The bucket of every decision of this plan: {kind: {level: bucket}}; no M2L decision on the
+    levels `classes`."""
     L = plan.nlevels
     boxes = [len(plan.box_keys(l)) for l in range(L)]
     out = {"m2l": {}, "l2l": {}, "m2m": {}, "p2p": {}, "stage": {}}
@@ -66,7 +78,7 @@ def level_buckets(plan) -> dict:
     for l in range(2, L):
         npairs = len(plan.list("v", l)[1])
         total += npairs
-        if npairs:
+        if npairs and l not in classes:
             out["m2l"][l] = bucket(npairs)
     if total:
         out["stage"][0] = bucket(total)
@@ -170,7 +182,7 @@ def resolve(plan, p, precision, gradients, device, m2l, directory, budget):
     ones tuned within `budget` seconds and stored.  Returns (tuning, info)."""
     cache = TuningCache(directory)
     key = cache_key(p, precision, gradients, m2l, device)
-    buckets = level_buckets(plan)
+    buckets = level_buckets(plan, m2l_class_levels(plan, p, precision, m2l))
     t, missing = cache.lookup(key, buckets, precision)
     info = {"key": key, "cached": not missing, "tuned_s": 0.0}
     if missing and budget > 0:

@@ -168,10 +168,11 @@ int32_t fmmh_m2l_rotation_table(int32_t p, int32_t offset, double *table);
  * autotuner takes them.  Per level index 0..16. */
 typedef struct {
   int32_t p2p_uniform_min; /* mixed P2P: chunks of at least this many targets read sources by
-                              uniform loads, smaller ones through LDS tiles (0: 33) */
+                              uniform loads, smaller ones through LDS tiles (0: 43) */
   int32_t m2l_stage;       /* mixed dense M2L: 0 or 1 one k-step per pipeline stage, 2 two k-steps
                               in a ring of two LDS buffers (where the table fits) */
-  int32_t m2l_mode[17];    /* dense M2L of the level: 0 static rule (by density: reflection classes, box or clustered mode), 1 box mode, 2 clustered */
+  int32_t m2l_mode[17];    /* dense M2L of the level: 0 static rule (by density: reflection classes,
+                              box or clustered mode), 1 box mode, 2 clustered */
   int32_t l2l_width[17];   /* L2L into the level: 0 static rule, or 16, 64, 128 columns per task */
   int32_t m2m_form[17];    /* M2M into the parents of the level: 0 static, 1 per-tile, 2 split */
 } fmmh_tuning;
@@ -195,6 +196,10 @@ int32_t fmmh_operator_create_tuned(const fmmh_plan *plan, const fmmh_operator_op
  * decisions is the caller's (fmm_amd/tune.py). */
 int32_t fmmh_autotune(const fmmh_plan *plan, const fmmh_operator_options *options, double budget_seconds,
                       fmmh_tuning *out, double *report);
+/* out[level] (nlevels of them): 1 where an operator of these options runs the level's dense
+ * M2L by reflection classes under the static rule.  Such levels share one launch and the
+ * autotune takes no M2L decision for them. */
+int32_t fmmh_m2l_class_levels(const fmmh_plan *plan, const fmmh_operator_options *options, int32_t *out);
 void fmmh_operator_free(fmmh_operator *op);
 int32_t fmmh_operator_stats(const fmmh_operator *op, fmmh_stats *out);
 /* Charges of the sources in caller order, on the host (on_device = 0) or on the GPU;

@@ -64,6 +64,27 @@ def test_level_buckets_of_a_plan():
     assert set(b["l2l"]) == set(range(1, plan.nlevels))
 
 
+@pytest.mark.parametrize("precision", ["f64", "mixed"])
+def test_no_decision_for_levels_by_reflection_classes(tmp_path, precision):
+    """The levels that the static rule runs by reflection classes share one launch: the tuner
+    decides nothing for them, and a decision cached for another plan's level with as many pairs
+    does not reach them."""
+    rng = O.Rng(85)
+    plan = fmm_amd.Plan(rng.cube(20000), leaf_points=8)
+    classes = tune.m2l_class_levels(plan, 8, precision)
+    # 143 pairs a box on level 4, 10 on level 5: the deepest level is left to contraction
+    assert plan.nlevels == 6 and classes == [2, 3, 4]
+    assert tune.m2l_class_levels(plan, 8, precision, "rotation") == []
+    t = _lib.Tuning()
+    every = tune.level_buckets(plan)
+    for l in every["m2l"]:
+        t.m2l_mode[l] = 2
+    cache = tune.TuningCache(tmp_path)
+    cache.store("k", every, t, np.zeros((5, 17, 5)), precision)
+    got, missing = cache.lookup("k", tune.level_buckets(plan, classes), precision)
+    assert not missing and [l for l in range(17) if got.m2l_mode[l]] == [5]
+
+
 def test_device_key_names_the_architecture():
     # the cache key's device part comes from the HIP runtime, never from a name that a
     # profiler or another binding may report differently
@@ -116,9 +137,16 @@ def test_autotune_and_cache(_gpu, tmp_path, precision):
     assert not info["cached"] and info["tuned_s"] > 0
     d = info["decisions"]
     if precision == "mixed":
-        assert d["p2p_uniform_min"] in (33, 17, 49, 65, 129)
+        assert d["p2p_uniform_min"] in tune.P2P_CANDIDATES
     assert all(m in (0, 1, 2) for m in d["m2l_mode"])
     assert all(w in (0, 16, 64, 128) for w in d["l2l_width"])
+    classes = tune.m2l_class_levels(f1.plan, 8, precision)
+    assert classes and all(d["m2l_mode"][l] == 0 for l in classes)
+    report = info["report_ms"]
+    assert all(np.isnan(report[1][l]).all() for l in classes)
+    if precision == "mixed":
+        # the static threshold is the first candidate
+        assert tune.P2P_CANDIDATES[0] == 43 and not np.isnan(report[0][0][0])
     # the second build takes every decision from the cache
     b2 = fmm_amd.FmmBuilder(8).precision(precision).max_points_per_leaf(64).tuning_cache(tmp_path)
     f2 = b2.build(pts)
