@@ -472,20 +472,19 @@ HelmholtzOperator::HelmholtzOperator(const Plan &plan, const HelmholtzOptions &o
   }
   // dense levels whose M2L runs by reflection classes: the tables of the 56 classes' offsets
   // alone, their real and imaginary parts as two sets, and each box's re and im expansions
-  // as two rows (Re L += Tr Re M + Ti (-Im M), Im L += Tr Im M + Ti Re M).  Trees of fewer
-  // than 100,000 pairs keep a table per offset: there the per-pair rotation, the form chosen to
-  // hold less memory, would hold more than the classes' tables (3,000 points, p = 10: 94 MB
-  // against 67).
+  // as two rows (Re L += Tr Re M + Ti (-Im M), Im L += Tr Im M + Ti Re M).  Small trees gain the
+  // most, since a table per offset is read for few pairs each (3,000 points, p = 10: 598 -> 140
+  // us and 196 -> 68 MB in f64, 225 -> 98 us and 149 -> 60 MB mixed; 3,000 Plummer points,
+  // p = 15, f64: 4.8 -> 0.44 ms, 1480 -> 510 MB).
   std::vector<char> reflected(nlevels_, 0);
   {
     std::vector<uint64_t> pairs(nlevels_, 0), boxes(nlevels_, 0);
-    uint64_t total = 0;
     for (int l = 2; l < nlevels_; ++l)
       if (dense_level[l]) {
-        total += pairs[l] = plan.v[l].size();
+        pairs[l] = plan.v[l].size();
         boxes[l] = plan.nboxes(l);
       }
-    if (total >= 100000 && ReflectM2l::fits(p, opt_.precision == kMixed, 3 * nbox_total_))
+    if (ReflectM2l::fits(p, opt_.precision == kMixed, 3 * nbox_total_))
       reflected = ReflectM2l::levels(p, pairs, boxes);
   }
   if (std::count(reflected.begin(), reflected.end(), char(1)) > 0) {

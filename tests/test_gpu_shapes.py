@@ -99,7 +99,7 @@ def test_helmholtz_p2p_rows_over_waves(k, leaf, gradients, precision, tol):
 @pytest.mark.parametrize("precision,tol", [("f64", 1e-12), ("mixed", 2e-6)])
 @pytest.mark.parametrize("p,k", [(5, 3.0 + 0.2j), (9, 6.0)])
 def test_helmholtz_m2l_reflection_classes(p, k, precision, tol):
-    """Enough pairs for the classes (100,000): complex tables as two sets, a level at a time."""
+    """Complex tables as two sets, a level at a time, over 100,000 pairs."""
     _log(f"case Helmholtz M2L reflection p={p} k={k} {precision}")
     rng = O.Rng(56)
     pts = np.vstack([rng.cube(9000), rng.plummer(1000, (0.5, 0.5, 0.5), 0.02)])
@@ -109,6 +109,26 @@ def test_helmholtz_m2l_reflection_classes(p, k, precision, tol):
     assert sum(len(fmm.plan.list("v", level)[1]) for level in range(2, fmm.plan.nlevels)) >= 100_000
     out = fmm.evaluate(q)
     phi, grad = O.Fmm(pts, p=p, leaf_points=10).evaluate_helmholtz(k, q)
+    errs = [np.linalg.norm(out.potential - phi) / np.linalg.norm(phi),
+            np.linalg.norm(out.gradient - grad) / np.linalg.norm(grad)]
+    _log(f"  errors {errs}")
+    assert max(errs) < tol, errs
+
+
+@pytest.mark.parametrize("precision,tol", [("f64", 1e-12), ("mixed", 2e-6)])
+def test_helmholtz_small_trees_take_the_classes(precision, tol):
+    """A tree of few pairs holds 56 offsets' tables a level, not one for each of its offsets."""
+    p, k = 10, 25.0
+    _log(f"case Helmholtz M2L reflection on a small tree {precision}")
+    rng = O.Rng(58)
+    pts = rng.cube(3000)
+    q = rng.normals(len(pts)) + 1j * rng.normals(len(pts))
+    fmm = fmm_amd.HelmholtzFmmBuilder(k, degree=p).max_points_per_leaf(40).precision(precision).build(pts)
+    per_offset = [len(np.unique(fmm.plan.list("v", level)[2])) for level in range(2, fmm.plan.nlevels)]
+    assert 0 < sum(len(fmm.plan.list("v", level)[1]) for level in range(2, fmm.plan.nlevels)) < 100_000
+    assert fmm.operator.stats()["device_bytes"] < 0.6 * sum(per_offset) * 2 * (p + 1) ** 4 * 8
+    out = fmm.evaluate(q)
+    phi, grad = O.Fmm(pts, p=p, leaf_points=40).evaluate_helmholtz(k, q)
     errs = [np.linalg.norm(out.potential - phi) / np.linalg.norm(phi),
             np.linalg.norm(out.gradient - grad) / np.linalg.norm(grad)]
     _log(f"  errors {errs}")
