@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import fmm_amd
+from fmm_amd import tune
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -50,6 +51,12 @@ def test_m2p_rows_over_waves(p, leaf, gradients):
     _check(fmm, O.Fmm(pts, p=p, leaf_points=leaf, gradients=gradients), q, gradients)
 
 
+def _class_rows(plan, p, precision):
+    """The boxes whose M2L runs by reflection classes."""
+    return sum(int(np.count_nonzero(np.diff(plan.list("v", level)[0])))
+               for level in tune.m2l_class_levels(plan, p, precision))
+
+
 @pytest.mark.parametrize("precision,tol", [("f64", 1e-12), ("mixed", 1e-6)])
 @pytest.mark.parametrize("p", [5, 6, 8, 10, 11, 12, 13, 14, 15])
 def test_m2l_reflection_classes(p, precision, tol):
@@ -60,16 +67,40 @@ def test_m2l_reflection_classes(p, precision, tol):
     pts = np.vstack([rng.cube(4500), rng.plummer(1500, (0.4, 0.6, 0.5), 0.03)])
     q = rng.normals(len(pts))
     fmm = fmm_amd.FmmBuilder(p).max_points_per_leaf(24).precision(precision).build(pts)
+    rows = _class_rows(fmm.plan, p, precision)
+    assert 0 < rows < 512 * 16  # less than a round of workgroups: every row through scratch rows
     _check(fmm, O.Fmm(pts, p=p, leaf_points=24), q, tol=tol)
 
 
-def test_m2l_reflection_level_calls():
-    """The level calls run each level's share of the tasks (whole and split into parts)."""
-    _log("case M2L reflection, level by level")
+@pytest.mark.parametrize("precision,tol", [("f64", 1e-12), ("mixed", 1e-6)])
+@pytest.mark.parametrize("p", [4, 7, 12])
+def test_m2l_reflection_whole_rounds(p, precision, tol):
+    """More than a round of workgroups (1,024 of 16 boxes in f64, 512 of 32 mixed): the rows of the
+    whole rounds add to the locals themselves, those of the last go through scratch rows.  Against
+    the rotation M2L in f64, another path from the multipoles to the locals."""
+    _log(f"case M2L reflection, whole rounds p={p} {precision}")
     rng = O.Rng(92)
     pts = rng.cube(60000)
     q = rng.normals(len(pts))
-    fmm = fmm_amd.FmmBuilder(7).max_points_per_leaf(8).build(pts)
+    plan = fmm_amd.Plan(pts, leaf_points=8)
+    rows = _class_rows(plan, p, precision)
+    assert rows > 16384 and rows % 16384 != 0
+    out = fmm_amd.Fmm(plan, fmm_amd.Operator(plan, p, precision)).evaluate(q)
+    ref = fmm_amd.Fmm(plan, fmm_amd.Operator(plan, p, "f64", m2l="rotation")).evaluate(q)
+    errs = [O.error_norms(out.potential, ref.potential)[0], O.error_norms(out.gradient, ref.gradient, True)[0]]
+    _log(f"  errors {errs}")
+    assert max(errs) < tol, errs
+
+
+@pytest.mark.parametrize("precision", ["f64", "mixed"])
+def test_m2l_reflection_level_calls(precision):
+    """The level calls run each level's share of the tasks (whole and split into parts)."""
+    _log(f"case M2L reflection, level by level {precision}")
+    rng = O.Rng(92)
+    pts = rng.cube(60000)
+    q = rng.normals(len(pts))
+    fmm = fmm_amd.FmmBuilder(7).max_points_per_leaf(8).precision(precision).build(pts)
+    assert _class_rows(fmm.plan, 7, precision) > 16384
     a, b = fmm.evaluate(q), fmm.evaluate_levels(q)
     assert O.error_norms(b.potential, a.potential)[0] < 1e-14
     assert O.error_norms(b.gradient, a.gradient, True)[0] < 1e-14
@@ -107,6 +138,9 @@ def test_helmholtz_m2l_reflection_classes(p, k, precision, tol):
     b = fmm_amd.HelmholtzFmmBuilder(k, degree=p).max_points_per_leaf(10).precision(precision)
     fmm = b.build(pts)
     assert sum(len(fmm.plan.list("v", level)[1]) for level in range(2, fmm.plan.nlevels)) >= 100_000
+    # (a table for each offset would be twice what the operator holds)
+    per_offset = [len(np.unique(fmm.plan.list("v", level)[2])) for level in range(2, fmm.plan.nlevels)]
+    _log(f"  {fmm.operator.stats()['device_bytes']} bytes, tables per offset {sum(per_offset) * 2 * (p + 1) ** 4 * 8}")
     out = fmm.evaluate(q)
     phi, grad = O.Fmm(pts, p=p, leaf_points=10).evaluate_helmholtz(k, q)
     errs = [np.linalg.norm(out.potential - phi) / np.linalg.norm(phi),
