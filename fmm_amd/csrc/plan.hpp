@@ -125,7 +125,8 @@ int coaxial_block_size(int p);
 void build_rotation_tables(int p, std::vector<double> &fwd, std::vector<double> &bwd, std::vector<double> &coax,
                            std::vector<uint16_t> &dist_of, std::vector<double> &dist2);
 
+// (with `only`, the M2L of those offset indices alone, in their order)
 void build_tables(int p, std::vector<double> &m2m, std::vector<double> &l2l,
-                  std::vector<double> &m2l);
+                  std::vector<double> &m2l, const std::vector<uint16_t> *only = nullptr);
 
 }  // namespace fmmh

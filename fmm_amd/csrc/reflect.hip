@@ -673,10 +673,12 @@ void ReflectM2l::begin(int p, bool mixed, const std::vector<size_t> &level_vec, 
 uint32_t ReflectM2l::add_tables(const std::function<const double *(int, int)> &table) {
   const size_t sz = mixed_ ? dev::reflect_table_size_bf16(lay_) : dev::reflect_table_size(lay_);
   size_t at = sz * kReflectClasses * ntables_;
+  // (after the last chunk a wave reads, and drops, the next chunk's tiles)
+  const size_t past = size_t(lay_.tiles + 4) * (mixed_ ? 1536 : 256);
   if (mixed_)
-    tables16_h_.resize(at + sz * kReflectClasses * sets_);
+    tables16_h_.resize(at + sz * kReflectClasses * sets_ + past);
   else
-    tables_h_.resize(at + sz * kReflectClasses * sets_);
+    tables_h_.resize(at + sz * kReflectClasses * sets_ + past);
   for (int s = 0; s < sets_; ++s)
     for (int c = 0; c < kReflectClasses; ++c, at += sz) {
       if (mixed_)
@@ -810,14 +812,10 @@ void ReflectM2l::finish() {
   args_.row_flip = static_cast<const uint8_t *>(at(o_flip));
   args_.src = static_cast<const uint32_t *>(at(o_src));
   scratch_.alloc(size_t(nscratch) * lay_.nc);
-  // (after the last chunk a wave reads, and drops, the next chunk's tiles)
-  if (mixed_) {
-    tables16_h_.resize(tables16_h_.size() + size_t(lay_.tiles + 4) * 1536);
+  if (mixed_)
     tables16_.upload(tables16_h_);
-  } else {
-    tables_h_.resize(tables_h_.size() + size_t(lay_.tiles + 4) * 256);
+  else
     tables_.upload(tables_h_);
-  }
   sorted_.alloc((nvec_ + 1) * lay_.kp);
   hip_check(hipMemset(sorted_.ptr + nvec_ * lay_.kp, 0, size_t(lay_.kp) * sizeof(double)), "reflection zero row");
   args_.nc = lay_.nc;

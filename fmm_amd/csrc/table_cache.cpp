@@ -143,14 +143,15 @@ void table_cache_stats(int64_t *hits, int64_t *misses) {
   if (misses) *misses = g_misses;
 }
 
-void cached_tables(int p, std::vector<double> &m2m, std::vector<double> &l2l, std::vector<double> &m2l) {
+void cached_tables(int p, std::vector<double> &m2m, std::vector<double> &l2l, std::vector<double> &m2l,
+                   const std::vector<uint16_t> *only) {
   std::string dir;
   {
     std::lock_guard<std::mutex> lock(g_mu);
     dir = g_dir;
   }
   if (dir.empty()) {
-    build_tables(p, m2m, l2l, m2l);
+    build_tables(p, m2m, l2l, m2l, only);
     return;
   }
   const bool hit = load(dir, 1, p, m2m) && load(dir, 2, p, l2l) && load(dir, 3, p, m2l);
@@ -158,11 +159,19 @@ void cached_tables(int p, std::vector<double> &m2m, std::vector<double> &l2l, st
     std::lock_guard<std::mutex> lock(g_mu);
     ++(hit ? g_hits : g_misses);
   }
-  if (hit) return;
-  build_tables(p, m2m, l2l, m2l);
-  store(dir, 1, p, m2m);
-  store(dir, 2, p, l2l);
-  store(dir, 3, p, m2l);
+  if (!hit) {
+    build_tables(p, m2m, l2l, m2l);
+    store(dir, 1, p, m2m);
+    store(dir, 2, p, l2l);
+    store(dir, 3, p, m2l);
+  }
+  if (only) {
+    const size_t n2 = size_t(ncoef(p)) * ncoef(p);
+    std::vector<double> some(only->size() * n2);
+    for (size_t i = 0; i < only->size(); ++i)
+      std::memcpy(some.data() + i * n2, m2l.data() + (*only)[i] * n2, n2 * sizeof(double));
+    m2l.swap(some);
+  }
 }
 
 }  // namespace fmmh

@@ -350,21 +350,22 @@ void build_rotation_tables(int p, std::vector<double> &fwd, std::vector<double> 
 }
 
 void build_tables(int p, std::vector<double> &m2m, std::vector<double> &l2l,
-                  std::vector<double> &m2l) {
+                  std::vector<double> &m2l, const std::vector<uint16_t> *only) {
   require(p >= 0 && p <= 30, "build_tables: p must lie in 0..30");
   const size_t n2 = size_t(ncoef(p)) * ncoef(p);
   m2m.assign(8 * n2, 0.0);
   l2l.assign(8 * n2, 0.0);
-  m2l.assign(316 * n2, 0.0);
+  const int count = only ? int(only->size()) : 316;
+  m2l.assign(size_t(count) * n2, 0.0);
   for (int o = 0; o < 8; ++o) {
     const double s[3] = {0.5 * (2 * ((o >> 2) & 1) - 1), 0.5 * (2 * ((o >> 1) & 1) - 1), 0.5 * (2 * (o & 1) - 1)};
     m2m_table(p, s, 0.5, m2m.data() + o * n2);
     l2l_table(p, s, 0.5, l2l.data() + o * n2);
   }
 #pragma omp parallel for schedule(dynamic, 4)
-  for (int t = 0; t < 316; ++t) {
+  for (int t = 0; t < count; ++t) {
     int d[3];
-    offset_of_index(t, d);
+    offset_of_index(only ? (*only)[t] : t, d);
     const double b[3] = {2.0 * d[0], 2.0 * d[1], 2.0 * d[2]};
     m2l_table(p, b, 1.0, m2l.data() + t * n2);
   }

@@ -92,6 +92,32 @@ def test_m2l_reflection_whole_rounds(p, precision, tol):
     assert max(errs) < tol, errs
 
 
+@pytest.mark.parametrize("points,every", [(1000, False), (20000, True)])
+def test_m2l_class_tables_of_an_operator(tmp_path, points, every):
+    """The M2L tables that an operator builds (the classes' alone where no level takes a
+    contraction, all with a level that does), built, stored and loaded: the same bits."""
+    _log(f"case M2L class tables, {points} points")
+    rng = O.Rng(93)
+    pts = rng.cube(points)
+    q = rng.normals(points)
+    plan = fmm_amd.Plan(pts, leaf_points=8)
+    classes = tune.m2l_class_levels(plan, 6, "f64")
+    others = [l for l in range(2, plan.nlevels) if len(plan.list("v", l)[1]) and l not in classes]
+    assert classes and bool(others) == every
+    out = []
+    try:
+        for directory in (None, tmp_path, tmp_path):
+            fmm_amd.set_table_cache(directory)
+            out.append(fmm_amd.Fmm(plan, fmm_amd.Operator(plan, 6, "f64")).evaluate(q))
+        assert fmm_amd.table_cache_stats() == (1, 0)
+    finally:
+        fmm_amd.set_table_cache(None)
+    ref = fmm_amd.Fmm(plan, fmm_amd.Operator(plan, 6, "f64", m2l="rotation")).evaluate(q)
+    assert O.error_norms(out[0].potential, ref.potential)[0] < 1e-12
+    for o in out[1:]:
+        assert np.array_equal(o.potential, out[0].potential) and np.array_equal(o.gradient, out[0].gradient)
+
+
 @pytest.mark.parametrize("precision", ["f64", "mixed"])
 def test_m2l_reflection_level_calls(precision):
     """The level calls run each level's share of the tasks (whole and split into parts)."""
