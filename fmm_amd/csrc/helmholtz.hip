@@ -556,8 +556,10 @@ __global__ __launch_bounds__(SING ? 64 * kRowWaves : 64) void k_h_evaluate(int p
 // pair arithmetic in f32, each source leaf's f32 sums added to f64 accumulators.
 // Pair kernel pieces per precision.  f64: 1/r by v_rsq_f64 and a third-order step, r = r^2 /
 // r corrected once (the bits of sqrt; 1/r within 0.99 ulp, rms 5.2e-17, where 1 / sqrt rounds
-// twice: 1.49 and 6.7e-17), sine and cosine by sincos_f64 (about 345 cycles per 64 pairs against 830
-// with the math library's, whose reductions for huge arguments they carry along).  f32: 1/r from v_rsq_f32 (1 ulp) and r = r^2 / r; sine and cosine from v_sin_f32
+// twice: 1.49 and 6.7e-17), the phase by sincos_reduced and its quadrant applied to the product
+// (81 vector instructions, about 340 cycles per 64 pairs, against 830 with the math library's,
+// whose reductions for huge arguments they carry along; 200,000 uniform points, 2.2e8 pairs:
+// 0.79 ms).  f32: 1/r from v_rsq_f32 (1 ulp) and r = r^2 / r; sine and cosine from v_sin_f32
 // and v_cos_f32 of the fraction of x / (2 pi).
 template <typename T>
 struct PairMath;
@@ -572,7 +574,15 @@ struct PairMath<double> {
     r = r2 * ir;
     r = fma(0.5 * ir, fma(-r, r, r2), r);
   }
-  __device__ static __forceinline__ void sincos(double x, double *s, double *c) { sincos_f64(x, s, c); }
+  // (a + i b) e^{ix} w: i^n to the product in place of a sign and a choice for sine and cosine each
+  __device__ static __forceinline__ void times_phase(double x, double a, double b, double w, double &re, double &im) {
+    double s, c;
+    const uint32_t n = sincos_reduced(x, &s, &c);
+    const double u = a * c - b * s, v = a * s + b * c;
+    w = __hiloint2double(__double2hiint(w) ^ int((n << 30) & 0x80000000u), __double2loint(w));
+    re = ((n & 1) ? -v : u) * w;
+    im = ((n & 1) ? u : v) * w;
+  }
 };
 
 template <>
@@ -588,6 +598,12 @@ struct PairMath<float> {
     const float t = __builtin_amdgcn_fractf(x * 0.159154943091895336f);
     *s = __builtin_amdgcn_sinf(t);
     *c = __builtin_amdgcn_cosf(t);
+  }
+  __device__ static __forceinline__ void times_phase(float x, float a, float b, float w, float &re, float &im) {
+    float s, c;
+    sincos(x, &s, &c);
+    re = (a * c - b * s) * w;
+    im = (a * s + b * c) * w;
   }
 };
 
@@ -802,11 +818,9 @@ __device__ __forceinline__ void h_p2p_staged(HP2pStage<T> &sh, uint32_t lf, uint
             const T r2 = dx * dx + dy * dy + dz * dz;
             T rr, ir;
             PairMath<T>::rinv(r2, rr, ir);
-            T sn, cs;
-            PairMath<T>::sincos(kre * rr, &sn, &cs);
-            const T dmp = DAMP ? T(exp(-kim * rr)) : T(1);
-            const T q0 = ys[i][6], q1 = ys[i][7], es = DAMP ? dmp * ir : ir;
-            const T pr = (q0 * cs - q1 * sn) * es, pi = (q0 * sn + q1 * cs) * es;  // q e^{ikr} / r
+            const T es = DAMP ? T(exp(-kim * rr)) * ir : ir;
+            T pr, pi;  // q e^{ikr} / r
+            PairMath<T>::times_phase(kre * rr, ys[i][6], ys[i][7], es, pr, pi);
             loc[a][0] += pr;
             loc[a][1] += pi;
             if (GRAD) {
@@ -879,9 +893,10 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_h_p2p(
                                          tz, phi_hat, grad_hat);
       continue;
     }
-    // one target per lane unless two fill more of the lanes' target slots
+    // two targets per lane unless one fills more of the lanes' target slots (two share each
+    // source's LDS reads, and one takes 11 register moves a pair for the polynomials' constants)
     const int slots1 = n <= 64 ? int(n) * (64 / int(n)) : 0, slots2 = int(n) * (64 / ((int(n) + 1) / 2));
-    if (2 * slots1 >= slots2)
+    if (2 * slots1 > slots2)
       h_p2p_staged<T, GRAD, DAMP, 1>(sh, lf, tb, n, e0, e1, kre, kim, near_ent, leaf_cell, src_start, sx, sy, sz, qr,
                                      qi, tx, ty, tz, phi_hat, grad_hat);
     else

@@ -16,7 +16,9 @@ namespace dev {
 // beyond any k r of a leaf pair.  Against long double over (0, 6), (0, 60) and (0, 600): at most
 // 0.77 ulp, rms 0.293 (the math library's: 0.78 and 0.294; without tl and the carried rounding
 // 1.54 and 0.418).
-__host__ __device__ __forceinline__ void sincos_f64(double x, double *s, double *c) {
+
+// The sine and cosine of the reduced argument, and its quadrant n (its low two bits).
+__host__ __device__ __forceinline__ uint32_t sincos_reduced(double x, double *s, double *c) {
   constexpr double kShift = 6755399441055744.0;  // 1.5 2^52: the sum's low bits are rint(x 2/pi)
   const double m = std::fma(x, 0.6366197723675814, kShift), n = m - kShift;
   const uint32_t q = uint32_t(__builtin_bit_cast(uint64_t, m));
@@ -36,8 +38,14 @@ __host__ __device__ __forceinline__ void sincos_f64(double x, double *s, double 
   pc = std::fma(z, pc, 0.041666666666666664);
   // 1 - z / 2, and what its rounding left out
   const double w = std::fma(-0.5, z, 1.0), e = std::fma(-0.5, z, 1.0 - w);
-  const double st = t + std::fma(t * z, ps, w * tl);
-  const double ct = w + std::fma(z * z, pc, std::fma(-t, tl, e));
+  *s = t + std::fma(t * z, ps, w * tl);
+  *c = w + std::fma(z * z, pc, std::fma(-t, tl, e));
+  return q;
+}
+
+__host__ __device__ __forceinline__ void sincos_f64(double x, double *s, double *c) {
+  double st, ct;
+  const uint32_t q = sincos_reduced(x, &st, &ct);
   const double sv = (q & 1) ? ct : st, cv = (q & 1) ? st : ct;
   *s = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, sv) ^ (uint64_t(q & 2) << 62));
   *c = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, cv) ^ (uint64_t((q + 1) & 2) << 62));
