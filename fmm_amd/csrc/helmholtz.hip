@@ -307,7 +307,7 @@ __device__ __forceinline__ void add_waves(int wave, int lane, double (&acc)[8], 
 // L2P: one wave per target leaf, one target per lane (chunks of 64).  M2P: kRowWaves waves
 // per leaf and chunk, which take the row's boxes in turn, each with its own coefficients in
 // LDS, their sums added in wave order (rows are few and their boxes many: 80,000 Plummer
-// points, 31 rows: 1.5 -> 0.3 ms).  With C the entry box's
+// points, 31 rows: 1.5 -> 0.16 ms).  With C the entry box's
 // coefficients (two planes in LDS) and v the target in the box's units,
 //   F = sum_n c_n sum_m C_n^m S_n^m(v),   grad F = sum_n c_n grad(...) + (sum_n d_n ...) v,
 // L2P: c_n = e^-beta (kh/s)^n g_n, d_n = -kh^2 e^-beta (kh/s)^n g_{n+1};

@@ -1121,7 +1121,7 @@ __global__ __launch_bounds__(64) void k_l2p(int p, uint32_t rows, const uint32_t
 // (n, m >= 0) of LDS holds what the lane needs at that step of its column, weighted by 2
 // for m > 0: (Re, Im) of the coefficient of I_n^m and, with gradients, of its three
 // derivative coefficients, in the order the columns are walked.  150,000 Plummer points,
-// p = 8 (1,886 rows of 27 boxes, at most 98): 1.85 -> 0.46 ms; 43 rows of 123 boxes, p = 9,
+// p = 8 (1,886 rows of 27 boxes, at most 98): 1.85 -> 0.30 ms; 43 rows of 123 boxes, p = 9,
 // potentials alone: 1.28 -> 0.07 ms.
 struct M2pEntry {
   double c[2], x[2], y[2], z[2];

@@ -116,7 +116,7 @@ void output_pass(hipStream_t s, uint32_t nleaves, const uint32_t *tgt_start, con
                  int gradients);
 
 // P2P over the leaves leaf_first .. leaf_first + count (global leaf indices), computed in
-// T (double, or float with fixed-point or double-float separations); f64 coordinates and
+// T (double, or float with fixed-point separations); f64 coordinates and
 // charges.  T = float also reads the source records of build_source_records (4 words per
 // source; rec is unused for T = double and may be null).  uniform_min: for T = float,
 // chunks of at least this many targets (and at most 128) take the uniform-source form;

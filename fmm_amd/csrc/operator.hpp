@@ -30,7 +30,7 @@ constexpr uint32_t kM2lXcdRun = 8;
 
 enum Precision : int {
   kPlainF64 = 0,  // every operator in f64
-  kMixed = 1,     // P2P in f32 (double-float separations), M2L in bf16x3 on MFMA
+  kMixed = 1,     // P2P in f32 (fixed-point separations), M2L in bf16x3 on MFMA
 };
 
 // One contraction launch: tasks of COLS output columns, groups of (table, sources).
