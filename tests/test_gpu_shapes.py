@@ -58,9 +58,9 @@ def _class_rows(plan, p, precision):
 
 
 @pytest.mark.parametrize("precision,tol", [("f64", 1e-12), ("mixed", 1e-6)])
-@pytest.mark.parametrize("p", [5, 6, 8, 10, 11, 12, 13, 14, 15])
+@pytest.mark.parametrize("p", [0, 1, 4, 5, 6, 8, 10, 11, 12, 13, 14, 15])
 def test_m2l_reflection_classes(p, precision, tol):
-    """Dense levels at every count of row tiles (8 to 20) and of coefficient chunks, boundary
+    """Dense levels at every count of row tiles (1 to 20) and of coefficient chunks, boundary
     boxes (sources missing at some reflections), target rows that do not fill a workgroup."""
     _log(f"case M2L reflection p={p} {precision}")
     rng = O.Rng(91 + p)
