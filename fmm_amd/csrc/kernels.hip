@@ -257,7 +257,7 @@ __global__ void k_vjp_combine(size_t n, const double *q, const double *g, const 
 // (c'' = (C_t - C_s) / r_s, rho = r_t / r_s), and rounded to the same fixed point: in a
 // 2:1-balanced tree a near leaf (U list, or W/X pairs moved to P2P by the near rule) has
 // |x'| <= 1 + 2 rho + 2 <= 7 per axis, so |x' 2^28| < 2^31 and the separation
-// d' = x' - u_s, within 8 half-widths (less one unit, p2p_fixed), is one exact integer
+// d' = x' - u_s, within 8 half-widths (p2p_fixed_target), is one exact integer
 // subtraction per axis, then one conversion to f32 (relative rounding 2^-24).  The
 // coordinates' quantisation, 2^-29 source-leaf units at either end, bounds the error of a
 // pair at 2^-28 / |d'| per axis: 2^-23.5 from |d'| = 2^-4.5 half-widths on; a closer pair (r^2 under 2^47 integer units, rare: one in ~10^6 pairs
@@ -269,12 +269,16 @@ __global__ void k_vjp_combine(size_t n, const double *q, const double *g, const 
 // Off the own leaf r^2 starts from 1/4 (integer units) in the quantised form and from the
 // smallest normal float in the f64 form: distinct points keep a finite r^2.
 // A position up to 7 half-widths out, seen from the other leaf of a near pair, in the fixed
-// point.  One unit is kept from the ends: 7 half-widths against a coordinate of 1 on the other
-// side would be 2^31, past an int32.
-__device__ __forceinline__ int p2p_fixed(double u) {
-  constexpr int kReach = 7 * (1 << 28) - 1;
+// point.  One unit is kept from one end: 7 half-widths less a coordinate of -1 (a target, from
+// which the sources' coordinates are subtracted), or a coordinate of 1 less -7 half-widths (a
+// source), would be 2^31, one past an int32; -2^31 is one.
+__device__ __forceinline__ int p2p_fixed_target(double u) {
   const int v = __double2int_rn(u * kP2pFixed);
-  return v > kReach ? kReach : v < -kReach ? -kReach : v;
+  return min(v, 7 * (1 << 28) - 1);
+}
+__device__ __forceinline__ int p2p_fixed_source(double u) {
+  const int v = __double2int_rn(u * kP2pFixed);
+  return max(v, 1 - 7 * (1 << 28));
 }
 
 template <bool GRAD, bool TWO>
@@ -315,7 +319,7 @@ __device__ __forceinline__ void p2p_uniform(uint32_t lf, uint32_t tb, uint32_t n
 #pragma unroll
     for (int a = 0; a < A; ++a)
 #pragma unroll
-      for (int k = 0; k < 3; ++k) xi[a][k] = p2p_fixed(fma(rho, u[a][k], c[k]));
+      for (int k = 0; k < 3; ++k) xi[a][k] = p2p_fixed_target(fma(rho, u[a][k], c[k]));
     const bool own = sl == lf;
     // entries flagged at build (a pair of the entry closer than the threshold) and the
     // own leaf test their pairs; the others run the separations unchecked
@@ -494,22 +498,28 @@ __device__ __forceinline__ void p2p_staged(P2pStage<T> &sh, uint32_t lf, uint32_
     ap[a] = ax[a] = ay[a] = az[a] = T(0);
   }
   // f32 sums are per tile (at most 64 terms) and go into f64 after each tile,
-  // so long near rows do not lose digits to one growing f32 sum; `unit` is what the tile's sums
-  // of charges are counted in
-  double unit = 1.0;
+  // so long near rows do not lose digits to one growing f32 sum
+  bool large = false;  // the tile's charges are counted in units of kUnit (stage)
+  constexpr double kUnit = GRAD ? 0x1p30 : kP2pFixed;
   double cp[A], cx[A], cy[A], cz[A];
 #pragma unroll
   for (int a = 0; a < A; ++a) cp[a] = cx[a] = cy[a] = cz[a] = 0.0;
   auto flush = [&]() {
     if (FIXED) {
+      auto add = [&](double unit) {
 #pragma unroll
-      for (int a = 0; a < A; ++a) {
-        cp[a] = fma(double(ap[a]), unit, cp[a]);
-        cx[a] = fma(double(ax[a]), unit / kP2pFixed, cx[a]);
-        cy[a] = fma(double(ay[a]), unit / kP2pFixed, cy[a]);
-        cz[a] = fma(double(az[a]), unit / kP2pFixed, cz[a]);
-        ap[a] = ax[a] = ay[a] = az[a] = T(0);
-      }
+        for (int a = 0; a < A; ++a) {
+          cp[a] = fma(double(ap[a]), unit, cp[a]);
+          cx[a] = fma(double(ax[a]), unit / kP2pFixed, cx[a]);
+          cy[a] = fma(double(ay[a]), unit / kP2pFixed, cy[a]);
+          cz[a] = fma(double(az[a]), unit / kP2pFixed, cz[a]);
+          ap[a] = ax[a] = ay[a] = az[a] = T(0);
+        }
+      };
+      if (large)
+        add(kUnit);
+      else
+        add(1.0);
     }
   };
   auto minus = [](C a, C b) {
@@ -588,11 +598,10 @@ __device__ __forceinline__ void p2p_staged(P2pStage<T> &sh, uint32_t lf, uint32_
     // charge beyond 2^38 counts in larger units, so that neither leaves f32 where the plain
     // q / r^3 and q / r would not; what a small charge of such a tile loses is far below the
     // rounding of the large one's term (at most 8 sqrt 3 half-widths away).
-    double per_unit = 1.0;
     if constexpr (FIXED) {
-      const bool large = __any(valid && fabs(q) > 0x1p38);
-      unit = large ? (GRAD ? 0x1p30 : kP2pFixed) : 1.0;
-      per_unit = large ? (GRAD ? 0x1p-30 : 1.0) : (GRAD ? 1.0 : kP2pFixed);
+      large = __any(valid && fabs(q) > 0x1p38);
+      if (!GRAD) q *= kP2pFixed;
+      if (large) q *= 1.0 / kUnit;
     }
     __syncthreads();
     if (lane < steps * phases) {
@@ -602,8 +611,7 @@ __device__ __forceinline__ void p2p_staged(P2pStage<T> &sh, uint32_t lf, uint32_
       }
       V4 v;
       if constexpr (FIXED) {
-        v = make_int4(p2p_fixed(yx), p2p_fixed(yy), p2p_fixed(yz),
-                      __float_as_int(float(q * per_unit)));
+        v = make_int4(p2p_fixed_source(yx), p2p_fixed_source(yy), p2p_fixed_source(yz), __float_as_int(float(q)));
         sh.yd[lane][0] = yx;
         sh.yd[lane][1] = yy;
         sh.yd[lane][2] = yz;
@@ -1436,9 +1444,9 @@ __global__ __launch_bounds__(64) void k_p2p_close_flags(uint32_t count, const ui
     for (uint32_t tb = t0; tb < t1; tb += 64) {
       const uint32_t i = tb + uint32_t(lane);
       if (i >= t1) break;
-      const int xi0 = p2p_fixed(fma(rho, tx[i], c[0]));
-      const int xi1 = p2p_fixed(fma(rho, ty[i], c[1]));
-      const int xi2 = p2p_fixed(fma(rho, tz[i], c[2]));
+      const int xi0 = p2p_fixed_target(fma(rho, tx[i], c[0]));
+      const int xi1 = p2p_fixed_target(fma(rho, ty[i], c[1]));
+      const int xi2 = p2p_fixed_target(fma(rho, tz[i], c[2]));
       for (uint32_t j = s0; j < s1; ++j) {
         const int4 h = rec[j];
         const float dx = float(xi0 - h.x), dy = float(xi1 - h.y), dz = float(xi2 - h.z);
